@@ -161,12 +161,14 @@ struct SysDesc {
   const double *rap;  // 1/ap per cell (tiled LDS sweeps), correctly rounded
 };
 
-// A single right-hand side in FP32: the correction system of the
-// mixed-precision pressure-correction solve (ap, anb, residual, correction)
-struct SysDesc32 {
+// A single right-hand side for the colour sweeps of the pc system: the system
+// itself, or in FP32 the correction system of the mixed-precision solve (ap,
+// anb, residual, correction).
+template <typename T>
+struct ColSys {
   const int *row, *nbr;
-  const float *ap, *anb, *b;
-  float *phi;
+  const T *ap, *anb, *b;
+  T *phi;
 };
 
 // (x / a) / s, correctly rounded at each step, from y = 1/a and ys = 1/s
@@ -1045,9 +1047,13 @@ __global__ void k_mass_imbalance(MeshDev m, const double *__restrict__ mip, doub
 // 287-307).  phi(e) = (sumnb + (sor-1)*ap*phi(e))/ap/sor.
 // ---------------------------------------------------------------------------
 // cells == nullptr: the cells are base .. base + n - 1 (a colour range).
+// reps: consecutive updates of the same cells.  A forward sweep ends and the
+// backward sweep starts with the same colour, whose cells have no neighbour
+// of that colour: both updates see the same row sum, so they share one pass
+// over the row (fused_turns says which launches).
 template <int NC>
 __device__ inline void d_gs_level(int bx_, SysDesc s, const int *__restrict__ cells, int base, int n, double sor,
-                           const int *__restrict__ active) {
+                           int reps, const int *__restrict__ active) {
   const int t = bx_ * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int e = cells ? cells[t] : base + t;
@@ -1073,7 +1079,9 @@ __device__ inline void d_gs_level(int bx_, SysDesc s, const int *__restrict__ ce
       double sum = s.b[c][e];
 #pragma unroll
       for (int k = 0; k < 6; k++) sum = sum + an[k] * v[k];
-      phi[e] = (sum + (sor - 1.0) * a * phi[e]) / a / sor;
+      double x = phi[e];
+      for (int r = 0; r < reps; r++) x = (sum + (sor - 1.0) * a * x) / a / sor;
+      phi[e] = x;
     }
     return;
   }
@@ -1083,40 +1091,42 @@ __device__ inline void d_gs_level(int bx_, SysDesc s, const int *__restrict__ ce
     double *phi = s.phi[c];
     double sum = s.b[c][e];
     for (int k = r0; k < r1; k++) sum = sum + s.anb[k] * phi[s.nbr[k]];
-    phi[e] = (sum + (sor - 1.0) * a * phi[e]) / a / sor;
+    double x = phi[e];
+    for (int r = 0; r < reps; r++) x = (sum + (sor - 1.0) * a * x) / a / sor;
+    phi[e] = x;
   }
 }
 template <int NC>
 __global__ void k_gs_level(SysDesc s, const int *__restrict__ cells, int base, int n, double sor,
-                           const int *__restrict__ active) {
-  d_gs_level<NC>(blockIdx.x, s, cells, base, n, sor, active);
+                           int reps, const int *__restrict__ active) {
+  d_gs_level<NC>(blockIdx.x, s, cells, base, n, sor, reps, active);
 }
 
-// The same update in FP32 on a correction system: cells of one colour (all
-// independent), row sum in CSR order, then (sum + (sor-1)*ap*phi)/ap/sor with
-// IEEE single-precision divisions.
-// One colour is a contiguous cell range in each subdomain of the colour
-// numbering: cells beg[y] .. beg[y] + off[y+1] - off[y] - 1 are launch
-// positions off[y] .. off[y+1] - 1.  HEX: every row has six entries, so row
-// e starts at 6e.
+// One colour of the pc system in the colour numbering, FP64 (T = double) or
+// the FP32 correction system of the mixed mode: all cells independent, row
+// sum in CSR order, then reps updates (sum + (sor-1)*ap*phi)/ap/sor with IEEE
+// divisions.
+// A colour is a contiguous cell range in each subdomain: cells beg[y] ..
+// beg[y] + off[y+1] - off[y] - 1 are launch positions off[y] .. off[y+1] - 1.
+// HEX: every row has six entries, so row e starts at 6e.
 struct ColRanges {
   int n;
   int beg[kMaxSys], off[kMaxSys + 1];
 };
-template <bool HEX>
-__global__ void k_gs_level32(SysDesc32 s, ColRanges cr, float sor,
-                             const int *__restrict__ active) {
+template <typename T, bool HEX>
+__global__ void k_pc_colour(ColSys<T> s, ColRanges cr, T sor, int reps,
+                            const int *__restrict__ active) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= cr.off[cr.n] || !active[0]) return;
   int y = 0;
   while (t >= cr.off[y + 1]) y++;
   const int e = cr.beg[y] + (t - cr.off[y]);
   const int r0 = HEX ? 6 * e : s.row[e], r1 = HEX ? r0 + 6 : s.row[e + 1];
-  const float a = s.ap[e];
-  float sum = s.b[e];
+  const T a = s.ap[e];
+  T sum = s.b[e];
   if (r1 - r0 == 6) {
     int nb[6];
-    float an[6], v[6];
+    T an[6], v[6];
 #pragma unroll
     for (int k = 0; k < 6; k++) {
       nb[k] = s.nbr[r0 + k];
@@ -1129,7 +1139,10 @@ __global__ void k_gs_level32(SysDesc32 s, ColRanges cr, float sor,
   } else {
     for (int k = r0; k < r1; k++) sum = sum + s.anb[k] * s.phi[s.nbr[k]];
   }
-  s.phi[e] = (sum + (sor - 1.0f) * a * s.phi[e]) / a / sor;
+  const T one = static_cast<T>(1);
+  T x = s.phi[e];
+  for (int r = 0; r < reps; r++) x = (sum + (sor - one) * a * x) / a / sor;
+  s.phi[e] = x;
 }
 
 // Mixed-precision pc solve: FP32 copies of ap and anb, and a zero correction
@@ -2043,13 +2056,16 @@ __global__ void gb_gs_iter_end(GroupMap g, const BSlot *__restrict__ S) {
   BSLOT;
   d_gs_iter_end(bx, x.gctl, x.red, 3, static_cast<double>(x.md.ne), x.nit);
 }
-// colour i of the case's forward order, or of its reverse (backward)
+// colour i of the case's forward order, or of its reverse (backward); the
+// last forward colour is updated twice, the second time as the backward
+// sweep's first
 __global__ void gb_gs_colour(GroupMap g, const BSlot *__restrict__ S, int i, int backward,
                              double sor) {
   BSLOT;
   const int q = backward ? x.nq - 1 - i : i;
   const int b0 = x.gq[q];
-  d_gs_level<3>(bx, x.sys, nullptr, b0, x.gq[q + 1] - b0, sor, x.gctl->active);
+  d_gs_level<3>(bx, x.sys, nullptr, b0, x.gq[q + 1] - b0, sor, !backward && i == x.nq - 1 ? 2 : 1,
+                x.gctl->active);
 }
 // flags[k]: case k's momentum solve is still running
 __global__ void gb_gs_flags(int n, const BSlot *__restrict__ S, int *flags) {
@@ -2169,8 +2185,7 @@ struct cfdl_ctx {
   std::vector<int> co;  // subdomain cell offsets (nsubd+1)
   Sched pcl;            // pc system by forward level (CFDL_GS_MODE=level)
   // colour order of the pc smoother (cfdl_set_pc_order, an extension): the
-  // colours of a greedy colouring in each subdomain's local order, as levels
-  Sched pcc;
+  // colours of a greedy colouring of each subdomain in global cell order
   std::vector<ColRanges> pcc_rng;  // per colour, its range in each subdomain
   bool pc_hex = false;             // every pc row has six entries (row e at 6e)
   int pc_order = CFDL_PC_REFERENCE;
@@ -2314,10 +2329,10 @@ static int sweep(cfdl_ctx *c, const Sched &s, const SysDesc &sys, int nc, double
     const int n = s.ptr[l + 1] - s.ptr[l];
     if (nc == 3)
       hipLaunchKernelGGL(k_gs_level<3>, dim3(nblocks(n)), dim3(kBlock), 0, c->st, sys,
-                         s.cells + s.ptr[l], 0, n, sor, active);
+                         s.cells + s.ptr[l], 0, n, sor, 1, active);
     else
       hipLaunchKernelGGL(k_gs_level<1>, dim3(nblocks(n)), dim3(kBlock), 0, c->st, sys,
-                         s.cells + s.ptr[l], 0, n, sor, active);
+                         s.cells + s.ptr[l], 0, n, sor, 1, active);
   }
   c->gs_launches += s.nlev;
   HIPCHK(hipGetLastError());
@@ -2364,7 +2379,7 @@ static int pc_sweep(cfdl_ctx *c, const Sched &s, const SysDesc &sys, bool forwar
     const int l = forward ? i : s.nlev - 1 - i;
     const int n = s.ptr[l + 1] - s.ptr[l];
     hipLaunchKernelGGL(k_gs_level<1>, dim3(nblocks(n)), dim3(kBlock), 0, c->st, sys,
-                       s.cells + s.ptr[l], 0, n, 1.02, active);
+                       s.cells + s.ptr[l], 0, n, 1.02, 1, active);
   }
   CALL(sample_end(c, smp, s.nlev, c->ne));
   c->pc_launches += s.nlev;
@@ -2374,24 +2389,54 @@ static int pc_sweep(cfdl_ctx *c, const Sched &s, const SysDesc &sys, bool forwar
   return CFDL_OK;
 }
 
-// An FP32 colour sweep of the mixed-precision correction system (sor 1.02 in
-// single precision), colours in order forward and in reverse backward.
-static int pc_sweep32(cfdl_ctx *c, const SysDesc32 &sys, bool forward, const int *active) {
+// The launches of nsym symmetric sweeps over nq colours (colours in order,
+// then in reverse, nsym times): consecutive updates of the same colour, at
+// every turn, are one launch of several updates.  At two colours the two
+// symmetric iterations of a pc block are 5 launches instead of 8, a solve_gs
+// iteration 3 instead of 4.  A colour's updates can share a pass because its
+// cells are not neighbours; the greedy colouring guarantees that while it
+// needs at most 64 colours (beyond, each update keeps its own launch).  The
+// sweeps are bound by memory, so an update without a row read costs only its
+// divisions: ten outer iterations of the 96^3 cavity in colour order took
+// 61.5 ms with a launch per update and 45.6 ms with these, twelve of the
+// 128^3 cavity in the mixed mode 116.3 ms and 89.3 ms.
+struct ColourTurn {
+  int q, reps;
+};
+static std::vector<ColourTurn> fused_turns(int nq, int nsym) {
+  std::vector<ColourTurn> t;
+  for (int i = 0; i < 2 * nsym * nq; i++) {
+    const int j = i % nq, q = (i / nq) % 2 == 0 ? j : nq - 1 - j;
+    if (!t.empty() && t.back().q == q && nq <= 64)
+      t.back().reps++;
+    else
+      t.push_back(ColourTurn{q, 1});
+  }
+  return t;
+}
+
+// The two symmetric iterations of a pc block in colour order (sor 1.02, in
+// single precision for the mixed mode's correction system).
+template <typename T>
+static int pc_block_colour(cfdl_ctx *c, const ColSys<T> &sys, const int *active) {
+  const T sor = sizeof(T) == 8 ? static_cast<T>(1.02) : static_cast<T>(1.02f);
   cfdl_ctx::Sample *smp = nullptr;
   CALL(sample_begin(c, &smp));
-  const int nl = static_cast<int>(c->pcc_rng.size());
-  for (int i = 0; i < nl; i++) {
-    const ColRanges &cr = c->pcc_rng[forward ? i : nl - 1 - i];
+  const std::vector<ColourTurn> turns = fused_turns(static_cast<int>(c->pcc_rng.size()), 2);
+  for (const ColourTurn &t : turns) {
+    const ColRanges &cr = c->pcc_rng[t.q];
+    const dim3 g(nblocks(cr.off[cr.n]));
     if (c->pc_hex)
-      hipLaunchKernelGGL(k_gs_level32<true>, dim3(nblocks(cr.off[cr.n])), dim3(kBlock), 0, c->st,
-                         sys, cr, 1.02f, active);
+      hipLaunchKernelGGL((k_pc_colour<T, true>), g, dim3(kBlock), 0, c->st, sys, cr, sor, t.reps,
+                         active);
     else
-      hipLaunchKernelGGL(k_gs_level32<false>, dim3(nblocks(cr.off[cr.n])), dim3(kBlock), 0,
-                         c->st, sys, cr, 1.02f, active);
+      hipLaunchKernelGGL((k_pc_colour<T, false>), g, dim3(kBlock), 0, c->st, sys, cr, sor, t.reps,
+                         active);
   }
-  CALL(sample_end(c, smp, nl, c->ne));
+  const int nl = static_cast<int>(turns.size());
+  CALL(sample_end(c, smp, nl, 4 * int64_t{c->ne}));
   c->pc_launches += nl;
-  c->pc_cells += c->ne;
+  c->pc_cells += 4 * int64_t{c->ne};
   c->gs_launches += nl;
   HIPCHK(hipGetLastError());
   return CFDL_OK;
@@ -2554,20 +2599,20 @@ static int solve_gs_n(cfdl_ctx *c, int ny, double **phi, const double **b,
   // one SysDesc per sweep kernel with its RHS subset in slots 0..ny-1
   for (int it = 0; it < c->nit; it++) {
     if (gcol) {
-      // colours in order, then in reverse; one launch per colour
-      const int nq = static_cast<int>(c->gcol_ptr.size()) - 1;
-      for (int d = 0; d < 2; d++)
-        for (int i = 0; i < nq; i++) {
-          const int q = d == 0 ? i : nq - 1 - i;
-          const int b0 = c->gcol_ptr[q], n = c->gcol_ptr[q + 1] - b0;
-          if (ny == 3)
-            hipLaunchKernelGGL(k_gs_level<3>, dim3(nblocks(n)), dim3(kBlock), 0, c->st, s,
-                               static_cast<const int *>(nullptr), b0, n, sor, gs_active(c));
-          else
-            hipLaunchKernelGGL(k_gs_level<1>, dim3(nblocks(n)), dim3(kBlock), 0, c->st, s,
-                               static_cast<const int *>(nullptr), b0, n, sor, gs_active(c));
-        }
-      c->gs_launches += 2 * nq;
+      // colours in order, then in reverse; one launch per colour, the turn's
+      // two updates of the last colour in one
+      const std::vector<ColourTurn> turns =
+          fused_turns(static_cast<int>(c->gcol_ptr.size()) - 1, 1);
+      for (const ColourTurn &t : turns) {
+        const int b0 = c->gcol_ptr[t.q], n = c->gcol_ptr[t.q + 1] - b0;
+        if (ny == 3)
+          hipLaunchKernelGGL(k_gs_level<3>, dim3(nblocks(n)), dim3(kBlock), 0, c->st, s,
+                             static_cast<const int *>(nullptr), b0, n, sor, t.reps, gs_active(c));
+        else
+          hipLaunchKernelGGL(k_gs_level<1>, dim3(nblocks(n)), dim3(kBlock), 0, c->st, s,
+                             static_cast<const int *>(nullptr), b0, n, sor, t.reps, gs_active(c));
+      }
+      c->gs_launches += static_cast<int>(turns.size());
       HIPCHK(hipGetLastError());
     } else if (tiled) {
       const int nl = static_cast<int>(c->tm.launch_ptr.size()) - 1;
@@ -2637,7 +2682,8 @@ static int multi_subdomain_solver(cfdl_ctx *c) {
   // correction is added to the FP64 values and cleared, and the FP64 true
   // residual gives both the stop test's norms and the next r.
   const int nall = ne + c->nh;
-  SysDesc32 s32{rowp, nbrp, c->a32, c->anb32, c->r32, c->d32};
+  const ColSys<float> s32{rowp, nbrp, c->a32, c->anb32, c->r32, c->d32};
+  const ColSys<double> s64{rowp, nbrp, c->ap_p, c->anb_p, c->b_p, c->phic_p};
   if (mixed)
     hipLaunchKernelGGL(k_mixed_prep, dim3(std::min(nblocks(std::max(c->Lp, nall)), 4096)),
                        dim3(kBlock), 0, c->st,
@@ -2649,14 +2695,11 @@ static int multi_subdomain_solver(cfdl_ctx *c) {
   const int *act = pc_active(c);
   const int nblock = (c->nit + 1) / 2;
   for (int blk = 1; blk <= nblock; blk++) {
-    for (int rep = 0; rep < 2; rep++) {  // smoother_gs(..., 2): two symmetric iterations
-      if (mixed) {
-        CALL(pc_sweep32(c, s32, true, act));
-        CALL(pc_sweep32(c, s32, false, act));
-      } else if (c->pc_order == CFDL_PC_COLORED) {
-        CALL(pc_sweep(c, c->pcc, s1, true, act));
-        CALL(pc_sweep(c, c->pcc, s1, false, act));
-      } else if (c->tiled) {
+    // smoother_gs(..., 2): two symmetric iterations
+    if (mixed) CALL(pc_block_colour(c, s32, act));
+    if (c->pc_order == CFDL_PC_COLORED) CALL(pc_block_colour(c, s64, act));
+    for (int rep = 0; rep < 2 && !col; rep++) {
+      if (c->tiled) {
         CALL(pc_sweep_tiled(c, s1, true, act));
         CALL(pc_sweep_tiled(c, s1, false, act));
       } else {
@@ -3392,11 +3435,11 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
     for (size_t j = 0; j < xsrc_old.size(); j++) xsrcc[j] = o2c[xsrc_old[j]];
     CALL(build_tile_tables(C, rowp, nbrp, sdn, launchn, tidn, levn, 1, &C->ts));
     CALL(make_sched(C, levn, ne, &C->pcl));
-    CALL(make_sched(C, coln, ne, &C->pcc));
+    const int ncol = *std::max_element(coln.begin(), coln.end());
     // the same colours as ranges per subdomain (colour numbering is
     // subdomain-major, colour-minor)
-    C->pcc_rng.assign(C->pcc.nlev, ColRanges{});
-    for (int l = 0; l < C->pcc.nlev; l++) {
+    C->pcc_rng.assign(ncol, ColRanges{});
+    for (int l = 0; l < ncol; l++) {
       ColRanges &cr = C->pcc_rng[l];
       cr.n = nsubd;
       cr.off[0] = 0;
@@ -4388,8 +4431,9 @@ int seg_gs(cfdl_batch *b, int blk, int slot) {
   hipStream_t st = b->st;
   int nq = 0;
   for (cfdl_ctx *c : b->ctx) nq = std::max(nq, static_cast<int>(c->gcol_ptr.size()) - 1);
+  // (the backward sweep's first colour is updated with the forward sweep's last)
   for (int d = 0; d < 2; d++)
-    for (int i = 0; i < nq; i++) {
+    for (int i = d; i < nq; i++) {
       const int nb = L.map([&](cfdl_ctx *c) {
         const int q_n = static_cast<int>(c->gcol_ptr.size()) - 1;
         if (i >= q_n) return 0;
