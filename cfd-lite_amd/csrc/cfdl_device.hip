@@ -32,6 +32,7 @@
 #include <cstddef>
 #include <cstring>
 #include <type_traits>
+#include <future>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -2743,59 +2744,103 @@ static int multi_subdomain_solver(cfdl_ctx *c) {
   return CFDL_OK;
 }
 
-// Dense ids of spatial tiles of about edge[0] x edge[1] x edge[2] cells
-// (x, y, z): bins of the cell centres in the bounding box of each group of
-// positions [grp[s], grp[s+1]) (the subdomains of the pc system, or all
-// cells); tiles never cross groups.  cell[q] is the mesh cell at position q.
+// Mean distance between the centres of neighbouring cells along each axis
+// (each pair counted on the axis of its largest component; an axis without
+// pairs gets the cube root of the mean cell volume).
+static void cell_spacing(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
+                         const double *xc, const double *yc, const double *zc, const double *vol,
+                         double *h) {
+  double sum[3] = {0.0, 0.0, 0.0}, vsum = 0.0;
+  int64_t cnt[3] = {0, 0, 0};
+  for (int e = 0; e < ne; e++) {
+    vsum += vol[e];
+    for (int k = row[e]; k < row[e + 1]; k++) {
+      const int d = nbr[k];
+      if (d >= ne || d < e) continue;
+      const double r[3] = {std::fabs(xc[d] - xc[e]), std::fabs(yc[d] - yc[e]),
+                           std::fabs(zc[d] - zc[e])};
+      const int i = r[0] >= r[1] && r[0] >= r[2] ? 0 : r[1] >= r[2] ? 1 : 2;
+      sum[i] += r[i];
+      cnt[i]++;
+    }
+  }
+  for (int i = 0; i < 3; i++) h[i] = sum[i] > 0.0 ? sum[i] / cnt[i] : std::cbrt(vsum / ne);
+}
+
+// Dense ids of spatial tiles of edge[0] x edge[1] x edge[2] cell layers
+// (x, y, z): a cell's layer along an axis is its centre's distance from the
+// first one's in its group of positions [grp[s], grp[s+1]) (the subdomains of
+// the pc system, or all cells), in units of the cell spacing h, rounded to the
+// nearest.  Rounding puts the cuts between layers: a cut through a layer's
+// centres would leave a ragged face on meshes with distorted cells, where a
+// dependency chain along the face changes tile at every other cell, one
+// launch each (on the 61 x 47 x 53 box with vertices moved by 0.15 h, 69
+// launches a sweep instead of 19).  Tiles never cross groups.  cell[q] is the
+// mesh cell at position q.
 static void bin_tiles(const std::vector<int> &grp, const std::vector<int> &cell, const double *xc,
-                      const double *yc, const double *zc, const double *vol, const int *edge,
+                      const double *yc, const double *zc, const double *h, const int *edge,
                       std::vector<int> *tid) {
   std::unordered_map<int64_t, int> tid_of;
   tid->assign(cell.size(), 0);
   for (size_t s = 0; s + 1 < grp.size(); s++) {
-    double lo[3] = {1e300, 1e300, 1e300}, vsum = 0.0;
+    double lo[3] = {1e300, 1e300, 1e300};
     for (int q = grp[s]; q < grp[s + 1]; q++) {
       const int g = cell[q];
       const double r[3] = {xc[g], yc[g], zc[g]};
       for (int i = 0; i < 3; i++) lo[i] = std::min(lo[i], r[i]);
-      vsum += vol[g];
     }
-    const double h = std::cbrt(vsum / (grp[s + 1] - grp[s]));
-    const double hx = h * edge[0], hy = h * edge[1], hz = h * edge[2];
+    int64_t last_key = -1;
+    int last = 0;
     for (int q = grp[s]; q < grp[s + 1]; q++) {
       const int g = cell[q];
-      const int64_t bx = static_cast<int64_t>((xc[g] - lo[0]) / hx);
-      const int64_t by = static_cast<int64_t>((yc[g] - lo[1]) / hy);
-      const int64_t bz = static_cast<int64_t>((zc[g] - lo[2]) / hz);
-      const int64_t key = ((static_cast<int64_t>(s) * 4096 + bx) * 4096 + by) * 4096 + bz;
-      auto it = tid_of.find(key);
-      if (it == tid_of.end()) it = tid_of.emplace(key, static_cast<int>(tid_of.size())).first;
-      (*tid)[q] = it->second;
+      const double r[3] = {xc[g], yc[g], zc[g]};
+      int64_t key = static_cast<int64_t>(s);
+      for (int i = 0; i < 3; i++) {
+        const int64_t layer = static_cast<int64_t>((r[i] - lo[i]) / h[i] + 0.5);
+        key = key * (1 << 19) + layer / edge[i] % (1 << 19);
+      }
+      if (key != last_key) {
+        last = tid_of.emplace(key, static_cast<int>(tid_of.size())).first->second;
+        last_key = key;
+      }
+      (*tid)[q] = last;
     }
   }
 }
 
 // Space-time tiles of the pressure-correction sweeps, on the pc system in
 // its set-up order (cells 0..ne-1, halo slots >= ne).  lev is each cell's
-// forward dependency level inside its subdomain and tid its spatial tile
-// (dense ids; a tile never crosses subdomains).  In the forward sweep's
-// processing order (increasing level) each cell gets launch = max over the
-// neighbours it depends on of (their launch, +1 when the neighbour lies in
-// another tile).  So a dependency between two tiles always spans launches,
-// and inside one launch a tile's cells only depend on earlier cells of the
-// same tile.  A (launch, tile) batch spans fewer than `span` levels: a cell
-// that would stretch its batch further moves to the tile's batch in a later
-// launch.
-static void tile_launches(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
-                          const std::vector<int> &lev, const std::vector<int> &tid, int span,
-                          std::vector<int> *launch) {
-  std::vector<int> order(ne);
-  for (int e = 0; e < ne; e++) order[e] = e;
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return lev[a] < lev[b]; });
-  int64_t ntile = 1;
-  for (int e = 0; e < ne; e++) ntile = std::max<int64_t>(ntile, tid[e] + 1);
-  std::unordered_map<int64_t, int> first_level;  // (launch, tile) -> its first level
+// forward dependency level inside its subdomain, order the cells by level and
+// tid the spatial tile (dense ids; a tile never crosses subdomains).  In the
+// forward sweep's processing order (increasing level) each cell gets launch =
+// max over the neighbours it depends on of (their launch, +1 when the
+// neighbour lies in another tile).  So a dependency between two tiles always
+// spans launches, and inside one launch a tile's cells only depend on earlier
+// cells of the same tile.  A (launch, tile) batch spans fewer than `span`
+// levels: a cell that would stretch its batch further moves to the tile's
+// batch in a later launch.
+// Returns a sweep's time in microseconds for nrhs (1 or 3) right-hand sides by
+// this model: every launch costs its boundary and, per round of resident
+// workgroups (as many per CU as its LDS holds the largest batch of), the
+// gather (a latency and the largest batch's cells) and the levels of its
+// longest batch.  A schedule with a segment wider than a wavefront loses the
+// pipelined walk, and so counts three times.  The constants fit the measured
+// sweeps of the 16^3, 32^3, 64^3 and 128^3 cavities and the 61 x 47 x 53 box
+// in seven shapes each to within 10%.
+constexpr double kLaunchUs = 1.4, kGatherUs = 0.9, kCellUs = 1.0 / 512;
+static double tile_launches(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
+                            const std::vector<int> &lev, const std::vector<int> &order,
+                            const std::vector<int> &tid, int span, int nrhs,
+                            std::vector<int> *launch) {
+  int ntile = 1;
+  for (int e = 0; e < ne; e++) ntile = std::max(ntile, tid[e] + 1);
+  struct Batch {
+    int first = -1, last = -1;  // levels
+    int cells = 0, levels = 0, seg = 0, segmax = 0;
+  };
+  std::vector<std::vector<Batch>> bat(ntile);  // per tile, by launch
   launch->assign(ne, 0);
+  int nl = 0;
   for (int e : order) {
     int L = 0;
     for (int k = row[e]; k < row[e + 1]; k++) {
@@ -2803,17 +2848,88 @@ static void tile_launches(int ne, const std::vector<int> &row, const std::vector
       if (d >= ne || lev[d] >= lev[e]) continue;  // halo, or visited after e
       L = std::max(L, (*launch)[d] + (tid[d] != tid[e] ? 1 : 0));
     }
-    for (;;) {
-      const int64_t key = static_cast<int64_t>(L) * ntile + tid[e];
-      auto it = first_level.find(key);
-      if (it == first_level.end()) {
-        first_level.emplace(key, lev[e]);
-        break;
-      }
-      if (lev[e] - it->second < span) break;
-      L++;
+    std::vector<Batch> &tb = bat[tid[e]];
+    for (;; L++) {
+      if (static_cast<int>(tb.size()) <= L) tb.resize(L + 1);
+      if (tb[L].first < 0) tb[L].first = lev[e];
+      if (lev[e] - tb[L].first < span) break;
     }
     (*launch)[e] = L;
+    Batch &b = tb[L];
+    if (lev[e] != b.last) b.levels++, b.seg = 0;
+    b.last = lev[e];
+    b.cells++;
+    b.segmax = std::max(b.segmax, ++b.seg);
+    nl = std::max(nl, L + 1);
+  }
+  std::vector<int> nb(nl, 0), longest(nl, 0);
+  int cells = 1, seg = 0;
+  for (const auto &tb : bat)
+    for (size_t L = 0; L < tb.size(); L++)
+      if (tb[L].cells > 0) {
+        nb[L]++;
+        longest[L] = std::max(longest[L], tb[L].levels);
+        cells = std::max(cells, tb[L].cells);
+        seg = std::max(seg, tb[L].segmax);
+      }
+  // LDS of a batch cell: coefficients, addresses, values and right-hand sides,
+  // and about 0.7 outside neighbours
+  const double fit = 160.0 * 1024 / (80 + 21.6 * nrhs) / cells;
+  const double batch_us = kGatherUs + kCellUs * cells, level_us = nrhs == 1 ? 0.15 : 0.26;
+  double us = 0.0;
+  for (int L = 0; L < nl; L++)
+    us += kLaunchUs + std::ceil(nb[L] / (256.0 * std::max(1.0, std::floor(fit)))) *
+                          (batch_us + level_us * longest[L]);
+  return seg > kLdsThreads || fit < 1.0 ? 3.0 * us : us;
+}
+
+// A tile shape and the levels its batches may span
+struct TileShape {
+  int edge[3], span;
+};
+// The shapes a schedule is chosen from (CFDL_TILE / CFDL_TILE_SPAN replace
+// them): the model's best ones over cavities, jittered and odd boxes.  Small
+// batches (512 cells, several per CU) and large ones (1020 cells of at most
+// 60 a level: fewer launches, one batch per CU) each win on some meshes.
+// Runs of the reference order against one fixed 16 x 8 x 4 shape cut at the
+// first cell's centre: 16^3 13.1 -> 11.7 ms, 32^3 54.9 -> 46.2 ms, the
+// distorted 61 x 47 x 53 box 231 -> 72 ms, 128^3 352 -> 332 ms.
+constexpr TileShape kTileShapes[] = {{{16, 8, 4}, 32}, {{16, 16, 4}, 32}, {{16, 16, 4}, 20},
+                                     {{8, 8, 8}, 32},  {{12, 8, 8}, 32}};
+static void plan_tiles(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
+                       const std::vector<int> &lev, const std::vector<int> &grp,
+                       const std::vector<int> &cell, const double *xc, const double *yc,
+                       const double *zc, const double *h, int nrhs,
+                       const std::vector<TileShape> &shapes, std::vector<int> *tid,
+                       std::vector<int> *launch) {
+  // cells by level (stable: in set-up order within a level)
+  std::vector<int> start(*std::max_element(lev.begin(), lev.end()) + 2, 0), order(ne);
+  for (int e = 0; e < ne; e++) start[lev[e] + 1]++;
+  for (size_t l = 1; l < start.size(); l++) start[l] += start[l - 1];
+  for (int e = 0; e < ne; e++) order[start[lev[e]]++] = e;
+  struct Plan {
+    std::vector<int> tid, launch;
+    double us;
+  };
+  std::vector<std::future<Plan>> plans;  // one host thread per shape
+  for (const TileShape &s : shapes)
+    plans.push_back(std::async([&, s] {
+      Plan p;
+      bin_tiles(grp, cell, xc, yc, zc, h, s.edge, &p.tid);
+      p.us = tile_launches(ne, row, nbr, lev, order, p.tid, s.span, nrhs, &p.launch);
+      return p;
+    }));
+  double best = 0.0;
+  for (size_t i = 0; i < shapes.size(); i++) {
+    Plan p = plans[i].get();
+    if (trace_on())
+      std::fprintf(stderr, "cfdl: tiles %dx%dx%d span %d: %d launches, %.0f us a sweep\n",
+                   shapes[i].edge[0], shapes[i].edge[1], shapes[i].edge[2], shapes[i].span,
+                   *std::max_element(p.launch.begin(), p.launch.end()) + 1, p.us);
+    if (i > 0 && p.us >= best) continue;
+    best = p.us;
+    tid->swap(p.tid);
+    launch->swap(p.launch);
   }
 }
 
@@ -3193,25 +3309,26 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
   C->en = EnergyDev{F[CFDL_T], F[CFDL_GT], F[CFDL_ENTH], F[CFDL_ENTH0], F[CFDL_GENTH]};
   hipLaunchKernelGGL(k_energy_init, dim3(nblocks(n)), dim3(kBlock), 0, C->st, C->md, C->en);
   trace("ctx_create: fields");
-  // sweep schedules: spatial tiles of edge[0] x edge[1] x edge[2] cells
-  // (CFDL_TILE = "A" for A^3 or "AxBxC"), batches spanning fewer than `span`
-  // levels; CFDL_GS_MODE=level keeps one launch per level.  16 x 8 x 4 cells
-  // and 32 levels measured fastest on the 128^3 cavity (fewest launches
-  // whose batches keep level segments within 64 cells and LDS within half
-  // a CU's, so two batches fit per CU).
-  int edge[3] = {16, 8, 4};
-  if (const char *te = std::getenv("CFDL_TILE")) {
+  // sweep schedules: the best of kTileShapes by the model of tile_launches,
+  // or the one CFDL_TILE ("A" for A^3 or "AxBxC") and CFDL_TILE_SPAN name;
+  // CFDL_GS_MODE=level keeps one launch per level
+  std::vector<TileShape> shapes(std::begin(kTileShapes), std::end(kTileShapes));
+  const char *te = std::getenv("CFDL_TILE"), *sp = std::getenv("CFDL_TILE_SPAN");
+  if (te || sp) {
+    TileShape f = shapes[0];
     int a = 0, b = 0, d = 0;
-    const int n = std::sscanf(te, "%dx%dx%d", &a, &b, &d);
-    if (n == 3) {
-      edge[0] = a, edge[1] = b, edge[2] = d;
-    } else if (n >= 1) {
-      edge[0] = edge[1] = edge[2] = a;
+    const int k = te ? std::sscanf(te, "%dx%dx%d", &a, &b, &d) : 0;
+    if (k == 3) {
+      f.edge[0] = a, f.edge[1] = b, f.edge[2] = d;
+    } else if (k >= 1) {
+      f.edge[0] = f.edge[1] = f.edge[2] = a;
     }
-    for (int i = 0; i < 3; i++) edge[i] = std::max(1, edge[i]);
+    for (int i = 0; i < 3; i++) f.edge[i] = std::max(1, f.edge[i]);
+    if (sp) f.span = std::min(63, std::max(1, std::atoi(sp)));
+    shapes.assign(1, f);
   }
-  const char *sp = std::getenv("CFDL_TILE_SPAN");
-  const int span = sp ? std::min(63, std::max(1, std::atoi(sp))) : 32;
+  double hmean[3];
+  cell_spacing(ne, row, nbr, xc, yc, zc, vol, hmean);
   const char *mode = std::getenv("CFDL_GS_MODE");
   C->tiled = !(mode && std::string(mode) == "level");
   const char *rc = std::getenv("CFDL_TILE_RCP");
@@ -3225,8 +3342,7 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
       // the global system in tile numbering, for the tiled solve_gs
       std::vector<int> all(ne), grp{0, ne}, tid, launch;
       for (int e = 0; e < ne; e++) all[e] = e;
-      bin_tiles(grp, all, xc, yc, zc, vol, edge, &tid);
-      tile_launches(ne, row, nbr, lev, tid, span, &launch);
+      plan_tiles(ne, row, nbr, lev, grp, all, xc, yc, zc, hmean, 3, shapes, &tid, &launch);
       std::vector<int> n2o(all), o2n(ne);
       std::stable_sort(n2o.begin(), n2o.end(), [&](int x, int y) {
         if (launch[x] != launch[y]) return launch[x] < launch[y];
@@ -3355,10 +3471,9 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
     C->pc_nlev = 0;
     for (int s = 0; s < nsubd; s++) levels(rowo, nbro, C->co[s], C->co[s + 1], true, lev);
     for (int q = 0; q < ne; q++) C->pc_nlev = std::max(C->pc_nlev, lev[q]);
-    std::vector<int> tid;
-    bin_tiles(C->co, l2g, xc, yc, zc, vol, edge, &tid);
-    std::vector<int> launch;
-    tile_launches(ne, rowo, nbro, lev, tid, span, &launch);
+    std::vector<int> tid, launch;
+    plan_tiles(ne, rowo, nbro, lev, C->co, l2g, xc, yc, zc, hmean, 1, shapes, &tid,
+               &launch);
     // renumber the pc system by (subdomain, launch, tile, level): every
     // (launch, tile) batch of the tiled sweeps becomes a contiguous range
     std::vector<int> n2o(ne), o2n(ne);
