@@ -9,12 +9,12 @@
 //    calc_coef_p, no copies), vectors in the global cell order.  Every dot
 //    product and norm is a blocked reduction of fixed shape: block x of 256
 //    lanes owns a contiguous chunk, lane t sums its strided elements in
-//    order, the lanes combine as s[t] += s[t+h] for h = 128, 64 (LDS) and
-//    32 .. 1 (wavefront shuffles), and the last block to finish (a ticket
-//    counter) combines the block sums in the same way and does the scalar
-//    work (alpha, beta, the stop test) in the same launch.  So each CG
-//    iteration is four launches besides the preconditioner, and the result
-//    does not depend on scheduling.
+//    order (1024 threads compute them), the lanes combine as
+//    s[t] += s[t+h] for h = 128, 64 (LDS) and 32 .. 1 (wavefront shuffles),
+//    and the last block to finish (a ticket counter) combines the block sums
+//    in the same way and does the scalar work (alpha, beta, the stop test)
+//    in the same launch.  So each CG iteration is four launches besides the
+//    preconditioner, and the result does not depend on scheduling.
 //  * The preconditioner is one V-cycle of agglomeration multigrid (the
 //    hierarchy of cfdl_mg.cpp): Galerkin coarse operators summed once per
 //    solve from lists (no atomics), one forward colour Gauss-Seidel sweep
@@ -59,7 +59,15 @@ namespace {
     }                                                                               \
   } while (0)
 
-constexpr int kRed = 256;          // lanes per reduction block
+constexpr int kRed = 256;          // lanes of a blocked sum
+// Threads of a reduction block.  The blocked sums fix 256 lanes a block and
+// 4,096 elements a block, which is 2 wavefronts a SIMD on a 128^3 mesh: too
+// few loads in flight.  Four lane groups compute the elements of a block, its
+// 256 lanes add them in order (blocked_acc).  With the partials passed without
+// fences (put_part), at 128^3: A p with p.q 78 -> 35 us, the update 57 -> 22
+// us, r.z 36 -> 9 us.
+constexpr int kRedThreads = 1024;
+constexpr int kRedSeg = 16 * kRed;  // elements staged in LDS at a time
 constexpr int kMaxRedBlocks = 1024;
 constexpr int kBlk = 256;          // lanes per block of the grid-wide V-cycle kernels
 constexpr int kCoarseMax = 4096;   // levels at most this large run in one workgroup
@@ -85,10 +93,11 @@ Red red_of(int n) {
 }
 
 // s[t] += s[t+h], h = 128, 64 in LDS, then 32 .. 1 by shuffles in wave 0;
-// lane 0 returns the block's sum (the same pairing as the LDS tree)
+// v from threads 0 .. 255, the block's sum in thread 0 (the pairing of an LDS
+// tree)
 __device__ inline double tree_sum(double v, double *s) {
   const int t = threadIdx.x;
-  s[t] = v;
+  if (t < kRed) s[t] = v;
   __syncthreads();
   if (t < 128) s[t] = s[t] + s[t + 128];
   __syncthreads();
@@ -101,43 +110,76 @@ __device__ inline double tree_sum(double v, double *s) {
   __syncthreads();
   return x;
 }
-__device__ inline double tree_max(double v, double *s) {
+// the maximum over all kRedThreads threads (the same in any order), in thread 0
+__device__ inline double block_max(double v, double *s) {
   const int t = threadIdx.x;
-  s[t] = v;
-  __syncthreads();
-  if (t < 128) s[t] = fmax(s[t], s[t + 128]);
-  __syncthreads();
-  double x = 0.0;
-  if (t < 64) {
-    x = fmax(s[t], s[t + 64]);
 #pragma unroll
-    for (int h = 32; h >= 1; h >>= 1) x = fmax(x, __shfl_down(x, h, 64));
-  }
+  for (int h = 32; h >= 1; h >>= 1) v = fmax(v, __shfl_down(v, h, 64));
+  if (t % 64 == 0) s[t / 64] = v;
   __syncthreads();
-  return x;
+  if (t == 0)
+    for (int w = 1; w < kRedThreads / 64; w++) v = fmax(v, s[w]);
+  __syncthreads();
+  return v;
 }
 
-// Writes this block's partial(s) and returns true in every lane of the last
-// block to arrive, after which the partials of all blocks are visible.
+// Lane t's sum (threads 0 .. 255) of f(i) over i = lo + t, lo + t + 256, ... <
+// hi, in that order from 0: all threads of the block evaluate f, once per i,
+// into LDS (s: kRedSeg doubles), a segment at a time, and the lanes add.
+template <typename F>
+__device__ inline double blocked_acc(int lo, int hi, double *s, F f) {
+  const int t = threadIdx.x;
+  double acc = 0.0;
+  for (int base = lo; base < hi; base += kRedSeg) {
+    const int n = min(kRedSeg, hi - base);
+#pragma unroll
+    for (int j = 0; j < kRedSeg / kRedThreads; j++) {
+      const int o = t + j * kRedThreads;
+      if (o < n) s[o] = f(base + o);
+    }
+    __syncthreads();
+    if (t < kRed)
+      for (int o = t; o < n; o += kRed) acc = acc + s[o];
+    __syncthreads();
+  }
+  return acc;
+}
+
+// Block partials pass through memory at agent scope (stores and loads that
+// bypass the XCD's L2), so no block needs a fence: a fence writes back and
+// invalidates an L2, per wavefront that executes it, which took longer than
+// the sums (with 16 wavefronts a block each of the three kernels took 100 to
+// 130 us more at 128^3).
+__device__ inline void put_part(double *part, double v) {
+  __hip_atomic_store(part, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline double get_part(const double *part) {
+  return __hip_atomic_load(part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Returns true in every thread of the last block to arrive, which then sees
+// the partials of all blocks.  Thread 0 wrote this block's; it waits until
+// they are in memory before it takes the ticket.
 __device__ inline bool arrive_last(CgCtl *c, int nblk) {
   __shared__ int last;
-  __threadfence();
+  if (threadIdx.x == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(&c->ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+           nblk - 1;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) last = atomicAdd(&c->ticket, 1) == nblk - 1;
-  __syncthreads();
-  if (last) __threadfence();
   return last;
 }
 // the last block's sum of the nblk partials part[k * stride]
 __device__ inline double final_sum(const double *part, int nblk, int stride, double *s) {
   double acc = 0.0;
-  for (int i = threadIdx.x; i < nblk; i += kRed) acc = acc + part[i * stride];
+  if (threadIdx.x < kRed)
+    for (int i = threadIdx.x; i < nblk; i += kRed) acc = acc + get_part(part + i * stride);
   return tree_sum(acc, s);
 }
 __device__ inline double final_max(const double *part, int nblk, int stride, double *s) {
   double acc = 0.0;
-  for (int i = threadIdx.x; i < nblk; i += kRed) acc = fmax(acc, part[i * stride]);
-  return tree_max(acc, s);
+  for (int i = threadIdx.x; i < nblk; i += kRedThreads) acc = fmax(acc, get_part(part + i * stride));
+  return block_max(acc, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -155,20 +197,19 @@ __device__ inline void d_cg_init(int bx, Red R, const int *__restrict__ row,
                                  const double *__restrict__ phi, double *__restrict__ r,
                                  T *__restrict__ rt, T *__restrict__ z, CgCtl *c, double *part,
                                  int nit) {
-  __shared__ double s[kRed];
+  __shared__ double s[kRedSeg];
   const int lo = bx * R.chunk, hi = min(lo + R.chunk, R.n);
-  double acc = 0.0;
-  for (int i = lo + threadIdx.x; i < hi; i += kRed) {
+  const double acc = blocked_acc(lo, hi, s, [&](int i) {
     double v = b[i];
     for (int k = row[i]; k < row[i + 1]; k++) v = v + anb[k] * phi[nbr[k]];
     v = v - ap[i] * phi[i];
     r[i] = v;
     if (rt) rt[i] = static_cast<T>(v);
     z[i] = static_cast<T>(0);
-    acc = acc + v * v;
-  }
+    return v * v;
+  });
   const double bs = tree_sum(acc, s);
-  if (threadIdx.x == 0) part[bx] = bs;
+  if (threadIdx.x == 0) put_part(part + bx, bs);
   if (!arrive_last(c, R.nblk)) return;
   const double rr = final_sum(part, R.nblk, 1, s);
   if (threadIdx.x == 0) {
@@ -189,13 +230,13 @@ __device__ inline void d_cg_init(int bx, Red R, const int *__restrict__ row,
 template <typename T>
 __device__ inline void d_cg_rz(int bx, Red R, const double *__restrict__ r,
                                const T *__restrict__ z, CgCtl *c, double *part) {
-  __shared__ double s[kRed];
+  __shared__ double s[kRedSeg];
   if (!c->active) return;
   const int lo = bx * R.chunk, hi = min(lo + R.chunk, R.n);
-  double acc = 0.0;
-  for (int i = lo + threadIdx.x; i < hi; i += kRed) acc = acc + r[i] * static_cast<double>(z[i]);
+  const double acc =
+      blocked_acc(lo, hi, s, [&](int i) { return r[i] * static_cast<double>(z[i]); });
   const double bs = tree_sum(acc, s);
-  if (threadIdx.x == 0) part[bx] = bs;
+  if (threadIdx.x == 0) put_part(part + bx, bs);
   if (!arrive_last(c, R.nblk)) return;
   const double rho = final_sum(part, R.nblk, 1, s);
   if (threadIdx.x == 0) {
@@ -222,11 +263,10 @@ __device__ inline void d_cg_spmv(int bx, Red R, const int *__restrict__ row,
                                  const int *__restrict__ nbr, const double *__restrict__ ap,
                                  const double *__restrict__ anb, const double *__restrict__ p,
                                  double *__restrict__ q, CgCtl *c, double *part) {
-  __shared__ double s[kRed];
+  __shared__ double s[kRedSeg];
   if (!c->active) return;
   const int lo = bx * R.chunk, hi = min(lo + R.chunk, R.n);
-  double acc = 0.0;
-  for (int i = lo + threadIdx.x; i < hi; i += kRed) {
+  const double acc = blocked_acc(lo, hi, s, [&](int i) {
     const int r0 = row[i], r1 = row[i + 1];
     double sm = 0.0;
     if (r1 - r0 == 6) {  // hexahedral row: all loads first, the sum in CSR order
@@ -246,10 +286,10 @@ __device__ inline void d_cg_spmv(int bx, Red R, const int *__restrict__ row,
     }
     const double pi = p[i], qi = ap[i] * pi - sm;
     q[i] = qi;
-    acc = acc + pi * qi;
-  }
+    return pi * qi;
+  });
   const double bs = tree_sum(acc, s);
-  if (threadIdx.x == 0) part[bx] = bs;
+  if (threadIdx.x == 0) put_part(part + bx, bs);
   if (!arrive_last(c, R.nblk)) return;
   const double sigma = final_sum(part, R.nblk, 1, s);
   if (threadIdx.x == 0) {
@@ -268,24 +308,24 @@ __device__ inline void d_cg_update(int bx, Red R, double *__restrict__ phi,
                                    const double *__restrict__ p, const double *__restrict__ q,
                                    double *__restrict__ r, T *__restrict__ rt, T *__restrict__ z,
                                    CgCtl *c, double *part) {
-  __shared__ double s[kRed];
+  __shared__ double s[kRedSeg];
   if (!c->active) return;
   const double alpha = c->alpha;
   const int lo = bx * R.chunk, hi = min(lo + R.chunk, R.n);
-  double acc = 0.0, mx = 0.0;
-  for (int i = lo + threadIdx.x; i < hi; i += kRed) {
+  double mx = 0.0;
+  const double acc = blocked_acc(lo, hi, s, [&](int i) {
     phi[i] = phi[i] + alpha * p[i];
     const double v = r[i] - alpha * q[i];
     r[i] = v;
     if (rt) rt[i] = static_cast<T>(v);
     z[i] = static_cast<T>(0);
-    acc = acc + v * v;
     mx = fmax(mx, fabs(v));
-  }
-  const double bs = tree_sum(acc, s), bm = tree_max(mx, s);
+    return v * v;
+  });
+  const double bs = tree_sum(acc, s), bm = block_max(mx, s);
   if (threadIdx.x == 0) {
-    part[2 * bx] = bs;
-    part[2 * bx + 1] = bm;
+    put_part(part + 2 * bx, bs);
+    put_part(part + 2 * bx + 1, bm);
   }
   if (!arrive_last(c, R.nblk)) return;
   const double rr = final_sum(part, R.nblk, 2, s);
@@ -313,7 +353,7 @@ __device__ inline void d_cg_log(const CgCtl *c, LogLine *log, int *nlog, const L
 }
 
 template <typename T>
-__global__ void __launch_bounds__(kRed)
+__global__ void __launch_bounds__(kRedThreads)
 k_cg_init(Red R, const int *__restrict__ row, const int *__restrict__ nbr,
           const double *__restrict__ ap, const double *__restrict__ anb,
           const double *__restrict__ b, const double *__restrict__ phi, double *__restrict__ r,
@@ -321,7 +361,7 @@ k_cg_init(Red R, const int *__restrict__ row, const int *__restrict__ nbr,
   d_cg_init<T>(blockIdx.x, R, row, nbr, ap, anb, b, phi, r, rt, z, c, part, nit);
 }
 template <typename T>
-__global__ void __launch_bounds__(kRed)
+__global__ void __launch_bounds__(kRedThreads)
 k_cg_rz(Red R, const double *__restrict__ r, const T *__restrict__ z, CgCtl *c, double *part) {
   d_cg_rz<T>(blockIdx.x, R, r, z, c, part);
 }
@@ -329,14 +369,14 @@ template <typename T>
 __global__ void k_cg_p(int n, const T *__restrict__ z, double *__restrict__ p, const CgCtl *c) {
   d_cg_p<T>(blockIdx.x * blockDim.x + threadIdx.x, n, z, p, c);
 }
-__global__ void __launch_bounds__(kRed)
+__global__ void __launch_bounds__(kRedThreads)
 k_cg_spmv(Red R, const int *__restrict__ row, const int *__restrict__ nbr,
           const double *__restrict__ ap, const double *__restrict__ anb,
           const double *__restrict__ p, double *__restrict__ q, CgCtl *c, double *part) {
   d_cg_spmv(blockIdx.x, R, row, nbr, ap, anb, p, q, c, part);
 }
 template <typename T>
-__global__ void __launch_bounds__(kRed)
+__global__ void __launch_bounds__(kRedThreads)
 k_cg_update(Red R, double *__restrict__ phi, const double *__restrict__ p,
             const double *__restrict__ q, double *__restrict__ r, T *__restrict__ rt,
             T *__restrict__ z, CgCtl *c, double *part) {
@@ -630,7 +670,7 @@ __global__ void g_mg_galerkin(GroupMap g, const MgSlot<T> *__restrict__ S, int l
   d_mg_galerkin<T>(bx * blockDim.x + threadIdx.x, F, C);
 }
 template <typename T>
-__global__ void __launch_bounds__(kRed) g_cg_init(GroupMap g, const MgSlot<T> *__restrict__ S) {
+__global__ void __launch_bounds__(kRedThreads) g_cg_init(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
   d_cg_init<T>(bx, x.R, x.row, x.nbr, x.ap, x.anb, x.b, x.phi, x.r, x.rt, x.z, x.ctl, x.part,
@@ -677,7 +717,7 @@ g_mg_coarse(GroupMap g, const MgSlot<T> *__restrict__ S) {
   d_mg_coarse<T>(x.lv, x.lc, x.nlev, x.ctl);
 }
 template <typename T>
-__global__ void __launch_bounds__(kRed) g_cg_rz(GroupMap g, const MgSlot<T> *__restrict__ S) {
+__global__ void __launch_bounds__(kRedThreads) g_cg_rz(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
   d_cg_rz<T>(bx, x.R, x.r, x.z, x.ctl, x.part);
@@ -689,13 +729,13 @@ __global__ void g_cg_p(GroupMap g, const MgSlot<T> *__restrict__ S) {
   d_cg_p<T>(bx * blockDim.x + threadIdx.x, x.ne, x.z, x.p, x.ctl);
 }
 template <typename T>
-__global__ void __launch_bounds__(kRed) g_cg_spmv(GroupMap g, const MgSlot<T> *__restrict__ S) {
+__global__ void __launch_bounds__(kRedThreads) g_cg_spmv(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
   d_cg_spmv(bx, x.R, x.row, x.nbr, x.ap, x.anb, x.p, x.q, x.ctl, x.part);
 }
 template <typename T>
-__global__ void __launch_bounds__(kRed) g_cg_update(GroupMap g, const MgSlot<T> *__restrict__ S) {
+__global__ void __launch_bounds__(kRedThreads) g_cg_update(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
   d_cg_update<T>(bx, x.R, x.phi, x.p, x.q, x.r, x.rt, x.z, x.ctl, x.part);
@@ -976,7 +1016,7 @@ int mgcg_solve(MgCgSolver *s, const MgCgSystem &sys, void *stream) {
     for (int l = 0; l + 1 < s->nlev; l++)
       hipLaunchKernelGGL(k_mg_galerkin<float>, dim3(nb(s->lvf[l + 1].n + s->lvf[l + 1].nnz, kBlk)),
                          dim3(kBlk), 0, st, s->lvf[l], s->lvf[l + 1]);
-    hipLaunchKernelGGL(k_cg_init<float>, dim3(R.nblk), dim3(kRed), 0, st, R, sys.row, sys.nbr,
+    hipLaunchKernelGGL(k_cg_init<float>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.row, sys.nbr,
                        sys.ap, sys.anb, sys.b, static_cast<const double *>(sys.phi), s->r, s->r32,
                        s->z32, s->ctl, s->part, sys.nit);
   } else {
@@ -992,7 +1032,7 @@ int mgcg_solve(MgCgSolver *s, const MgCgSystem &sys, void *stream) {
     for (int l = 0; l + 1 < s->nlev; l++)
       hipLaunchKernelGGL(k_mg_galerkin<double>, dim3(nb(s->lvd[l + 1].n + s->lvd[l + 1].nnz, kBlk)),
                          dim3(kBlk), 0, st, s->lvd[l], s->lvd[l + 1]);
-    hipLaunchKernelGGL(k_cg_init<double>, dim3(R.nblk), dim3(kRed), 0, st, R, sys.row, sys.nbr,
+    hipLaunchKernelGGL(k_cg_init<double>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.row, sys.nbr,
                        sys.ap, sys.anb, sys.b, static_cast<const double *>(sys.phi), s->r,
                        static_cast<double *>(nullptr), s->zd, s->ctl, s->part, sys.nit);
   }
@@ -1004,7 +1044,7 @@ int mgcg_solve(MgCgSolver *s, const MgCgSystem &sys, void *stream) {
   for (int it = 0; it < sys.nit; it++) {
     if (s->fp32) {
       MGCALL(vcycle<float>(s, s->lvf, s->d_lvf, st, s->ctl));
-      hipLaunchKernelGGL(k_cg_rz<float>, dim3(R.nblk), dim3(kRed), 0, st, R,
+      hipLaunchKernelGGL(k_cg_rz<float>, dim3(R.nblk), dim3(kRedThreads), 0, st, R,
                          static_cast<const double *>(s->r), static_cast<const float *>(s->z32),
                          s->ctl, s->part);
       hipLaunchKernelGGL(k_cg_p<float>, dim3(nb(ne, kBlk)), dim3(kBlk), 0, st, ne,
@@ -1012,21 +1052,21 @@ int mgcg_solve(MgCgSolver *s, const MgCgSystem &sys, void *stream) {
                          static_cast<const CgCtl *>(s->ctl));
     } else {
       MGCALL(vcycle<double>(s, s->lvd, s->d_lvd, st, s->ctl));
-      hipLaunchKernelGGL(k_cg_rz<double>, dim3(R.nblk), dim3(kRed), 0, st, R,
+      hipLaunchKernelGGL(k_cg_rz<double>, dim3(R.nblk), dim3(kRedThreads), 0, st, R,
                          static_cast<const double *>(s->r), static_cast<const double *>(s->zd),
                          s->ctl, s->part);
       hipLaunchKernelGGL(k_cg_p<double>, dim3(nb(ne, kBlk)), dim3(kBlk), 0, st, ne,
                          static_cast<const double *>(s->zd), s->p,
                          static_cast<const CgCtl *>(s->ctl));
     }
-    hipLaunchKernelGGL(k_cg_spmv, dim3(R.nblk), dim3(kRed), 0, st, R, sys.row, sys.nbr, sys.ap,
+    hipLaunchKernelGGL(k_cg_spmv, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.row, sys.nbr, sys.ap,
                        sys.anb, static_cast<const double *>(s->p), s->q, s->ctl, s->part);
     if (s->fp32)
-      hipLaunchKernelGGL(k_cg_update<float>, dim3(R.nblk), dim3(kRed), 0, st, R, sys.phi,
+      hipLaunchKernelGGL(k_cg_update<float>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.phi,
                          static_cast<const double *>(s->p), static_cast<const double *>(s->q),
                          s->r, s->r32, s->z32, s->ctl, s->part);
     else
-      hipLaunchKernelGGL(k_cg_update<double>, dim3(R.nblk), dim3(kRed), 0, st, R, sys.phi,
+      hipLaunchKernelGGL(k_cg_update<double>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.phi,
                          static_cast<const double *>(s->p), static_cast<const double *>(s->q),
                          s->r, static_cast<double *>(nullptr), s->zd, s->ctl, s->part);
     s->launches += 4;
@@ -1260,7 +1300,7 @@ int group_setup(MgGroup *G, hipStream_t st) {
     }
   }
   nbk = sh.map([&](int k) { return R.h[k].R.nblk; });
-  hipLaunchKernelGGL(g_cg_init<T>, dim3(nbk), dim3(kRed), 0, st, sh.g, S);
+  hipLaunchKernelGGL(g_cg_init<T>, dim3(nbk), dim3(kRedThreads), 0, st, sh.g, S);
   G->launches++;
   MGCHK(hipGetLastError());
   return CFDL_OK;
@@ -1340,12 +1380,12 @@ int group_iteration(MgGroup *G, hipStream_t st, int slot) {
   }
   // CG
   nbk = sh.map([&](int k) { return R.h[k].R.nblk; });
-  hipLaunchKernelGGL(g_cg_rz<T>, dim3(nbk), dim3(kRed), 0, st, sh.g, S);
+  hipLaunchKernelGGL(g_cg_rz<T>, dim3(nbk), dim3(kRedThreads), 0, st, sh.g, S);
   const GroupMap gR = sh.g;
   nbk = sh.map([&](int k) { return nb(R.ss[k]->ne, blk); });
   hipLaunchKernelGGL(g_cg_p<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S);
-  hipLaunchKernelGGL(g_cg_spmv<T>, dim3(gR.b0[gR.n]), dim3(kRed), 0, st, gR, S);
-  hipLaunchKernelGGL(g_cg_update<T>, dim3(gR.b0[gR.n]), dim3(kRed), 0, st, gR, S);
+  hipLaunchKernelGGL(g_cg_spmv<T>, dim3(gR.b0[gR.n]), dim3(kRedThreads), 0, st, gR, S);
+  hipLaunchKernelGGL(g_cg_update<T>, dim3(gR.b0[gR.n]), dim3(kRedThreads), 0, st, gR, S);
   hipLaunchKernelGGL(g_cg_flags<T>, dim3(1), dim3(kMaxGroup), 0, st, n, S, G->flags);
   G->launches += 5;
   MGCHK(hipGetLastError());
