@@ -19,12 +19,19 @@
 //    hierarchy of cfdl_mg.cpp): Galerkin coarse operators summed once per
 //    solve from lists (no atomics), one forward colour Gauss-Seidel sweep
 //    before and one backward after each coarse correction, so the operator
-//    is symmetric.  Levels of more than kCoarseMax nodes run as grid-wide
-//    launches (one per colour); the small levels below run inside one
-//    workgroup of 1024 lanes, which walks them with barriers instead of
-//    kernel boundaries.  In the mixed variant the preconditioner runs in
-//    FP32 (FP32 copies of ap, anb and of the residual); CG, its residual
-//    and the stop test stay FP64.
+//    is symmetric.  Every level is stored in its colours' order (struct Lev;
+//    level 0 is a copy of the system, in FP32 for the mixed variant), so a
+//    colour reads its rows and nothing between them; the forward sweep starts
+//    from zero without reading zeros and leaves the last colours' residuals;
+//    the prolongation skips the colour the backward sweep computes first.
+//    Levels of more than kCoarseMax nodes run as grid-wide launches (one per
+//    colour, the small trailing colours in one); the small levels below run
+//    inside one workgroup of 1024 threads, with their values in LDS and each
+//    colour's rows loaded while the one before computes.  In the mixed variant
+//    the V-cycle runs in FP32; CG, its residual and the stop test stay FP64.
+//    A V-cycle at 128^3 in FP32 took 329 us with the levels in mesh order and
+//    176 us so; at 80 x 100 x 72 in FP64 (up to nine colours a level) 636 us
+//    and 321 us.
 //  * All kernels read the solve's active flag and return at once when it is
 //    clear, so the host can queue an iteration before knowing whether the
 //    previous one stopped the solve.
@@ -73,8 +80,6 @@ constexpr int kBlk = 256;          // lanes per block of the grid-wide V-cycle k
 constexpr int kCoarseMax = 4096;   // levels at most this large run in one workgroup
 constexpr int kCoarseThreads = 1024;
 constexpr int kCoarseSweeps = 10;  // forward + backward sweep pairs on the coarsest level
-// a coarsest level at most this large is swept from LDS by one wavefront
-constexpr int kLdsNodes = 64, kLdsEntries = 4096;
 
 // control block of one solve
 struct CgCtl {
@@ -188,24 +193,46 @@ __device__ inline double final_max(const double *part, int nblk, int stride, dou
 // system's range in a grouped launch) and two thin kernels around it.
 // ---------------------------------------------------------------------------
 
-// r = b + sum anb phi_nb - ap phi; z = 0 (and r in FP32 for the mixed
-// preconditioner); res_i, target and the active flag from rms(r)
+// acc + sum over row i of anb * x[nbr], in CSR order; a six-entry
+// (hexahedral) row issues all its loads before the sum
+__device__ inline double csr_sum(const int *__restrict__ row, const int *__restrict__ nbr,
+                                 const double *__restrict__ anb, const double *__restrict__ x,
+                                 int i, double acc) {
+  const int r0 = row[i], r1 = row[i + 1];
+  if (r1 - r0 == 6) {
+    int c[6];
+    double a[6], v[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      c[k] = nbr[r0 + k];
+      a[k] = anb[r0 + k];
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) v[k] = x[c[k]];
+#pragma unroll
+    for (int k = 0; k < 6; k++) acc = acc + a[k] * v[k];
+    return acc;
+  }
+  for (int k = r0; k < r1; k++) acc = acc + anb[k] * x[nbr[k]];
+  return acc;
+}
+
+// r = b + sum anb phi_nb - ap phi, also as rt in the V-cycle's numbering
+// (pos) and type; res_i, target and the active flag from rms(r)
 template <typename T>
 __device__ inline void d_cg_init(int bx, Red R, const int *__restrict__ row,
-                                 const int *__restrict__ nbr, const double *__restrict__ ap,
-                                 const double *__restrict__ anb, const double *__restrict__ b,
-                                 const double *__restrict__ phi, double *__restrict__ r,
-                                 T *__restrict__ rt, T *__restrict__ z, CgCtl *c, double *part,
-                                 int nit) {
+                                 const int *__restrict__ nbr, const int *__restrict__ pos,
+                                 const double *__restrict__ ap, const double *__restrict__ anb,
+                                 const double *__restrict__ b, const double *__restrict__ phi,
+                                 double *__restrict__ r, T *__restrict__ rt, CgCtl *c,
+                                 double *part, int nit) {
   __shared__ double s[kRedSeg];
   const int lo = bx * R.chunk, hi = min(lo + R.chunk, R.n);
   const double acc = blocked_acc(lo, hi, s, [&](int i) {
-    double v = b[i];
-    for (int k = row[i]; k < row[i + 1]; k++) v = v + anb[k] * phi[nbr[k]];
+    double v = csr_sum(row, nbr, anb, phi, i, b[i]);
     v = v - ap[i] * phi[i];
     r[i] = v;
-    if (rt) rt[i] = static_cast<T>(v);
-    z[i] = static_cast<T>(0);
+    rt[pos[i]] = static_cast<T>(v);
     return v * v;
   });
   const double bs = tree_sum(acc, s);
@@ -229,12 +256,13 @@ __device__ inline void d_cg_init(int bx, Red R, const int *__restrict__ row,
 // rho = r.z, beta = rho / rho_old (0 on the first iteration)
 template <typename T>
 __device__ inline void d_cg_rz(int bx, Red R, const double *__restrict__ r,
-                               const T *__restrict__ z, CgCtl *c, double *part) {
+                               const T *__restrict__ z, const int *__restrict__ pos, CgCtl *c,
+                               double *part) {
   __shared__ double s[kRedSeg];
   if (!c->active) return;
   const int lo = bx * R.chunk, hi = min(lo + R.chunk, R.n);
   const double acc =
-      blocked_acc(lo, hi, s, [&](int i) { return r[i] * static_cast<double>(z[i]); });
+      blocked_acc(lo, hi, s, [&](int i) { return r[i] * static_cast<double>(z[pos[i]]); });
   const double bs = tree_sum(acc, s);
   if (threadIdx.x == 0) put_part(part + bx, bs);
   if (!arrive_last(c, R.nblk)) return;
@@ -248,13 +276,14 @@ __device__ inline void d_cg_rz(int bx, Red R, const double *__restrict__ r,
 
 // p = z, or z + beta p (element i)
 template <typename T>
-__device__ inline void d_cg_p(int i, int n, const T *__restrict__ z, double *__restrict__ p,
-                              const CgCtl *c) {
+__device__ inline void d_cg_p(int i, int n, const T *__restrict__ z, const int *__restrict__ pos,
+                              double *__restrict__ p, const CgCtl *c) {
   if (i >= n || !c->active) return;
+  const double zi = static_cast<double>(z[pos[i]]);
   if (c->it == 0)
-    p[i] = static_cast<double>(z[i]);
+    p[i] = zi;
   else
-    p[i] = static_cast<double>(z[i]) + c->beta * p[i];
+    p[i] = zi + c->beta * p[i];
 }
 
 // q = ap p - sum anb p_nb, sigma = p.q, alpha = rho / sigma (a breakdown,
@@ -267,23 +296,7 @@ __device__ inline void d_cg_spmv(int bx, Red R, const int *__restrict__ row,
   if (!c->active) return;
   const int lo = bx * R.chunk, hi = min(lo + R.chunk, R.n);
   const double acc = blocked_acc(lo, hi, s, [&](int i) {
-    const int r0 = row[i], r1 = row[i + 1];
-    double sm = 0.0;
-    if (r1 - r0 == 6) {  // hexahedral row: all loads first, the sum in CSR order
-      int nb[6];
-      double an[6], v[6];
-#pragma unroll
-      for (int k = 0; k < 6; k++) {
-        nb[k] = nbr[r0 + k];
-        an[k] = anb[r0 + k];
-      }
-#pragma unroll
-      for (int k = 0; k < 6; k++) v[k] = p[nb[k]];
-#pragma unroll
-      for (int k = 0; k < 6; k++) sm = sm + an[k] * v[k];
-    } else {
-      for (int k = r0; k < r1; k++) sm = sm + anb[k] * p[nbr[k]];
-    }
+    const double sm = csr_sum(row, nbr, anb, p, i, 0.0);
     const double pi = p[i], qi = ap[i] * pi - sm;
     q[i] = qi;
     return pi * qi;
@@ -301,13 +314,13 @@ __device__ inline void d_cg_spmv(int bx, Red R, const int *__restrict__ row,
   }
 }
 
-// phi += alpha p, r -= alpha q, z = 0 for the next V-cycle; rms and max |r|;
-// the iteration count and the stop test
+// phi += alpha p, r -= alpha q (also as rt for the next V-cycle); rms and max
+// |r|; the iteration count and the stop test
 template <typename T>
 __device__ inline void d_cg_update(int bx, Red R, double *__restrict__ phi,
                                    const double *__restrict__ p, const double *__restrict__ q,
-                                   double *__restrict__ r, T *__restrict__ rt, T *__restrict__ z,
-                                   CgCtl *c, double *part) {
+                                   const int *__restrict__ pos, double *__restrict__ r,
+                                   T *__restrict__ rt, CgCtl *c, double *part) {
   __shared__ double s[kRedSeg];
   if (!c->active) return;
   const double alpha = c->alpha;
@@ -317,8 +330,7 @@ __device__ inline void d_cg_update(int bx, Red R, double *__restrict__ phi,
     phi[i] = phi[i] + alpha * p[i];
     const double v = r[i] - alpha * q[i];
     r[i] = v;
-    if (rt) rt[i] = static_cast<T>(v);
-    z[i] = static_cast<T>(0);
+    rt[pos[i]] = static_cast<T>(v);
     mx = fmax(mx, fabs(v));
     return v * v;
   });
@@ -355,19 +367,22 @@ __device__ inline void d_cg_log(const CgCtl *c, LogLine *log, int *nlog, const L
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
 k_cg_init(Red R, const int *__restrict__ row, const int *__restrict__ nbr,
-          const double *__restrict__ ap, const double *__restrict__ anb,
-          const double *__restrict__ b, const double *__restrict__ phi, double *__restrict__ r,
-          T *__restrict__ rt, T *__restrict__ z, CgCtl *c, double *part, int nit) {
-  d_cg_init<T>(blockIdx.x, R, row, nbr, ap, anb, b, phi, r, rt, z, c, part, nit);
+          const int *__restrict__ pos, const double *__restrict__ ap,
+          const double *__restrict__ anb, const double *__restrict__ b,
+          const double *__restrict__ phi, double *__restrict__ r, T *__restrict__ rt, CgCtl *c,
+          double *part, int nit) {
+  d_cg_init<T>(blockIdx.x, R, row, nbr, pos, ap, anb, b, phi, r, rt, c, part, nit);
 }
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
-k_cg_rz(Red R, const double *__restrict__ r, const T *__restrict__ z, CgCtl *c, double *part) {
-  d_cg_rz<T>(blockIdx.x, R, r, z, c, part);
+k_cg_rz(Red R, const double *__restrict__ r, const T *__restrict__ z, const int *__restrict__ pos,
+        CgCtl *c, double *part) {
+  d_cg_rz<T>(blockIdx.x, R, r, z, pos, c, part);
 }
 template <typename T>
-__global__ void k_cg_p(int n, const T *__restrict__ z, double *__restrict__ p, const CgCtl *c) {
-  d_cg_p<T>(blockIdx.x * blockDim.x + threadIdx.x, n, z, p, c);
+__global__ void k_cg_p(int n, const T *__restrict__ z, const int *__restrict__ pos,
+                       double *__restrict__ p, const CgCtl *c) {
+  d_cg_p<T>(blockIdx.x * blockDim.x + threadIdx.x, n, z, pos, p, c);
 }
 __global__ void __launch_bounds__(kRedThreads)
 k_cg_spmv(Red R, const int *__restrict__ row, const int *__restrict__ nbr,
@@ -378,9 +393,9 @@ k_cg_spmv(Red R, const int *__restrict__ row, const int *__restrict__ nbr,
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
 k_cg_update(Red R, double *__restrict__ phi, const double *__restrict__ p,
-            const double *__restrict__ q, double *__restrict__ r, T *__restrict__ rt,
-            T *__restrict__ z, CgCtl *c, double *part) {
-  d_cg_update<T>(blockIdx.x, R, phi, p, q, r, rt, z, c, part);
+            const double *__restrict__ q, const int *__restrict__ pos, double *__restrict__ r,
+            T *__restrict__ rt, CgCtl *c, double *part) {
+  d_cg_update<T>(blockIdx.x, R, phi, p, q, pos, r, rt, c, part);
 }
 __global__ void k_cg_log(const CgCtl *c, LogLine *log, int *nlog, LogLine tmpl) {
   if (threadIdx.x == 0 && blockIdx.x == 0) d_cg_log(c, log, nlog, tmpl);
@@ -389,245 +404,434 @@ __global__ void k_cg_log(const CgCtl *c, LogLine *log, int *nlog, LogLine tmpl) 
 // ---------------------------------------------------------------------------
 // V-cycle kernels on one level (T = double or float)
 // ---------------------------------------------------------------------------
-// one level as the kernels see it (device pointers)
+// One level as the kernels see it (device pointers).  Its nodes are numbered
+// by colour: colour c is the positions cbeg[c] .. cbeg[c] + ccnt[c] - 1 (on
+// the grid-wide levels a colour starts at a multiple of 64; the positions in
+// between belong to no node), so a colour's rows, values and results are
+// contiguous.  In the mesh order the rows of two colours alternate and every
+// cache line of the matrix was fetched for each of them.  Rows are stored in
+// slices of 64 positions, entry-major: entry k of position p is at
+// mg_entry(p) + 64 k.  Row sums keep the entries' CSR order, so the numbering
+// changes no bit.
 template <typename T>
 struct Lev {
-  int n, nnz, ncol;
-  const int *row, *col, *cperm, *cptr;  // cptr on the device (coarse and grouped kernels)
-  const int *agg, *mptr, *mem, *iptr, *ilist, *gptr, *glist;
-  const T *ap, *anb;
-  T *b, *x;
-  T *apw, *anbw;  // writable views of ap / anb (coarse levels, Galerkin)
+  int n, npad, nnz, ncol;
+  int uni;    // entries of every row, 0 if they differ
+  int fin;    // first position of the final nodes, -1 if they are no such range
+  int ctail;  // colours from this one on share one workgroup (ncol: none do)
+  int kmax;   // longest row
+  const int *cbeg, *ccnt;  // per colour
+  const int *sptr;         // first entry of each slice (not uni)
+  // row length; bit 15: a final node, whose neighbours all have lower colours,
+  // so that a forward sweep leaves its row sum final
+  const unsigned short *info;
+  const int *col;  // position of the neighbour; npad + halo on level 0
+  const int *agg, *mptr, *mem, *iptr, *ilist, *gptr, *glist, *gpos;
+  T *ap, *anb, *b, *x, *t;  // t: residual after the forward sweep
 };
+constexpr int kTailNodes = 1024;
 
-// acc + sum over row i of anb * x[col], in CSR order; a six-entry
-// (hexahedral) row issues all its loads before the sum
 template <typename T>
-__device__ inline T row_sum(const Lev<T> &L, int i, T acc) {
-  const int r0 = L.row[i], r1 = L.row[i + 1];
-  if (r1 - r0 == 6) {
+__device__ inline int mg_entry(const Lev<T> &L, int p) {
+  return (L.uni ? (p >> 6) * 64 * L.uni : L.sptr[p >> 6]) + (p & 63);
+}
+template <typename T>
+__device__ inline bool mg_final(const Lev<T> &L, int p) {
+  return L.fin >= 0 ? p >= L.fin : (L.info[p] >> 15) != 0;
+}
+
+// acc + sum over row p of anb * val(neighbour), in entry order.  Loads go out
+// in groups of six or eight before their part of the sum; a short row's group
+// repeats its last entry and leaves it out of the sum.
+template <typename T, typename V>
+__device__ inline T row_sum(const Lev<T> &L, int p, T acc, V val) {
+  const int e = mg_entry(L, p);
+  if (L.uni == 6) {
     int c[6];
     T a[6], v[6];
 #pragma unroll
     for (int k = 0; k < 6; k++) {
-      c[k] = L.col[r0 + k];
-      a[k] = L.anb[r0 + k];
+      c[k] = L.col[e + 64 * k];
+      a[k] = L.anb[e + 64 * k];
     }
 #pragma unroll
-    for (int k = 0; k < 6; k++) v[k] = L.x[c[k]];
+    for (int k = 0; k < 6; k++) v[k] = val(c[k]);
 #pragma unroll
     for (int k = 0; k < 6; k++) acc = acc + a[k] * v[k];
     return acc;
   }
-  for (int k = r0; k < r1; k++) acc = acc + L.anb[k] * L.x[L.col[k]];
+  const int len = L.info[p] & 0x7fff;
+  for (int k0 = 0; k0 < len; k0 += 8) {
+    int c[8];
+    T a[8], v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int q = e + 64 * min(k0 + k, len - 1);
+      c[k] = L.col[q];
+      a[k] = L.anb[q];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = val(c[k]);
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc = k0 + k < len ? acc + a[k] * v[k] : acc;
+  }
   return acc;
 }
 
-// FP32 copies of the level-0 coefficients (mixed preconditioner), element i
-__device__ inline void d_mg_copy0(int i, int ne, int L, const double *__restrict__ ap,
-                                  const double *__restrict__ anb, float *__restrict__ ap32,
-                                  float *__restrict__ anb32) {
-  if (i < L) anb32[i] = static_cast<float>(anb[i]);
-  if (i < ne) ap32[i] = static_cast<float>(ap[i]);
+// Level 0: the system's coefficients into the level's numbering and type, one
+// thread per mesh cell g (its row is read whole; a colour's entries are
+// written next to each other).
+template <typename T>
+__device__ inline void d_mg_copy0(int g, const Lev<T> &L, const int *__restrict__ pos,
+                                  const int *__restrict__ row, const double *__restrict__ ap,
+                                  const double *__restrict__ anb) {
+  if (g >= L.n) return;
+  const int p = pos[g], e = mg_entry(L, p), r0 = row[g], r1 = row[g + 1];
+  L.ap[p] = static_cast<T>(ap[g]);
+  for (int k = r0; k < r1; k++) L.anb[e + 64 * (k - r0)] = static_cast<T>(anb[k]);
 }
 
-// Galerkin operator of the next level: thread g < nC sums aggregate g's
-// diagonal (members' ap in order, minus the inside entries in order), thread
-// nC + s sums coarse slot s (its list of fine entries in order)
+// Galerkin operator of the next level: thread g < C.npad sums the diagonal of
+// the aggregate at position g (members' ap in order, minus the inside entries
+// in order), thread C.npad + s sums coarse slot s (its list of fine entries in
+// order)
 template <typename T>
 __device__ inline void d_mg_galerkin(int g, const Lev<T> &F, const Lev<T> &C) {
-  if (g < C.n) {
+  if (g < C.npad) {
     T acc = static_cast<T>(0);
     for (int q = F.mptr[g]; q < F.mptr[g + 1]; q++) acc = acc + F.ap[F.mem[q]];
     for (int q = F.iptr[g]; q < F.iptr[g + 1]; q++) acc = acc - F.anb[F.ilist[q]];
-    C.apw[g] = acc;
-  } else if (g < C.n + C.nnz) {
-    const int sl = g - C.n;
+    C.ap[g] = acc;
+  } else if (g < C.npad + C.nnz) {
+    const int sl = g - C.npad;
     T acc = static_cast<T>(0);
     for (int q = F.gptr[sl]; q < F.gptr[sl + 1]; q++) acc = acc + F.anb[F.glist[q]];
-    C.anbw[sl] = acc;
+    C.anb[C.gpos[sl]] = acc;
   }
 }
 
-// one colour of a Gauss-Seidel sweep: x_i = (b_i + sum anb x_nb) / ap_i
+// Gauss-Seidel sweeps by colour, x_i = (b_i + sum anb x_nb) / ap_i.
+// kFwd0: the forward sweep from x = 0, which reads no x it has not written:
+// later colours and halos count as the zeros they stand for, and colour 0 is
+// (b_i + 0) / ap_i without its row (0 anb = 0: the coefficients are finite,
+// or cg_init's residual is not and the solve never starts).  Final nodes
+// leave their residual in t for the restriction.  kFwd, kBwd: from x as it is.
+enum { kFwd0 = 0, kFwd = 1, kBwd = 2 };
 template <typename T>
-__device__ inline void d_mg_sweep(int t, const Lev<T> &L, int c0, int cnt, const CgCtl *ctl) {
-  if (t >= cnt || !ctl->active) return;
-  const int i = L.cperm[c0 + t];
-  L.x[i] = row_sum(L, i, L.b[i]) / L.ap[i];
-}
-
-// restriction of the residual: b_C(I) = sum over members of
-// (b_i + sum anb x_nb) - ap_i x_i, from zero; x_C(I) = 0
-template <typename T>
-__device__ inline void d_mg_restrict(int I, const Lev<T> &F, const Lev<T> &C, const CgCtl *ctl) {
-  if (I >= C.n || !ctl->active) return;
-  T acc = static_cast<T>(0);
-  for (int q = F.mptr[I]; q < F.mptr[I + 1]; q++) {
-    const int i = F.mem[q];
-    const T t = row_sum(F, i, F.b[i]) - F.ap[i] * F.x[i];
-    acc = acc + t;
+__device__ inline void mg_node(const Lev<T> &L, int p, int c, int c0, int mode) {
+  const T a = L.ap[p], b = L.b[p], zero = static_cast<T>(0);
+  T s;
+  if (mode == kFwd0) {
+    if (c == 0)
+      s = L.uni || (L.info[p] & 0x7fff) ? b + zero : b;
+    else
+      s = row_sum(L, p, b, [&](int q) { return q < c0 ? L.x[q] : zero; });
+  } else {
+    s = row_sum(L, p, b, [&](int q) { return L.x[q]; });
   }
-  C.b[I] = acc;
-  C.x[I] = static_cast<T>(0);
+  const T x = s / a;
+  L.x[p] = x;
+  if (mode == kFwd0 && mg_final(L, p)) L.t[p] = s - a * x;
 }
-
-// The same restriction with NL lanes per aggregate (NL a power of two, at
-// least the aggregate's member count): lane j computes member j's term,
-// then every lane of the group adds the terms in member order from
-// shuffles, so the sum is the loop's above.  All lanes reach the shuffles
-// (the active flag is the same for the whole launch of a system).
-template <typename T, int NL>
-__device__ inline void d_mg_restrict_lanes(int gt, const Lev<T> &F, const Lev<T> &C,
-                                           const CgCtl *ctl) {
+// Step q of a sweep: colour q, or, at q = ctail, the remaining colours one
+// after the other in one workgroup (greedy colourings end in a few colours of
+// a few nodes, where a launch of its own costs more than its work).
+template <typename T>
+__device__ inline void d_mg_sweep(int bx, const Lev<T> &L, int q, int mode, const CgCtl *ctl) {
   if (!ctl->active) return;
-  const int I = gt / NL, j = gt % NL;
-  T t = static_cast<T>(0);
-  int cnt = 0;
-  if (I < C.n) {
-    const int q0 = F.mptr[I];
-    cnt = F.mptr[I + 1] - q0;
-    if (j < cnt) {
-      const int i = F.mem[q0 + j];
-      t = row_sum(F, i, F.b[i]) - F.ap[i] * F.x[i];
-    }
+  if (q < L.ctail) {
+    const int t = bx * blockDim.x + threadIdx.x, c0 = L.cbeg[q];
+    if (t < L.ccnt[q]) mg_node(L, c0 + t, q, c0, mode);
+    return;
   }
-  T acc = static_cast<T>(0);
-#pragma unroll
-  for (int jj = 0; jj < NL; jj++) {
-    const T v = __shfl(t, jj, NL);
-    if (jj < cnt) acc = acc + v;
-  }
-  if (j == 0 && I < C.n) {
-    C.b[I] = acc;
-    C.x[I] = static_cast<T>(0);
+  for (int i = L.ctail; i < L.ncol; i++) {
+    const int c = mode == kBwd ? L.ncol - 1 - (i - L.ctail) : i, c0 = L.cbeg[c], n = L.ccnt[c];
+    for (int t = threadIdx.x; t < n; t += blockDim.x) mg_node(L, c0 + t, c, c0, mode);
+    __syncthreads();
   }
 }
 
-// prolongation: x_i += x_C(agg_i)
+// Residual b_i + sum anb x_nb - ap_i x_i of the nodes the forward sweep has
+// not left it for.  A pass of its own in position order: the restriction takes
+// its members from all over the level, and rows gathered that way (4 lines of
+// 128 bytes for 24 used) cost more than the pass and its t together (mean over
+// the three grid-wide levels at 128^3 in FP32: 31 us fused, 7 + 7 us split).
 template <typename T>
-__device__ inline void d_mg_prolong(int i, const Lev<T> &F, const T *__restrict__ xc,
+__device__ inline int mg_open(const Lev<T> &F) {
+  return F.fin >= 0 ? F.fin : F.npad;
+}
+template <typename T>
+__device__ inline void mg_residual(const Lev<T> &F, int p) {
+  if (mg_final(F, p)) return;
+  F.t[p] = row_sum(F, p, F.b[p], [&](int q) { return F.x[q]; }) - F.ap[p] * F.x[p];
+}
+template <typename T>
+__device__ inline void d_mg_residual(int p, int n, const Lev<T> &F, const CgCtl *ctl) {
+  if (p < n && ctl->active) mg_residual(F, p);
+}
+// restriction to position I: the sum of its members' residuals in order, from zero
+template <typename T>
+__device__ inline void mg_restrict(int I, const Lev<T> &F, T *bC) {
+  const int q1 = F.mptr[I + 1];
+  T acc = static_cast<T>(0);
+  for (int q0 = F.mptr[I]; q0 < q1; q0 += 8) {
+    int m[8];
+    T v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) m[k] = F.mem[min(q0 + k, q1 - 1)];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = F.t[m[k]];
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc = q0 + k < q1 ? acc + v[k] : acc;
+  }
+  bC[I] = acc;
+}
+template <typename T>
+__device__ inline void d_mg_restrict(int I, int n, const Lev<T> &F, T *bC, const CgCtl *ctl) {
+  if (I < n && ctl->active) mg_restrict(I, F, bC);
+}
+
+// Prolongation x_i += x_C(agg_i), for every colour but the last: the backward
+// sweep computes that one first, from the others alone.
+template <typename T>
+__device__ inline int mg_prolonged(const Lev<T> &F) {
+  return F.cbeg[F.ncol - 1];
+}
+template <typename T>
+__device__ inline void d_mg_prolong(int i, int n, const Lev<T> &F, const T *__restrict__ xc,
                                     const CgCtl *ctl) {
-  if (i < F.n && ctl->active) F.x[i] = F.x[i] + xc[F.agg[i]];
+  if (i < n && ctl->active) F.x[i] = F.x[i] + xc[F.agg[i]];
 }
 
 // The small levels lc .. nlev-1 of the V-cycle in one workgroup: the same
 // sweeps, restrictions and prolongations as the grid-wide kernels, with a
 // barrier where those have a kernel boundary.  lv[lc].b is the restricted
-// residual and lv[lc].x is zero on entry.
+// residual.  The levels' x and the coarser ones' b live in LDS (coarse_lds
+// bytes, host), so a colour's only global loads are its rows, which depend on
+// nothing before them.
+// A level of that workgroup: x, b, and the tables of colours and slices in LDS.
 template <typename T>
-__device__ void wg_sweep(const Lev<T> &L, bool backward) {
-  for (int cc = 0; cc < L.ncol; cc++) {
-    const int c = backward ? L.ncol - 1 - cc : cc;
-    for (int q = L.cptr[c] + threadIdx.x; q < L.cptr[c + 1]; q += blockDim.x) {
-      const int i = L.cperm[q];
-      L.x[i] = row_sum(L, i, L.b[i]) / L.ap[i];
+struct WgLev {
+  Lev<T> L;
+  const int *cbeg, *ccnt, *sptr;  // sptr has one more entry, the total
+};
+// A node's row as loaded ahead of its turn: the first kAhead entries (a short
+// row's last one again), its scalars and what the rest needs.
+constexpr int kAhead = 8;
+template <typename T>
+struct WgRow {
+  int p, e, info, c[kAhead];
+  T a[kAhead], b, ap;
+};
+template <typename T>
+__device__ inline void wg_load(const WgLev<T> &W, int p, bool on, WgRow<T> &r) {
+  const Lev<T> &L = W.L;
+  r.p = on ? p : -1;
+  if (!on) return;
+  const int s0 = W.sptr[p >> 6], last = (W.sptr[(p >> 6) + 1] - s0) / 64 - 1;
+  r.e = s0 + (p & 63);
+  r.info = L.info[p];
+  r.b = L.b[p];
+  r.ap = L.ap[p];
+#pragma unroll
+  for (int k = 0; k < kAhead; k++) {
+    const int q = r.e + 64 * max(min(k, last), 0);
+    r.c[k] = L.col[q];
+    r.a[k] = L.anb[q];
+  }
+}
+// the row's sum from acc and the node's update: mg_node on a loaded row
+template <typename T>
+__device__ inline void wg_node(const WgLev<T> &W, const WgRow<T> &r, int c0, int mode) {
+  const Lev<T> &L = W.L;
+  if (r.p < 0) return;
+  const T zero = static_cast<T>(0);
+  const int len = r.info & 0x7fff;
+  T v[kAhead], acc = r.b;
+#pragma unroll
+  for (int k = 0; k < kAhead; k++)
+    v[k] = mode != kFwd0 || r.c[k] < c0 ? L.x[r.c[k]] : zero;
+#pragma unroll
+  for (int k = 0; k < kAhead; k++) acc = k < len ? acc + r.a[k] * v[k] : acc;
+  for (int k = kAhead; k < len; k++) {
+    const int q = L.col[r.e + 64 * k];
+    acc = acc + L.anb[r.e + 64 * k] * (mode != kFwd0 || q < c0 ? L.x[q] : zero);
+  }
+  const T x = acc / r.ap;
+  L.x[r.p] = x;
+  if (mode == kFwd0 && (r.info >> 15)) L.t[r.p] = acc - r.ap * x;
+}
+// A sweep: the colours in chunks of one node a thread, a barrier after each
+// colour; a chunk's rows are loaded while the one before computes, so a
+// colour waits for LDS and its division, not for memory.
+template <typename T>
+__device__ void wg_sweep(const WgLev<T> &W, int mode) {
+  const int ncol = W.L.ncol, nt = blockDim.x;
+  int i = 0, t0 = 0;
+  auto colour = [&](int j) { return mode == kBwd ? ncol - 1 - j : j; };
+  auto load = [&](int j, int t, WgRow<T> &r) {
+    const int c = colour(j), q = t + threadIdx.x;
+    wg_load(W, W.cbeg[c] + q, q < W.ccnt[c], r);
+  };
+  WgRow<T> A, B;
+  load(0, 0, A);
+  while (i < ncol) {
+    const int c = colour(i);
+    int ni = i, nt0 = t0 + nt;
+    if (nt0 >= W.ccnt[c]) ni = i + 1, nt0 = 0;
+    if (ni < ncol) load(ni, nt0, B);
+    wg_node(W, A, W.cbeg[c], mode);
+    if (ni != i) __syncthreads();
+    A = B;
+    i = ni;
+    t0 = nt0;
+  }
+}
+// kCoarseSweeps symmetric sweep pairs from x = 0 on a coarsest level of at
+// most 64 nodes by one wavefront, whose LDS accesses complete in program
+// order: lane p holds the row of node p in registers (K entries).  The colour
+// at a turn is computed once: its second value would come from the same
+// neighbour values.
+template <typename T, int K>
+__device__ void wave_coarsest(const Lev<T> &Z, const T *bz, T *xs) {
+  const int p = threadIdx.x, n = Z.n;
+  const int pc = min(p, n - 1), len = p < n ? Z.info[pc] & 0x7fff : 0, e = mg_entry(Z, pc);
+  int c[K];
+  T a[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const int q = e + 64 * min(k, max(len - 1, 0));
+    c[k] = len > 0 ? Z.col[q] : 0;
+    a[k] = len > 0 ? Z.anb[q] : static_cast<T>(0);
+  }
+  const T b = bz[pc], ap = Z.ap[pc];
+  int mine = -1;  // the lane's colour
+  for (int q = 0; q < Z.ncol; q++)
+    if (p >= Z.cbeg[q] && p < Z.cbeg[q] + Z.ccnt[q]) mine = q;
+  auto colour = [&](int q) {
+    if (q == mine) {
+      T v[K], acc = b;
+#pragma unroll
+      for (int k = 0; k < K; k++) v[k] = xs[c[k]];
+#pragma unroll
+      for (int k = 0; k < K; k++) acc = k < len ? acc + a[k] * v[k] : acc;
+      xs[p] = acc / ap;
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  if (p < n) xs[p] = static_cast<T>(0);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  colour(0);
+  for (int k = 0; k < kCoarseSweeps; k++) {
+    for (int q = 1; q < Z.ncol; q++) colour(q);
+    for (int q = Z.ncol - 2; q >= 0; q--) colour(q);
   }
 }
 template <typename T>
 __device__ inline void d_mg_coarse(const Lev<T> *__restrict__ lv, int lc, int nlev,
                                    const CgCtl *ctl) {
+  extern __shared__ double dyn_lds[];
   if (!ctl->active) return;
-  for (int l = lc; l < nlev - 1; l++) {
-    const Lev<T> &F = lv[l], &C = lv[l + 1];
-    wg_sweep(F, false);
-    for (int I = threadIdx.x; I < C.n; I += blockDim.x) {
-      T acc = static_cast<T>(0);
-      for (int q = F.mptr[I]; q < F.mptr[I + 1]; q++) {
-        const int i = F.mem[q];
-        const T t = row_sum(F, i, F.b[i]) - F.ap[i] * F.x[i];
-        acc = acc + t;
-      }
-      C.b[I] = acc;
-      C.x[I] = static_cast<T>(0);
+  // each level's view: x (and below lc, b) and its tables in LDS
+  T *at = reinterpret_cast<T *>(dyn_lds);
+  int *tab = reinterpret_cast<int *>(at);
+  {
+    int reals = 0;
+    for (int i = lc; i < nlev; i++) reals += (i == lc ? 1 : 2) * lv[i].npad;
+    tab = reinterpret_cast<int *>(at + reals);
+  }
+  auto level = [&](int l) {
+    WgLev<T> W;
+    T *q = at;
+    int *k = tab;
+    for (int i = lc; i < l; i++) {
+      q += (i == lc ? 1 : 2) * lv[i].npad;
+      k += 2 * lv[i].ncol + (lv[i].npad + 63) / 64 + 1;
     }
+    W.L = lv[l];
+    W.L.x = q;
+    if (l > lc) W.L.b = q + W.L.npad;
+    W.cbeg = k;
+    W.ccnt = k + W.L.ncol;
+    W.sptr = k + 2 * W.L.ncol;
+    return W;
+  };
+  for (int l = lc; l < nlev; l++) {
+    const WgLev<T> W = level(l);
+    int *k = const_cast<int *>(W.cbeg);
+    for (int i = threadIdx.x; i < W.L.ncol; i += blockDim.x) {
+      k[i] = W.L.cbeg[i];
+      k[W.L.ncol + i] = W.L.ccnt[i];
+    }
+    for (int i = threadIdx.x; i <= (W.L.npad + 63) / 64; i += blockDim.x)
+      k[2 * W.L.ncol + i] = W.L.sptr[i];
+  }
+  __syncthreads();
+  for (int l = lc; l < nlev - 1; l++) {
+    const WgLev<T> F = level(l), C = level(l + 1);
+    wg_sweep(F, kFwd0);
+    for (int p = threadIdx.x; p < mg_open(F.L); p += blockDim.x) mg_residual(F.L, p);
+    __syncthreads();
+    for (int I = threadIdx.x; I < C.L.npad; I += blockDim.x) mg_restrict(I, F.L, C.L.b);
     __syncthreads();
   }
-  const Lev<T> &Z = lv[nlev - 1];
-  if (Z.n <= kLdsNodes && Z.nnz <= kLdsEntries && Z.ncol <= kLdsNodes) {
-    // The coarsest level in LDS, swept by wavefront 0 alone: one wavefront
-    // holds every node of a colour, and its LDS accesses complete in program
-    // order, so no barrier is needed between colours.  The same operations
-    // in the same order as wg_sweep.
-    __shared__ T xs[kLdsNodes], bs[kLdsNodes], as[kLdsNodes], anbs[kLdsEntries];
-    __shared__ int rows[kLdsNodes + 1], cols[kLdsEntries], perms[kLdsNodes], cps[kLdsNodes + 1];
-    for (int i = threadIdx.x; i < Z.n; i += blockDim.x) {
-      xs[i] = Z.x[i];
-      bs[i] = Z.b[i];
-      as[i] = Z.ap[i];
-      perms[i] = Z.cperm[i];
-    }
-    for (int i = threadIdx.x; i <= Z.n; i += blockDim.x) rows[i] = Z.row[i];
-    for (int i = threadIdx.x; i <= Z.ncol; i += blockDim.x) cps[i] = Z.cptr[i];
-    for (int k = threadIdx.x; k < Z.nnz; k += blockDim.x) {
-      cols[k] = Z.col[k];
-      anbs[k] = Z.anb[k];
-    }
-    __syncthreads();
+  const WgLev<T> Z = level(nlev - 1);
+  if (Z.L.n <= 64 && Z.L.kmax <= 20) {
     if (threadIdx.x < 64) {
-      const int t = threadIdx.x;
-      auto colour = [&](int c) {
-        const int q = cps[c] + t;
-        if (q < cps[c + 1]) {
-          const int i = perms[q];
-          T acc = bs[i];
-          for (int k = rows[i]; k < rows[i + 1]; k++) acc = acc + anbs[k] * xs[cols[k]];
-          xs[i] = acc / as[i];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      };
-      for (int k = 0; k < kCoarseSweeps; k++) {
-        for (int c = 0; c < Z.ncol; c++) colour(c);
-        for (int c = Z.ncol - 1; c >= 0; c--) colour(c);
-      }
-      for (int i = t; i < Z.n; i += 64) Z.x[i] = xs[i];
+      if (Z.L.kmax <= 6)
+        wave_coarsest<T, 6>(Z.L, Z.L.b, Z.L.x);
+      else if (Z.L.kmax <= 12)
+        wave_coarsest<T, 12>(Z.L, Z.L.b, Z.L.x);
+      else
+        wave_coarsest<T, 20>(Z.L, Z.L.b, Z.L.x);
     }
     __syncthreads();
   } else {
     for (int k = 0; k < kCoarseSweeps; k++) {
-      wg_sweep(Z, false);
-      wg_sweep(Z, true);
+      wg_sweep(Z, k == 0 ? kFwd0 : kFwd);
+      wg_sweep(Z, kBwd);
     }
   }
   for (int l = nlev - 2; l >= lc; l--) {
-    const Lev<T> &F = lv[l];
-    const T *xc = lv[l + 1].x;
-    for (int i = threadIdx.x; i < F.n; i += blockDim.x) F.x[i] = F.x[i] + xc[F.agg[i]];
+    const WgLev<T> F = level(l);
+    const T *xc = level(l + 1).L.x;
+    const int n = F.cbeg[F.L.ncol - 1];
+    for (int i = threadIdx.x; i < n; i += blockDim.x) F.L.x[i] = F.L.x[i] + xc[F.L.agg[i]];
     __syncthreads();
-    wg_sweep(F, true);
+    wg_sweep(F, kBwd);
   }
+  const Lev<T> F = level(lc).L;
+  for (int i = threadIdx.x; i < F.npad; i += blockDim.x) lv[lc].x[i] = F.x[i];
 }
 
-__global__ void k_mg_copy0(int ne, int L, const double *__restrict__ ap,
-                           const double *__restrict__ anb, float *__restrict__ ap32,
-                           float *__restrict__ anb32) {
-  const int stride = gridDim.x * blockDim.x;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < L || i < ne; i += stride)
-    d_mg_copy0(i, ne, L, ap, anb, ap32, anb32);
+template <typename T>
+__global__ void k_mg_copy0(Lev<T> L, const int *__restrict__ pos, const int *__restrict__ row,
+                           const double *__restrict__ ap, const double *__restrict__ anb) {
+  d_mg_copy0<T>(blockIdx.x * blockDim.x + threadIdx.x, L, pos, row, ap, anb);
 }
 template <typename T>
 __global__ void k_mg_galerkin(Lev<T> F, Lev<T> C) {
   d_mg_galerkin<T>(blockIdx.x * blockDim.x + threadIdx.x, F, C);
 }
 template <typename T>
-__global__ void k_mg_sweep(Lev<T> L, int c0, int cnt, const CgCtl *ctl) {
-  d_mg_sweep<T>(blockIdx.x * blockDim.x + threadIdx.x, L, c0, cnt, ctl);
+__global__ void __launch_bounds__(1024) k_mg_sweep(Lev<T> L, int q, int mode, const CgCtl *ctl) {
+  d_mg_sweep<T>(blockIdx.x, L, q, mode, ctl);
 }
 template <typename T>
-__global__ void k_mg_restrict(Lev<T> F, Lev<T> C, const CgCtl *ctl) {
-  d_mg_restrict<T>(blockIdx.x * blockDim.x + threadIdx.x, F, C, ctl);
-}
-template <typename T, int NL>
-__global__ void k_mg_restrict_lanes(Lev<T> F, Lev<T> C, const CgCtl *ctl) {
-  d_mg_restrict_lanes<T, NL>(blockIdx.x * blockDim.x + threadIdx.x, F, C, ctl);
+__global__ void k_mg_residual(Lev<T> F, int n, const CgCtl *ctl) {
+  d_mg_residual<T>(blockIdx.x * blockDim.x + threadIdx.x, n, F, ctl);
 }
 template <typename T>
-__global__ void k_mg_prolong(Lev<T> F, const T *__restrict__ xc, const CgCtl *ctl) {
-  d_mg_prolong<T>(blockIdx.x * blockDim.x + threadIdx.x, F, xc, ctl);
+__global__ void k_mg_restrict(Lev<T> F, int n, T *bC, const CgCtl *ctl) {
+  d_mg_restrict<T>(blockIdx.x * blockDim.x + threadIdx.x, n, F, bC, ctl);
+}
+template <typename T>
+__global__ void k_mg_prolong(Lev<T> F, int n, const T *__restrict__ xc, const CgCtl *ctl) {
+  d_mg_prolong<T>(blockIdx.x * blockDim.x + threadIdx.x, n, F, xc, ctl);
 }
 template <typename T>
 __global__ void __launch_bounds__(kCoarseThreads)
@@ -638,17 +842,16 @@ k_mg_coarse(const Lev<T> *__restrict__ lv, int lc, int nlev, const CgCtl *ctl) {
 // ---------------------------------------------------------------------------
 // Grouped kernels: one launch runs a step for every system of a group.  Each
 // system's descriptor (device memory) holds its vectors, its control block
-// and its levels with level 0 bound to the system.
+// and its levels.
 // ---------------------------------------------------------------------------
 template <typename T>
 struct MgSlot {
   Red R;
   int ne, nit, nlev, lc;
-  const int *row, *nbr;
+  const int *row, *nbr, *pos;
   const double *ap, *anb, *b;
   double *phi, *r, *p, *q, *part;
-  T *rt, *z;              // FP32 residual copy (nullptr for FP64), preconditioned residual
-  float *ap32, *anb32;    // FP32 level-0 coefficients (mixed)
+  T *rt, *z;              // level 0's right-hand side and values
   CgCtl *ctl;
   const Lev<T> *lv;       // device levels
   LogLine *log;
@@ -660,7 +863,8 @@ template <typename T>
 __global__ void g_mg_copy0(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
-  d_mg_copy0(bx * blockDim.x + threadIdx.x, x.ne, x.lv[0].nnz, x.ap, x.anb, x.ap32, x.anb32);
+  const Lev<T> L = x.lv[0];
+  d_mg_copy0<T>(bx * blockDim.x + threadIdx.x, L, x.pos, x.row, x.ap, x.anb);
 }
 template <typename T>
 __global__ void g_mg_galerkin(GroupMap g, const MgSlot<T> *__restrict__ S, int l) {
@@ -673,41 +877,40 @@ template <typename T>
 __global__ void __launch_bounds__(kRedThreads) g_cg_init(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
-  d_cg_init<T>(bx, x.R, x.row, x.nbr, x.ap, x.anb, x.b, x.phi, x.r, x.rt, x.z, x.ctl, x.part,
+  d_cg_init<T>(bx, x.R, x.row, x.nbr, x.pos, x.ap, x.anb, x.b, x.phi, x.r, x.rt, x.ctl, x.part,
                x.nit);
 }
-// colour cc (counted from the last colour when backward) of level l, or of
-// the system's coarsest level for l < 0
+// step i of a sweep of level l, or of the system's coarsest level for l < 0
+// (backward: counted from the last step)
 template <typename T>
-__global__ void g_mg_sweep(GroupMap g, const MgSlot<T> *__restrict__ S, int l, int cc,
-                           int backward) {
+__global__ void __launch_bounds__(1024)
+g_mg_sweep(GroupMap g, const MgSlot<T> *__restrict__ S, int l, int i, int mode) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
   const Lev<T> L = x.lv[l < 0 ? x.nlev - 1 : l];
-  const int c = backward ? L.ncol - 1 - cc : cc;
-  const int c0 = L.cptr[c];
-  d_mg_sweep<T>(bx * blockDim.x + threadIdx.x, L, c0, L.cptr[c + 1] - c0, x.ctl);
+  const int nstep = L.ctail < L.ncol ? L.ctail + 1 : L.ncol;
+  d_mg_sweep<T>(bx, L, mode == kBwd ? nstep - 1 - i : i, mode, x.ctl);
+}
+template <typename T>
+__global__ void g_mg_residual(GroupMap g, const MgSlot<T> *__restrict__ S, int l) {
+  int bx;
+  const MgSlot<T> &x = S[group_slot(g, bx)];
+  const Lev<T> F = x.lv[l];
+  d_mg_residual<T>(bx * blockDim.x + threadIdx.x, mg_open(F), F, x.ctl);
 }
 template <typename T>
 __global__ void g_mg_restrict(GroupMap g, const MgSlot<T> *__restrict__ S, int l) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
-  const Lev<T> F = x.lv[l], C = x.lv[l + 1];
-  d_mg_restrict<T>(bx * blockDim.x + threadIdx.x, F, C, x.ctl);
-}
-template <typename T, int NL>
-__global__ void g_mg_restrict_lanes(GroupMap g, const MgSlot<T> *__restrict__ S, int l) {
-  int bx;
-  const MgSlot<T> &x = S[group_slot(g, bx)];
-  const Lev<T> F = x.lv[l], C = x.lv[l + 1];
-  d_mg_restrict_lanes<T, NL>(bx * blockDim.x + threadIdx.x, F, C, x.ctl);
+  const Lev<T> F = x.lv[l];
+  d_mg_restrict<T>(bx * blockDim.x + threadIdx.x, x.lv[l + 1].npad, F, x.lv[l + 1].b, x.ctl);
 }
 template <typename T>
 __global__ void g_mg_prolong(GroupMap g, const MgSlot<T> *__restrict__ S, int l) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
   const Lev<T> F = x.lv[l];
-  d_mg_prolong<T>(bx * blockDim.x + threadIdx.x, F, x.lv[l + 1].x, x.ctl);
+  d_mg_prolong<T>(bx * blockDim.x + threadIdx.x, mg_prolonged(F), F, x.lv[l + 1].x, x.ctl);
 }
 template <typename T>
 __global__ void __launch_bounds__(kCoarseThreads)
@@ -720,13 +923,13 @@ template <typename T>
 __global__ void __launch_bounds__(kRedThreads) g_cg_rz(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
-  d_cg_rz<T>(bx, x.R, x.r, x.z, x.ctl, x.part);
+  d_cg_rz<T>(bx, x.R, x.r, x.z, x.pos, x.ctl, x.part);
 }
 template <typename T>
 __global__ void g_cg_p(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
-  d_cg_p<T>(bx * blockDim.x + threadIdx.x, x.ne, x.z, x.p, x.ctl);
+  d_cg_p<T>(bx * blockDim.x + threadIdx.x, x.ne, x.z, x.pos, x.p, x.ctl);
 }
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads) g_cg_spmv(GroupMap g, const MgSlot<T> *__restrict__ S) {
@@ -738,7 +941,7 @@ template <typename T>
 __global__ void __launch_bounds__(kRedThreads) g_cg_update(GroupMap g, const MgSlot<T> *__restrict__ S) {
   int bx;
   const MgSlot<T> &x = S[group_slot(g, bx)];
-  d_cg_update<T>(bx, x.R, x.phi, x.p, x.q, x.r, x.rt, x.z, x.ctl, x.part);
+  d_cg_update<T>(bx, x.R, x.phi, x.p, x.q, x.pos, x.r, x.rt, x.ctl, x.part);
 }
 // the active flags of systems 0 .. n-1, and their log lines at the end
 template <typename T>
@@ -754,70 +957,25 @@ __global__ void g_cg_log(int n, const MgSlot<T> *__restrict__ S) {
 
 inline int nb(int n, int b) { return (n + b - 1) / b; }
 
-// lanes per aggregate of the restriction from a level whose aggregates have
-// at most maxm members: the least power of two >= maxm, 0 (one lane per
-// aggregate, k_mg_restrict) above a wavefront
-inline int restrict_lanes(int maxm) {
-  int nl = 1;
-  while (nl < maxm) nl <<= 1;
-  return nl <= 64 ? nl : 0;
-}
-
-// the restriction from level l of a solve alone
-template <typename T>
-void launch_restrict(int nl, const Lev<T> &F, const Lev<T> &C, const CgCtl *ctl, hipStream_t st) {
-  const int n = C.n * (nl > 0 ? nl : 1);
-  const dim3 g(nb(n, kBlk)), b(kBlk);
-  switch (nl) {
-    case 1: hipLaunchKernelGGL((k_mg_restrict_lanes<T, 1>), g, b, 0, st, F, C, ctl); break;
-    case 2: hipLaunchKernelGGL((k_mg_restrict_lanes<T, 2>), g, b, 0, st, F, C, ctl); break;
-    case 4: hipLaunchKernelGGL((k_mg_restrict_lanes<T, 4>), g, b, 0, st, F, C, ctl); break;
-    case 8: hipLaunchKernelGGL((k_mg_restrict_lanes<T, 8>), g, b, 0, st, F, C, ctl); break;
-    case 16: hipLaunchKernelGGL((k_mg_restrict_lanes<T, 16>), g, b, 0, st, F, C, ctl); break;
-    case 32: hipLaunchKernelGGL((k_mg_restrict_lanes<T, 32>), g, b, 0, st, F, C, ctl); break;
-    case 64: hipLaunchKernelGGL((k_mg_restrict_lanes<T, 64>), g, b, 0, st, F, C, ctl); break;
-    default: hipLaunchKernelGGL(k_mg_restrict<T>, g, b, 0, st, F, C, ctl); break;
-  }
-}
-// the same for a grouped launch (nbk blocks of blk lanes)
-template <typename T>
-void launch_restrict_group(int nl, int nbk, int blk, const GroupMap &gm, const MgSlot<T> *S, int l,
-                           hipStream_t st) {
-  const dim3 g(nbk), b(blk);
-  switch (nl) {
-    case 1: hipLaunchKernelGGL((g_mg_restrict_lanes<T, 1>), g, b, 0, st, gm, S, l); break;
-    case 2: hipLaunchKernelGGL((g_mg_restrict_lanes<T, 2>), g, b, 0, st, gm, S, l); break;
-    case 4: hipLaunchKernelGGL((g_mg_restrict_lanes<T, 4>), g, b, 0, st, gm, S, l); break;
-    case 8: hipLaunchKernelGGL((g_mg_restrict_lanes<T, 8>), g, b, 0, st, gm, S, l); break;
-    case 16: hipLaunchKernelGGL((g_mg_restrict_lanes<T, 16>), g, b, 0, st, gm, S, l); break;
-    case 32: hipLaunchKernelGGL((g_mg_restrict_lanes<T, 32>), g, b, 0, st, gm, S, l); break;
-    case 64: hipLaunchKernelGGL((g_mg_restrict_lanes<T, 64>), g, b, 0, st, gm, S, l); break;
-    default: hipLaunchKernelGGL(g_mg_restrict<T>, g, b, 0, st, gm, S, l); break;
-  }
-}
-
 }  // namespace
 // device copy of the hierarchy and the solve's work vectors
 struct MgCgSolver {
   int fp32 = 0, ne = 0, nbf = 0, nlev = 0, lc = 0;
+  size_t coarse_lds = 0;  // LDS of the workgroup that runs levels lc ..
   std::vector<void *> mem;
-  std::vector<std::vector<int>> cptr;  // host colour offsets per level
-  std::vector<int> lanes;              // restriction lanes per aggregate, per level
-  // per level, for each real type (index 0 double, 1 float)
+  std::vector<std::vector<int>> ccnt;  // nodes per colour and level (host)
+  std::vector<int> open, prolonged;    // positions of d_mg_residual and d_mg_prolong, per level
+  // the levels for one real type (host copies of the device descriptors)
   std::vector<Lev<double>> lvd;
   std::vector<Lev<float>> lvf;
   Lev<double> *d_lvd = nullptr;
   Lev<float> *d_lvf = nullptr;
-  double *r = nullptr, *p = nullptr, *q = nullptr, *zd = nullptr, *part = nullptr;
-  float *r32 = nullptr, *z32 = nullptr, *ap32 = nullptr, *anb32 = nullptr;
+  const int *pos = nullptr;  // level 0's position of each cell
+  double *r = nullptr, *p = nullptr, *q = nullptr, *part = nullptr;
   CgCtl *ctl = nullptr;
   int *hflag = nullptr;  // pinned
   hipEvent_t ev[2] = {nullptr, nullptr};
   int launches = 0;
-  // grouped solves: the arrays level 0 was last bound to on the device
-  // (d_lvd[0] / d_lvf[0]); nullptr until the first grouped solve
-  const int *bound_row = nullptr;
-  const double *bound_ap = nullptr;
 
   ~MgCgSolver() {
     for (void *m : mem) (void)hipFree(m);
@@ -837,10 +995,11 @@ struct MgCgSolver {
     *p = static_cast<X *>(v);
     return CFDL_OK;
   }
-  int upload(const std::vector<int> &v, const int **out) {
-    int *d = nullptr;
+  template <typename X>
+  int upload(const std::vector<X> &v, const X **out) {
+    X *d = nullptr;
     if (int rc = alloc(&d, v.size())) return rc;
-    if (!v.empty()) MGCHK(hipMemcpy(d, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice));
+    if (!v.empty()) MGCHK(hipMemcpy(d, v.data(), sizeof(X) * v.size(), hipMemcpyHostToDevice));
     *out = d;
     return CFDL_OK;
   }
@@ -854,53 +1013,193 @@ struct MgCgSolver {
 
 namespace {
 template <typename T>
-int fill_levels(MgCgSolver *s, const MgHier &h, std::vector<Lev<T>> &lv) {
-  lv.assign(s->nlev, Lev<T>{});
-  for (int l = 0; l < s->nlev; l++) {
-    const MgLevel &H = h.lv[l];
-    Lev<T> &L = lv[l];
-    L.n = H.n;
-    L.nnz = H.nnz;
-    L.ncol = H.ncol;
-    if (l > 0) {
-      MGCALL(s->upload(H.row, &L.row));
-      MGCALL(s->upload(H.col, &L.col));
-      T *a = nullptr, *an = nullptr, *b = nullptr, *x = nullptr;
-      MGCALL(s->alloc(&a, H.n));
-      MGCALL(s->alloc(&an, H.nnz));
-      MGCALL(s->alloc(&b, H.n));
-      MGCALL(s->alloc(&x, H.n));
-      L.ap = L.apw = a;
-      L.anb = L.anbw = an;
-      L.b = b;
-      L.x = x;
-    }
-    MGCALL(s->upload(H.cperm, &L.cperm));
-    MGCALL(s->upload(H.cptr, &L.cptr));
-    if (l + 1 < s->nlev) {
-      MGCALL(s->upload(H.agg, &L.agg));
-      MGCALL(s->upload(H.mptr, &L.mptr));
-      MGCALL(s->upload(H.mem, &L.mem));
-      MGCALL(s->upload(H.iptr, &L.iptr));
-      MGCALL(s->upload(H.ilist, &L.ilist));
-      MGCALL(s->upload(H.gptr, &L.gptr));
-      MGCALL(s->upload(H.glist, &L.glist));
+std::vector<Lev<T>> &host_levels(MgCgSolver *s);
+template <>
+std::vector<Lev<double>> &host_levels<double>(MgCgSolver *s) { return s->lvd; }
+template <>
+std::vector<Lev<float>> &host_levels<float>(MgCgSolver *s) { return s->lvf; }
+template <typename T>
+Lev<T> *&dev_levels(MgCgSolver *s);
+template <>
+Lev<double> *&dev_levels<double>(MgCgSolver *s) { return s->d_lvd; }
+template <>
+Lev<float> *&dev_levels<float>(MgCgSolver *s) { return s->d_lvf; }
+
+// One level's numbering by colour and its sliced rows (struct Lev).
+struct Numbering {
+  std::vector<int> pos;              // position of each node
+  std::vector<int> cbeg, ccnt;       // per colour
+  std::vector<int> sptr, slot;       // slice starts; entry of each CSR slot
+  std::vector<unsigned short> info;  // per position
+  int npad = 0, nent = 0, uni = 0, fin = -1, kmax = 0;
+};
+// align: positions a colour's start is rounded up to (64, or 1 inside the
+// workgroup-only levels, whose coarsest is one node a lane)
+int number_level(const MgLevel &H, int align, bool level0, Numbering *out) {
+  Numbering &N = *out;
+  N.pos.assign(H.n, 0);
+  std::vector<int> node;
+  for (int c = 0; c < H.ncol; c++) {
+    while (static_cast<int>(node.size()) % align) node.push_back(-1);
+    N.cbeg.push_back(static_cast<int>(node.size()));
+    N.ccnt.push_back(H.cptr[c + 1] - H.cptr[c]);
+    for (int q = H.cptr[c]; q < H.cptr[c + 1]; q++) {
+      N.pos[H.cperm[q]] = static_cast<int>(node.size());
+      node.push_back(H.cperm[q]);
     }
   }
+  while (static_cast<int>(node.size()) % align) node.push_back(-1);
+  N.npad = static_cast<int>(node.size());
+  bool six = level0;
+  int64_t at = 0;
+  N.info.assign(N.npad, 0);
+  for (int p0 = 0; p0 < N.npad; p0 += 64) {
+    int k = 0;
+    for (int p = p0; p < std::min(p0 + 64, N.npad); p++)
+      if (node[p] >= 0) k = std::max(k, H.row[node[p] + 1] - H.row[node[p]]);
+    N.sptr.push_back(static_cast<int>(at));
+    at += 64 * int64_t{k};
+  }
+  if (at > 0x7fffffff) {
+    set_error("mgcg_create: level too large");
+    return CFDL_EINVAL;
+  }
+  N.nent = static_cast<int>(at);
+  N.sptr.push_back(N.nent);
+  N.slot.assign(H.nnz, 0);
+  for (int c = 0, p = 0; p < N.npad; p++) {
+    const int i = node[p];
+    if (i < 0) continue;
+    while (c + 1 < H.ncol && p >= N.cbeg[c + 1]) c++;
+    const int len = H.row[i + 1] - H.row[i];
+    if (len > 0x7fff) {
+      set_error("mgcg_create: row of more than 32767 entries");
+      return CFDL_EINVAL;
+    }
+    six = six && len == 6;
+    bool final = true;
+    for (int k = H.row[i]; k < H.row[i + 1]; k++) {
+      N.slot[k] = N.sptr[p >> 6] + 64 * (k - H.row[i]) + (p & 63);
+      if (H.col[k] < H.n && N.pos[H.col[k]] >= N.cbeg[c]) final = false;
+    }
+    N.info[p] = static_cast<unsigned short>(len | (final ? 0x8000 : 0));
+    N.kmax = std::max(N.kmax, len);
+  }
+  if (six) N.uni = 6;  // every slice then holds 6 entries a position
+  // the final nodes as a range at the end, when they are one
+  int f = N.npad;
+  while (f > 0 && (node[f - 1] < 0 || (N.info[f - 1] >> 15))) f--;
+  bool range = true;
+  for (int p = 0; p < f && range; p++) range = node[p] < 0 || !(N.info[p] >> 15);
+  if (range) N.fin = f;
   return CFDL_OK;
 }
 
-// one V-cycle: z = M r on level 0 (lv[0].b = r, lv[0].x = z, zero on entry)
 template <typename T>
-int vcycle(MgCgSolver *s, const std::vector<Lev<T>> &lv, const Lev<T> *d_lv, hipStream_t st,
-           const CgCtl *ctl) {
+int fill_levels(MgCgSolver *s, const MgHier &h) {
+  std::vector<Lev<T>> &lv = host_levels<T>(s);
+  lv.assign(s->nlev, Lev<T>{});
+  std::vector<Numbering> num(s->nlev);
+  for (int l = 0; l < s->nlev; l++)
+    MGCALL(number_level(h.lv[l], l < s->lc ? 64 : 1, l == 0, &num[l]));
+  auto zeroed = [&](T **p, size_t n) -> int {
+    MGCALL(s->alloc(p, n));
+    MGCHK(hipMemset(*p, 0, sizeof(T) * (n > 0 ? n : 1)));
+    return CFDL_OK;
+  };
+  for (int l = 0; l < s->nlev; l++) {
+    const MgLevel &H = h.lv[l];
+    const Numbering &N = num[l];
+    Lev<T> &L = lv[l];
+    L.n = H.n;
+    L.npad = N.npad;
+    L.nnz = H.nnz;
+    L.ncol = H.ncol;
+    L.uni = N.uni;
+    L.fin = N.fin;
+    L.kmax = N.kmax;
+    // the tail: the trailing colours of together at most kTailNodes nodes,
+    // if they are at least two
+    int tail = H.ncol, left = 0;
+    while (tail > 1 && left + N.ccnt[tail - 1] <= kTailNodes) left += N.ccnt[--tail];
+    L.ctail = H.ncol - tail >= 2 ? tail : H.ncol;
+    s->ccnt.push_back(N.ccnt);
+    s->prolonged.push_back(N.cbeg[H.ncol - 1]);
+    s->open.push_back(N.fin >= 0 ? N.fin : N.npad);
+    std::vector<int> col(N.nent + 64, 0);  // an empty slice's loads stay inside
+    for (int i = 0; i < H.n; i++)
+      for (int k = H.row[i]; k < H.row[i + 1]; k++)
+        col[N.slot[k]] = H.col[k] < H.n ? N.pos[H.col[k]] : N.npad + (H.col[k] - H.n);
+    MGCALL(s->upload(N.cbeg, &L.cbeg));
+    MGCALL(s->upload(N.ccnt, &L.ccnt));
+    MGCALL(s->upload(N.sptr, &L.sptr));
+    MGCALL(s->upload(N.info, &L.info));
+    MGCALL(s->upload(col, &L.col));
+    MGCALL(zeroed(&L.ap, N.npad));
+    MGCALL(zeroed(&L.anb, N.nent + 64));
+    MGCALL(zeroed(&L.b, N.npad));
+    MGCALL(zeroed(&L.x, N.npad + (l == 0 ? s->nbf : 0)));
+    MGCALL(zeroed(&L.t, N.npad));
+    if (l > 0) MGCALL(s->upload(N.slot, &L.gpos));
+    if (l == 0) MGCALL(s->upload(N.pos, &s->pos));
+    if (l + 1 == s->nlev) continue;
+    const Numbering &C = num[l + 1];
+    const MgLevel &HC = h.lv[l + 1];
+    std::vector<int> agg(N.npad, 0), at(C.npad, -1), mptr(1, 0), mem, iptr(1, 0), ilist;
+    for (int i = 0; i < H.n; i++) agg[N.pos[i]] = C.pos[H.agg[i]];
+    for (int g = 0; g < HC.n; g++) at[C.pos[g]] = g;
+    for (int p = 0; p < C.npad; p++) {
+      const int g = at[p];
+      for (int q = g < 0 ? 0 : H.mptr[g]; g >= 0 && q < H.mptr[g + 1]; q++)
+        mem.push_back(N.pos[H.mem[q]]);
+      for (int q = g < 0 ? 0 : H.iptr[g]; g >= 0 && q < H.iptr[g + 1]; q++)
+        ilist.push_back(N.slot[H.ilist[q]]);
+      mptr.push_back(static_cast<int>(mem.size()));
+      iptr.push_back(static_cast<int>(ilist.size()));
+    }
+    std::vector<int> glist(H.glist.size());
+    for (size_t q = 0; q < glist.size(); q++) glist[q] = N.slot[H.glist[q]];
+    MGCALL(s->upload(agg, &L.agg));
+    MGCALL(s->upload(mptr, &L.mptr));
+    MGCALL(s->upload(mem, &L.mem));
+    MGCALL(s->upload(iptr, &L.iptr));
+    MGCALL(s->upload(ilist, &L.ilist));
+    MGCALL(s->upload(H.gptr, &L.gptr));
+    MGCALL(s->upload(glist, &L.glist));
+  }
+  for (int l = s->lc; l < s->nlev; l++)
+    s->coarse_lds += sizeof(T) * (l == s->lc ? 1 : 2) * static_cast<size_t>(num[l].npad) +
+                     sizeof(int) * (num[l].cbeg.size() * 2 + num[l].sptr.size());
+  MGCALL(s->alloc(&dev_levels<T>(s), s->nlev));
+  MGCHK(hipMemcpy(dev_levels<T>(s), lv.data(), sizeof(Lev<T>) * s->nlev, hipMemcpyHostToDevice));
+  return CFDL_OK;
+}
+
+// steps of a sweep (d_mg_sweep), and the blocks of blk threads of step i
+// counted in the sweep's direction
+template <typename T>
+int sweep_steps(const Lev<T> &L) {
+  return L.ctail < L.ncol ? L.ctail + 1 : L.ncol;
+}
+template <typename T>
+int sweep_blocks(const MgCgSolver *s, int l, const Lev<T> &L, int i, int mode, int blk) {
+  const int n = sweep_steps(L), q = mode == kBwd ? n - 1 - i : i;
+  return i >= n ? 0 : q < L.ctail ? nb(s->ccnt[l][q], blk) : 1;
+}
+
+// one V-cycle: z = M r on level 0 (lv[0].b = r, lv[0].x = z)
+template <typename T>
+int vcycle(MgCgSolver *s, hipStream_t st) {
+  const std::vector<Lev<T>> &lv = host_levels<T>(s);
+  const CgCtl *ctl = s->ctl;
   const int nlev = s->nlev, lc = s->lc;
-  auto sweep = [&](int l, bool backward) {
+  auto sweep = [&](int l, int mode) {
     const Lev<T> &L = lv[l];
-    for (int cc = 0; cc < L.ncol; cc++) {
-      const int c = backward ? L.ncol - 1 - cc : cc;
-      const int c0 = s->cptr[l][c], cnt = s->cptr[l][c + 1] - c0;
-      hipLaunchKernelGGL(k_mg_sweep<T>, dim3(nb(cnt, kBlk)), dim3(kBlk), 0, st, L, c0, cnt, ctl);
+    const int n = sweep_steps(L);
+    for (int i = 0; i < n; i++) {
+      const int q = mode == kBwd ? n - 1 - i : i;
+      const dim3 g(sweep_blocks(s, l, L, i, mode, kBlk)), b(q < L.ctail ? kBlk : kTailNodes);
+      hipLaunchKernelGGL(k_mg_sweep<T>, g, b, 0, st, L, q, mode, ctl);
       s->launches++;
     }
   };
@@ -908,24 +1207,31 @@ int vcycle(MgCgSolver *s, const std::vector<Lev<T>> &lv, const Lev<T> *d_lv, hip
   // levels follow, smoothed in place)
   const int top = lc < nlev ? lc : nlev - 1;
   for (int l = 0; l < top; l++) {
-    sweep(l, false);
-    launch_restrict<T>(s->lanes[l], lv[l], lv[l + 1], ctl, st);
-    s->launches++;
+    sweep(l, kFwd0);
+    if (s->open[l] > 0)
+      hipLaunchKernelGGL(k_mg_residual<T>, dim3(nb(s->open[l], kBlk)), dim3(kBlk), 0, st, lv[l],
+                         s->open[l], ctl);
+    hipLaunchKernelGGL(k_mg_restrict<T>, dim3(nb(lv[l + 1].npad, kBlk)), dim3(kBlk), 0, st, lv[l],
+                       lv[l + 1].npad, lv[l + 1].b, ctl);
+    s->launches += 2;
   }
   if (lc < nlev) {
-    hipLaunchKernelGGL(k_mg_coarse<T>, dim3(1), dim3(kCoarseThreads), 0, st, d_lv, lc, nlev, ctl);
+    hipLaunchKernelGGL(k_mg_coarse<T>, dim3(1), dim3(kCoarseThreads), s->coarse_lds, st,
+                       static_cast<const Lev<T> *>(dev_levels<T>(s)), lc, nlev, ctl);
     s->launches++;
   } else {
     for (int k = 0; k < kCoarseSweeps; k++) {
-      sweep(nlev - 1, false);
-      sweep(nlev - 1, true);
+      sweep(nlev - 1, k == 0 ? kFwd0 : kFwd);
+      sweep(nlev - 1, kBwd);
     }
   }
   for (int l = top - 1; l >= 0; l--) {
-    hipLaunchKernelGGL(k_mg_prolong<T>, dim3(nb(lv[l].n, kBlk)), dim3(kBlk), 0, st, lv[l],
-                       static_cast<const T *>(lv[l + 1].x), ctl);
-    s->launches++;
-    sweep(l, true);
+    if (s->prolonged[l] > 0) {
+      hipLaunchKernelGGL(k_mg_prolong<T>, dim3(nb(s->prolonged[l], kBlk)), dim3(kBlk), 0, st,
+                         lv[l], s->prolonged[l], static_cast<const T *>(lv[l + 1].x), ctl);
+      s->launches++;
+    }
+    sweep(l, kBwd);
   }
   MGCHK(hipGetLastError());
   return CFDL_OK;
@@ -936,22 +1242,20 @@ int mgcg_create(const MgHier &h, int nbf, int fp32, MgCgSolver **out) {
   std::unique_ptr<MgCgSolver> s(new MgCgSolver());
   s->fp32 = fp32 ? 1 : 0;
   s->nlev = static_cast<int>(h.lv.size());
-  s->ne = h.lv[0].n;
-  s->nbf = nbf;
-  if (s->nlev < 1 || s->ne < 1) {
+  if (s->nlev < 1 || h.lv[0].n < 1) {
     set_error("mgcg_create: empty hierarchy");
     return CFDL_EINVAL;
   }
+  s->ne = h.lv[0].n;
+  s->nbf = nbf;
   // the small levels that run in one workgroup: the trailing levels (below
-  // level 0) of at most kCoarseMax nodes
+  // level 0) of at most kCoarseMax nodes whose x, b and tables fit 64 KB of LDS
   s->lc = s->nlev;
-  while (s->lc - 1 >= 1 && h.lv[s->lc - 1].n <= kCoarseMax) s->lc--;
-  for (int l = 0; l < s->nlev; l++) {
-    s->cptr.push_back(h.lv[l].cptr);
-    int maxm = 1;
-    const std::vector<int> &mp = h.lv[l].mptr;
-    for (size_t g = 0; g + 1 < mp.size(); g++) maxm = std::max(maxm, mp[g + 1] - mp[g]);
-    s->lanes.push_back(restrict_lanes(maxm));
+  size_t below = 0, real = fp32 ? sizeof(float) : sizeof(double);
+  while (s->lc - 1 >= 1 && h.lv[s->lc - 1].n <= kCoarseMax &&
+         below + real * h.lv[s->lc - 1].n <= 57344) {
+    s->lc--;
+    below += 2 * real * h.lv[s->lc].n;
   }
   const int ne = s->ne, nall = ne + nbf;
   MGCALL(s->alloc(&s->r, ne));
@@ -961,23 +1265,7 @@ int mgcg_create(const MgHier &h, int nbf, int fp32, MgCgSolver **out) {
   MGCALL(s->alloc(&s->ctl, 1));
   MGCHK(hipMemset(s->ctl, 0, sizeof(CgCtl)));
   MGCHK(hipMemset(s->p, 0, sizeof(double) * nall));
-  if (s->fp32) {
-    MGCALL(s->alloc(&s->r32, ne));
-    MGCALL(s->alloc(&s->z32, nall));
-    MGCALL(s->alloc(&s->ap32, ne));
-    MGCALL(s->alloc(&s->anb32, h.lv[0].nnz));
-    MGCHK(hipMemset(s->z32, 0, sizeof(float) * nall));
-    MGCALL(fill_levels<float>(s.get(), h, s->lvf));
-    MGCALL(s->alloc(&s->d_lvf, s->nlev));
-    // the workgroup kernel reads levels >= 1 only, which never change
-    MGCHK(hipMemcpy(s->d_lvf, s->lvf.data(), sizeof(Lev<float>) * s->nlev, hipMemcpyHostToDevice));
-  } else {
-    MGCALL(s->alloc(&s->zd, nall));
-    MGCHK(hipMemset(s->zd, 0, sizeof(double) * nall));
-    MGCALL(fill_levels<double>(s.get(), h, s->lvd));
-    MGCALL(s->alloc(&s->d_lvd, s->nlev));
-    MGCHK(hipMemcpy(s->d_lvd, s->lvd.data(), sizeof(Lev<double>) * s->nlev, hipMemcpyHostToDevice));
-  }
+  MGCALL(s->fp32 ? fill_levels<float>(s.get(), h) : fill_levels<double>(s.get(), h));
   MGCHK(hipHostMalloc(reinterpret_cast<void **>(&s->hflag), 2 * sizeof(int), hipHostMallocDefault));
   MGCHK(hipEventCreateWithFlags(&s->ev[0], hipEventDisableTiming));
   MGCHK(hipEventCreateWithFlags(&s->ev[1], hipEventDisableTiming));
@@ -992,83 +1280,39 @@ void mgcg_stats(const MgCgSolver *s, int *launches, int *levels) {
   if (levels) *levels = s ? s->nlev : 0;
 }
 
-int mgcg_solve(MgCgSolver *s, const MgCgSystem &sys, void *stream) {
-  if (!s || sys.ne != s->ne || sys.nbf != s->nbf) {
-    set_error("mgcg_solve: system does not match the hierarchy");
-    return CFDL_EINVAL;
-  }
-  hipStream_t st = static_cast<hipStream_t>(stream);
+namespace {
+template <typename T>
+int solve(MgCgSolver *s, const MgCgSystem &sys, hipStream_t st) {
   const int ne = s->ne;
   const Red R = red_of(ne);
+  std::vector<Lev<T>> &lv = host_levels<T>(s);
+  T *rt = lv[0].b;
+  const T *z = lv[0].x;
   s->launches = 0;
-  // level 0 is the system itself (FP32 copies for the mixed preconditioner)
-  if (s->fp32) {
-    Lev<float> &z = s->lvf[0];
-    z.row = sys.row;
-    z.col = sys.nbr;
-    const int Lnz = z.nnz;
-    hipLaunchKernelGGL(k_mg_copy0, dim3(std::min(nb(std::max(Lnz, ne), kBlk), 8192)), dim3(kBlk), 0,
-                       st, ne, Lnz, sys.ap, sys.anb, s->ap32, s->anb32);
-    z.ap = z.apw = s->ap32;
-    z.anb = z.anbw = s->anb32;
-    z.b = s->r32;
-    z.x = s->z32;
-    for (int l = 0; l + 1 < s->nlev; l++)
-      hipLaunchKernelGGL(k_mg_galerkin<float>, dim3(nb(s->lvf[l + 1].n + s->lvf[l + 1].nnz, kBlk)),
-                         dim3(kBlk), 0, st, s->lvf[l], s->lvf[l + 1]);
-    hipLaunchKernelGGL(k_cg_init<float>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.row, sys.nbr,
-                       sys.ap, sys.anb, sys.b, static_cast<const double *>(sys.phi), s->r, s->r32,
-                       s->z32, s->ctl, s->part, sys.nit);
-  } else {
-    Lev<double> &z = s->lvd[0];
-    z.row = sys.row;
-    z.col = sys.nbr;
-    z.ap = sys.ap;
-    z.anb = sys.anb;
-    z.apw = nullptr;
-    z.anbw = nullptr;
-    z.b = s->r;
-    z.x = s->zd;
-    for (int l = 0; l + 1 < s->nlev; l++)
-      hipLaunchKernelGGL(k_mg_galerkin<double>, dim3(nb(s->lvd[l + 1].n + s->lvd[l + 1].nnz, kBlk)),
-                         dim3(kBlk), 0, st, s->lvd[l], s->lvd[l + 1]);
-    hipLaunchKernelGGL(k_cg_init<double>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.row, sys.nbr,
-                       sys.ap, sys.anb, sys.b, static_cast<const double *>(sys.phi), s->r,
-                       static_cast<double *>(nullptr), s->zd, s->ctl, s->part, sys.nit);
-  }
+  hipLaunchKernelGGL(k_mg_copy0<T>, dim3(nb(ne, kBlk)), dim3(kBlk), 0, st, lv[0], s->pos, sys.row,
+                     sys.ap, sys.anb);
+  for (int l = 0; l + 1 < s->nlev; l++)
+    hipLaunchKernelGGL(k_mg_galerkin<T>, dim3(nb(lv[l + 1].npad + lv[l + 1].nnz, kBlk)), dim3(kBlk),
+                       0, st, lv[l], lv[l + 1]);
+  hipLaunchKernelGGL(k_cg_init<T>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.row, sys.nbr,
+                     s->pos, sys.ap, sys.anb, sys.b, static_cast<const double *>(sys.phi), s->r, rt,
+                     s->ctl, s->part, sys.nit);
   MGCHK(hipGetLastError());
+  const double *r = s->r, *p = s->p, *q = s->q;
   int *act = &s->ctl->active;
   // Iteration k is queued before the host reads the flag after iteration
   // k-1, so the GPU never waits for the host; an iteration queued after the
   // stop exits at once.
   for (int it = 0; it < sys.nit; it++) {
-    if (s->fp32) {
-      MGCALL(vcycle<float>(s, s->lvf, s->d_lvf, st, s->ctl));
-      hipLaunchKernelGGL(k_cg_rz<float>, dim3(R.nblk), dim3(kRedThreads), 0, st, R,
-                         static_cast<const double *>(s->r), static_cast<const float *>(s->z32),
-                         s->ctl, s->part);
-      hipLaunchKernelGGL(k_cg_p<float>, dim3(nb(ne, kBlk)), dim3(kBlk), 0, st, ne,
-                         static_cast<const float *>(s->z32), s->p,
-                         static_cast<const CgCtl *>(s->ctl));
-    } else {
-      MGCALL(vcycle<double>(s, s->lvd, s->d_lvd, st, s->ctl));
-      hipLaunchKernelGGL(k_cg_rz<double>, dim3(R.nblk), dim3(kRedThreads), 0, st, R,
-                         static_cast<const double *>(s->r), static_cast<const double *>(s->zd),
-                         s->ctl, s->part);
-      hipLaunchKernelGGL(k_cg_p<double>, dim3(nb(ne, kBlk)), dim3(kBlk), 0, st, ne,
-                         static_cast<const double *>(s->zd), s->p,
-                         static_cast<const CgCtl *>(s->ctl));
-    }
-    hipLaunchKernelGGL(k_cg_spmv, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.row, sys.nbr, sys.ap,
-                       sys.anb, static_cast<const double *>(s->p), s->q, s->ctl, s->part);
-    if (s->fp32)
-      hipLaunchKernelGGL(k_cg_update<float>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.phi,
-                         static_cast<const double *>(s->p), static_cast<const double *>(s->q),
-                         s->r, s->r32, s->z32, s->ctl, s->part);
-    else
-      hipLaunchKernelGGL(k_cg_update<double>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.phi,
-                         static_cast<const double *>(s->p), static_cast<const double *>(s->q),
-                         s->r, static_cast<double *>(nullptr), s->zd, s->ctl, s->part);
+    MGCALL(vcycle<T>(s, st));
+    hipLaunchKernelGGL(k_cg_rz<T>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, r, z, s->pos, s->ctl,
+                       s->part);
+    hipLaunchKernelGGL(k_cg_p<T>, dim3(nb(ne, kBlk)), dim3(kBlk), 0, st, ne, z, s->pos, s->p,
+                       static_cast<const CgCtl *>(s->ctl));
+    hipLaunchKernelGGL(k_cg_spmv, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.row, sys.nbr,
+                       sys.ap, sys.anb, p, s->q, s->ctl, s->part);
+    hipLaunchKernelGGL(k_cg_update<T>, dim3(R.nblk), dim3(kRedThreads), 0, st, R, sys.phi, p, q,
+                       s->pos, s->r, rt, s->ctl, s->part);
     s->launches += 4;
     MGCHK(hipGetLastError());
     MGCHK(hipMemcpyAsync(&s->hflag[it & 1], act, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1085,6 +1329,16 @@ int mgcg_solve(MgCgSolver *s, const MgCgSystem &sys, void *stream) {
   MGCHK(hipGetLastError());
   return CFDL_OK;
 }
+}  // namespace
+
+int mgcg_solve(MgCgSolver *s, const MgCgSystem &sys, void *stream) {
+  if (!s || sys.ne != s->ne || sys.nbf != s->nbf) {
+    set_error("mgcg_solve: system does not match the hierarchy");
+    return CFDL_EINVAL;
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return s->fp32 ? solve<float>(s, sys, st) : solve<double>(s, sys, st);
+}
 
 // ---------------------------------------------------------------------------
 // Grouped solves
@@ -1096,7 +1350,6 @@ template <typename T>
 struct GroupRun {
   std::vector<MgCgSolver *> ss;
   std::vector<MgSlot<T>> h;
-  std::vector<Lev<T>> l0;
   int n = 0, blk = 256, maxtop = 0, maxlev = 0, nitmax = 0;
 };
 }  // namespace
@@ -1137,50 +1390,6 @@ int mgcg_group_create(MgGroup **out) {
 void mgcg_group_destroy(MgGroup *g) { delete g; }
 
 namespace {
-// Level 0 of a grouped solve lives on the device (the grouped kernels read
-// every level from there); it is bound to the system's arrays once, with the
-// stream drained, and again only if they change.
-template <typename T>
-int bind_level0(MgCgSolver *s, const MgCgSystem &sys, std::vector<Lev<T>> &lv, Lev<T> *d_lv,
-                hipStream_t st, Lev<T> *out) {
-  Lev<T> z = lv[0];
-  z.row = sys.row;
-  z.col = sys.nbr;
-  if (s->fp32) {
-    z.ap = z.apw = reinterpret_cast<T *>(s->ap32);
-    z.anb = z.anbw = reinterpret_cast<T *>(s->anb32);
-    z.b = reinterpret_cast<T *>(s->r32);
-    z.x = reinterpret_cast<T *>(s->z32);
-  } else {
-    z.ap = reinterpret_cast<const T *>(sys.ap);
-    z.anb = reinterpret_cast<const T *>(sys.anb);
-    z.apw = z.anbw = nullptr;
-    z.b = reinterpret_cast<T *>(s->r);
-    z.x = reinterpret_cast<T *>(s->zd);
-  }
-  if (s->bound_row != sys.row || s->bound_ap != sys.ap) {
-    MGCHK(hipStreamSynchronize(st));
-    MGCHK(hipMemcpy(d_lv, &z, sizeof(Lev<T>), hipMemcpyHostToDevice));
-    s->bound_row = sys.row;
-    s->bound_ap = sys.ap;
-  }
-  *out = z;
-  return CFDL_OK;
-}
-
-template <typename T>
-Lev<T> *dev_levels(MgCgSolver *s);
-template <>
-Lev<double> *dev_levels<double>(MgCgSolver *s) { return s->d_lvd; }
-template <>
-Lev<float> *dev_levels<float>(MgCgSolver *s) { return s->d_lvf; }
-template <typename T>
-std::vector<Lev<T>> &host_levels(MgCgSolver *s);
-template <>
-std::vector<Lev<double>> &host_levels<double>(MgCgSolver *s) { return s->lvd; }
-template <>
-std::vector<Lev<float>> &host_levels<float>(MgCgSolver *s) { return s->lvf; }
-
 template <typename T>
 GroupRun<T> &run_of(MgGroup *G);
 template <>
@@ -1188,9 +1397,9 @@ GroupRun<double> &run_of<double>(MgGroup *G) { return G->rd; }
 template <>
 GroupRun<float> &run_of<float>(MgGroup *G) { return G->rf; }
 
-// The solve of mgcg_solve for n systems at once, in phases: begin (level 0
-// bound, descriptors uploaded when they changed; synchronises then, so it
-// runs outside any graph capture), setup (FP32 copies, Galerkin operators,
+// The solve of mgcg_solve for n systems at once, in phases: begin (descriptors
+// uploaded when they changed; synchronises then, so it
+// runs outside any graph capture), setup (level 0's copies, Galerkin operators,
 // initial residual), one iteration at a time (V-cycle and CG step, then the
 // systems' active flags copied to a host slot), finish (the log lines).
 // Every launch covers the systems that take part in its step; each system
@@ -1206,11 +1415,9 @@ int group_begin(MgGroup *G, MgCgSolver *const *ss, const MgCgSystem *sys, int n,
   R.blk = blk;
   R.h.assign(n, MgSlot<T>{});
   std::memset(static_cast<void *>(R.h.data()), 0, sizeof(MgSlot<T>) * n);  // the key compares bytes
-  R.l0.assign(n, Lev<T>{});
   R.maxtop = R.maxlev = R.nitmax = 0;
   for (int k = 0; k < n; k++) {
     MgCgSolver *s = ss[k];
-    MGCALL(bind_level0<T>(s, sys[k], host_levels<T>(s), dev_levels<T>(s), st, &R.l0[k]));
     MgSlot<T> &x = R.h[k];
     x.R = red_of(s->ne);
     x.ne = s->ne;
@@ -1227,10 +1434,9 @@ int group_begin(MgGroup *G, MgCgSolver *const *ss, const MgCgSystem *sys, int n,
     x.p = s->p;
     x.q = s->q;
     x.part = s->part;
-    x.rt = s->fp32 ? reinterpret_cast<T *>(s->r32) : nullptr;
-    x.z = s->fp32 ? reinterpret_cast<T *>(s->z32) : reinterpret_cast<T *>(s->zd);
-    x.ap32 = s->ap32;
-    x.anb32 = s->anb32;
+    x.pos = s->pos;
+    x.rt = host_levels<T>(s)[0].b;
+    x.z = host_levels<T>(s)[0].x;
     x.ctl = s->ctl;
     x.lv = dev_levels<T>(s);
     x.log = sys[k].log;
@@ -1281,18 +1487,14 @@ int group_setup(MgGroup *G, hipStream_t st) {
   const MgSlot<T> *S = static_cast<const MgSlot<T> *>(G->slots);
   const int blk = R.blk;
   int nbk = 0;
-  if (std::is_same<T, float>::value) {
-    nbk = sh.map([&](int k) { return nb(std::max(R.l0[k].nnz, R.ss[k]->ne), blk); });
-    if (nbk > 0) {
-      hipLaunchKernelGGL(g_mg_copy0<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S);
-      G->launches++;
-    }
-  }
+  nbk = sh.map([&](int k) { return nb(R.ss[k]->ne, blk); });
+  hipLaunchKernelGGL(g_mg_copy0<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S);
+  G->launches++;
   for (int l = 0; l + 1 < R.maxlev; l++) {
     nbk = sh.map([&](int k) {
       if (l + 1 >= R.ss[k]->nlev) return 0;
       const Lev<T> &C = host_levels<T>(R.ss[k])[l + 1];
-      return nb(C.n + C.nnz, blk);
+      return nb(C.npad + C.nnz, blk);
     });
     if (nbk > 0) {
       hipLaunchKernelGGL(g_mg_galerkin<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S, l);
@@ -1312,30 +1514,21 @@ int group_iteration(MgGroup *G, hipStream_t st, int slot) {
   GroupShape<T> sh(R);
   const MgSlot<T> *S = static_cast<const MgSlot<T> *>(G->slots);
   const int n = R.n, blk = R.blk;
-  auto colour_count = [&](int k, int l, int c) {
-    return R.ss[k]->cptr[l][c + 1] - R.ss[k]->cptr[l][c];
-  };
-  // colour cc of level l (l < 0: the coarsest level of systems without small
-  // levels), forward or backward
-  auto sweep = [&](int l, bool backward) {
-    int ncmax = 0;
-    for (int k = 0; k < n; k++) {
-      const int lk = l < 0 ? R.ss[k]->nlev - 1 : l;
-      const bool part = l < 0 ? R.ss[k]->lc == R.ss[k]->nlev : l < sh.top_of(k);
-      if (part) ncmax = std::max(ncmax, host_levels<T>(R.ss[k])[lk].ncol);
-    }
-    for (int cc = 0; cc < ncmax; cc++) {
+  // a sweep of level l (l < 0: the coarsest level of systems without small
+  // levels)
+  auto sweep = [&](int l, int mode) {
+    auto level_of = [&](int k) { return l < 0 ? R.ss[k]->nlev - 1 : l; };
+    auto part = [&](int k) { return l < 0 ? R.ss[k]->lc == R.ss[k]->nlev : l < sh.top_of(k); };
+    int steps = 0;
+    for (int k = 0; k < n; k++)
+      if (part(k)) steps = std::max(steps, sweep_steps(host_levels<T>(R.ss[k])[level_of(k)]));
+    for (int i = 0; i < steps; i++) {
       const int nbk = sh.map([&](int k) {
-        const int lk = l < 0 ? R.ss[k]->nlev - 1 : l;
-        const bool part = l < 0 ? R.ss[k]->lc == R.ss[k]->nlev : l < sh.top_of(k);
-        const int nc = host_levels<T>(R.ss[k])[lk].ncol;
-        if (!part || cc >= nc) return 0;
-        const int c = backward ? nc - 1 - cc : cc;
-        return nb(colour_count(k, lk, c), blk);
+        const int lk = level_of(k);
+        return part(k) ? sweep_blocks(R.ss[k], lk, host_levels<T>(R.ss[k])[lk], i, mode, blk) : 0;
       });
       if (nbk > 0) {
-        hipLaunchKernelGGL(g_mg_sweep<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S, l, cc,
-                           backward ? 1 : 0);
+        hipLaunchKernelGGL(g_mg_sweep<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S, l, i, mode);
         G->launches++;
       }
     }
@@ -1343,40 +1536,41 @@ int group_iteration(MgGroup *G, hipStream_t st, int slot) {
   int nbk = 0;
   // V-cycle
   for (int l = 0; l < R.maxtop; l++) {
-    sweep(l, false);
-    // one lane count for the launch: the largest of the systems taking part
-    // (0, one lane per aggregate, if any needs it); sums do not depend on it
-    int nl = 1;
-    for (int k = 0; k < n; k++)
-      if (l < sh.top_of(k))
-        nl = (nl == 0 || R.ss[k]->lanes[l] == 0) ? 0 : std::max(nl, R.ss[k]->lanes[l]);
+    sweep(l, kFwd0);
+    nbk = sh.map([&](int k) { return l < sh.top_of(k) ? nb(R.ss[k]->open[l], blk) : 0; });
+    if (nbk > 0) {
+      hipLaunchKernelGGL(g_mg_residual<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S, l);
+      G->launches++;
+    }
     nbk = sh.map([&](int k) {
-      return l < sh.top_of(k) ? nb(host_levels<T>(R.ss[k])[l + 1].n * (nl > 0 ? nl : 1), blk) : 0;
+      return l < sh.top_of(k) ? nb(host_levels<T>(R.ss[k])[l + 1].npad, blk) : 0;
     });
     if (nbk > 0) {
-      launch_restrict_group<T>(nl, nbk, blk, sh.g, S, l, st);
+      hipLaunchKernelGGL(g_mg_restrict<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S, l);
       G->launches++;
     }
   }
   nbk = sh.map([&](int k) { return R.ss[k]->lc < R.ss[k]->nlev ? 1 : 0; });
   if (nbk > 0) {
-    hipLaunchKernelGGL(g_mg_coarse<T>, dim3(nbk), dim3(kCoarseThreads), 0, st, sh.g, S);
+    size_t lds = 0;
+    for (int k = 0; k < n; k++) lds = std::max(lds, R.ss[k]->coarse_lds);
+    hipLaunchKernelGGL(g_mg_coarse<T>, dim3(nbk), dim3(kCoarseThreads), lds, st, sh.g, S);
     G->launches++;
   }
   bool any_flat = false;
   for (int k = 0; k < n; k++) any_flat = any_flat || R.ss[k]->lc == R.ss[k]->nlev;
   if (any_flat)
     for (int r = 0; r < kCoarseSweeps; r++) {
-      sweep(-1, false);
-      sweep(-1, true);
+      sweep(-1, r == 0 ? kFwd0 : kFwd);
+      sweep(-1, kBwd);
     }
   for (int l = R.maxtop - 1; l >= 0; l--) {
-    nbk = sh.map([&](int k) { return l < sh.top_of(k) ? nb(host_levels<T>(R.ss[k])[l].n, blk) : 0; });
+    nbk = sh.map([&](int k) { return l < sh.top_of(k) ? nb(R.ss[k]->prolonged[l], blk) : 0; });
     if (nbk > 0) {
       hipLaunchKernelGGL(g_mg_prolong<T>, dim3(nbk), dim3(blk), 0, st, sh.g, S, l);
       G->launches++;
     }
-    sweep(l, true);
+    sweep(l, kBwd);
   }
   // CG
   nbk = sh.map([&](int k) { return R.h[k].R.nblk; });
