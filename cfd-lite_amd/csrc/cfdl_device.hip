@@ -1713,56 +1713,88 @@ k_gs_tiles_lds(int batch0, const int4 *__restrict__ bdesc, const int *__restrict
 // (calc_residual, :239-251).  Fixed-order tree, so reproducible.
 // rout, when given, receives each cell's r rounded to FP32 (the right-hand
 // side of the mixed-precision correction system).
-__device__ inline void d_resid_partial(int bx_, SysDesc s, int chunk, int nblk, int absmax, double *part,
-                                float *rout) {
-  __shared__ double ssum[kBlock], smax[kBlock];
-  const int y = blockIdx.y, x = bx_, tid = threadIdx.x;
-  const int lo = s.beg[y] + x * chunk;
-  const int hi = min(lo + chunk, s.end[y]);
-  const double *phi = s.phi[y], *b = s.b[y];
-  double sum = 0.0, mx = 0.0;
-  for (int e = lo + tid; e < hi; e += blockDim.x) {
-    double r = b[e];
+// NC right-hand sides that share the cells and the matrix (NC = 3: u, v, w)
+// are summed in one pass over the rows, each in the order it has alone; a
+// pass per right-hand side read the rows three times (the eight-case batch:
+// 239 us against 64 us).
+template <int NC>
+__device__ inline void d_resid_partial(int bx_, const SysDesc &s, int chunk, int nblk, int absmax,
+                                       double *part, float *rout) {
+  __shared__ double ssum[NC][kBlock], smax[NC][kBlock];
+  const int y0 = NC == 1 ? blockIdx.y : 0, x = bx_, tid = threadIdx.x;
+  const int lo = s.beg[y0] + x * chunk;
+  const int hi = min(lo + chunk, s.end[y0]);
+  double sum[NC], mx[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) sum[c] = mx[c] = 0.0;
+  for (int e = lo + tid; e < hi; e += kBlock) {
+    double r[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++) r[c] = s.b[y0 + c][e];
     const int r0 = s.row[e], r1 = s.row[e + 1];
-    if (r1 - r0 == 6) {  // hexahedral row: all loads first, the sum in CSR order
+    if (r1 - r0 == 6) {  // hexahedral row: all loads first, the sums in CSR order
       int nb[6];
-      double an[6], v[6];
+      double an[6], v[NC][6];
 #pragma unroll
       for (int k = 0; k < 6; k++) {
         nb[k] = s.nbr[r0 + k];
         an[k] = s.anb[r0 + k];
       }
 #pragma unroll
-      for (int k = 0; k < 6; k++) v[k] = phi[nb[k]];
+      for (int c = 0; c < NC; c++)
 #pragma unroll
-      for (int k = 0; k < 6; k++) r = r + an[k] * v[k];
+        for (int k = 0; k < 6; k++) v[c][k] = s.phi[y0 + c][nb[k]];
+#pragma unroll
+      for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int k = 0; k < 6; k++) r[c] = r[c] + an[k] * v[c][k];
     } else {
-      for (int k = r0; k < r1; k++) r = r + s.anb[k] * phi[s.nbr[k]];
+      for (int k = r0; k < r1; k++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) r[c] = r[c] + s.anb[k] * s.phi[y0 + c][s.nbr[k]];
     }
-    r = r - s.ap[e] * phi[e];
-    if (rout) rout[e] = static_cast<float>(r);
-    if (absmax) r = fabs(r);
-    mx = fmax(r, mx);
-    sum = sum + r * r;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      double rc = r[c] - s.ap[e] * s.phi[y0 + c][e];
+      if (rout) rout[e] = static_cast<float>(rc);
+      if (absmax) rc = fabs(rc);
+      mx[c] = fmax(rc, mx[c]);
+      sum[c] = sum[c] + rc * rc;
+    }
   }
-  ssum[tid] = sum;
-  smax[tid] = mx;
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    ssum[c][tid] = sum[c];
+    smax[c][tid] = mx[c];
+  }
   __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-    if (tid < off) {
-      ssum[tid] = ssum[tid] + ssum[tid + off];
-      smax[tid] = fmax(smax[tid], smax[tid + off]);
+  // s[t] += s[t + h] for h = 128, 64 in LDS and 32 .. 1 by shuffles
+  if (tid < 128)
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      ssum[c][tid] = ssum[c][tid] + ssum[c][tid + 128];
+      smax[c][tid] = fmax(smax[c][tid], smax[c][tid + 128]);
     }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    part[2 * (y * nblk + x)] = ssum[0];
-    part[2 * (y * nblk + x) + 1] = smax[0];
-  }
+  __syncthreads();
+  if (tid < 64)
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      double a = ssum[c][tid] + ssum[c][tid + 64], m = fmax(smax[c][tid], smax[c][tid + 64]);
+#pragma unroll
+      for (int h = 32; h >= 1; h >>= 1) {
+        a = a + __shfl_down(a, h, 64);
+        m = fmax(m, __shfl_down(m, h, 64));
+      }
+      if (tid == 0) {
+        part[2 * ((y0 + c) * nblk + x)] = a;
+        part[2 * ((y0 + c) * nblk + x) + 1] = m;
+      }
+    }
 }
-__global__ void k_resid_partial(SysDesc s, int chunk, int nblk, int absmax, double *part,
-                                float *rout) {
-  d_resid_partial(blockIdx.x, s, chunk, nblk, absmax, part, rout);
+template <int NC>
+__global__ void __launch_bounds__(kBlock)
+k_resid_partial(SysDesc s, int chunk, int nblk, int absmax, double *part, float *rout) {
+  d_resid_partial<NC>(blockIdx.x, s, chunk, nblk, absmax, part, rout);
 }
 
 __device__ inline void d_resid_final(int bx_, const double *part, int nblk, double *red) {
@@ -1909,6 +1941,23 @@ __global__ void k_log_pc(const PcCtl *c, LogLine *log, int *nlog) {
   *nlog = k + 1;
 }
 
+// One row's n coefficients from src[r0 ..] to dst[d0 ..].  A hexahedral row's
+// six loads go out before its stores: in a loop each store waits for its own
+// load, a memory latency per entry (k_pc_assemble 246 -> 75 us, k_tile_gather
+// 212 -> 125 us at 128^3).
+__device__ inline void copy_row(double *__restrict__ dst, int d0, int n,
+                                const double *__restrict__ src, int r0) {
+  if (n == 6) {
+    double v[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) v[k] = src[r0 + k];
+#pragma unroll
+    for (int k = 0; k < 6; k++) dst[d0 + k] = v[k];
+  } else {
+    for (int k = 0; k < n; k++) dst[d0 + k] = src[r0 + k];
+  }
+}
+
 // assemble_coef / update_halos / update_phi, mod_subdomains.f90:162-229
 __global__ void k_pc_assemble(int ne, const int *l2g_cell, const int *rowp, const int *rowg,
                               const double *ap, const double *b, const double *anb,
@@ -1917,12 +1966,12 @@ __global__ void k_pc_assemble(int ne, const int *l2g_cell, const int *rowp, cons
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= ne) return;
   const int g = l2g_cell[c];
-  ap_p[c] = ap[g];
-  rap_p[c] = rcp_of(ap[g]);
+  const double a = ap[g];
+  ap_p[c] = a;
+  rap_p[c] = rcp_of(a);
   b_p[c] = b[g];
   phic_p[c] = phi[g];
-  const int kg = rowg[g];
-  for (int k = rowp[c]; k < rowp[c + 1]; k++) anb_p[k] = anb[kg + (k - rowp[c])];
+  copy_row(anb_p, rowp[c], rowp[c + 1] - rowp[c], anb, rowg[g]);
 }
 __global__ void k_gather(int n, const int *idx, const double *src, double *dst) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1956,14 +2005,24 @@ __device__ inline void d_tile_gather(int bx_, TileMap t) {
   const int i = bx_ * blockDim.x + threadIdx.x;
   if (i < t.ne) {
     const int g = t.l2g[i];
-    t.ap_m[i] = t.ap[g];
-    t.rap_m[i] = rcp_of(t.ap[g]);
     const int r = t.rowm[i], rg = t.rowg[g], n = t.rowg[g + 1] - rg;
-    for (int k = 0; k < n; k++) t.anb_m[r + k] = t.anb[rg + k];
-    for (int y = 0; y < t.ny; y++) {
-      t.b_m[y][i] = t.b[y][g];
-      t.phi_m[y][i] = t.phi[y][g];
+    const double a = t.ap[g];
+    double b[3], phi[3];
+#pragma unroll
+    for (int y = 0; y < 3; y++) {
+      const int yc = y < t.ny ? y : 0;
+      b[y] = t.b[yc][g];
+      phi[y] = t.phi[yc][g];
     }
+    copy_row(t.anb_m, r, n, t.anb, rg);
+    t.ap_m[i] = a;
+    t.rap_m[i] = rcp_of(a);
+#pragma unroll
+    for (int y = 0; y < 3; y++)
+      if (y < t.ny) {
+        t.b_m[y][i] = b[y];
+        t.phi_m[y][i] = phi[y];
+      }
   } else if (i < t.ne + t.nbf) {
     for (int y = 0; y < t.ny; y++) t.phi_m[y][i] = t.phi[y][i];
   }
@@ -1975,7 +2034,12 @@ __device__ inline void d_tile_scatter(int bx_, TileMap t) {
   const int i = bx_ * blockDim.x + threadIdx.x;
   if (i >= t.ne) return;
   const int g = t.l2g[i];
-  for (int y = 0; y < t.ny; y++) t.phi[y][g] = t.phi_m[y][i];
+  double v[3];
+#pragma unroll
+  for (int y = 0; y < 3; y++) v[y] = t.phi_m[y < t.ny ? y : 0][i];
+#pragma unroll
+  for (int y = 0; y < 3; y++)
+    if (y < t.ny) t.phi[y][g] = v[y];
 }
 __global__ void k_tile_scatter(TileMap t) {
   d_tile_scatter(blockIdx.x, t);
@@ -2039,10 +2103,9 @@ __global__ void gb_tile_scatter(GroupMap g, const BSlot *__restrict__ S) {
   BSLOT;
   d_tile_scatter(bx, x.tmap);
 }
-// grid (blocks, 3): the three right-hand sides in y, as k_resid_partial
 __global__ void __launch_bounds__(kBlock) gb_resid_partial(GroupMap g, const BSlot *__restrict__ S) {
   BSLOT;
-  d_resid_partial(bx, x.sys, x.chunk_g, x.nblk_g, 1, x.part, nullptr);
+  d_resid_partial<3>(bx, x.sys, x.chunk_g, x.nblk_g, 1, x.part, nullptr);
 }
 // grid (cases, 3): one block per case and right-hand side
 __global__ void __launch_bounds__(kBlock) gb_resid_final(GroupMap g, const BSlot *__restrict__ S) {
@@ -2529,8 +2592,17 @@ static int pc_sweep_tiled(cfdl_ctx *c, const SysDesc &sys, bool forward, const i
 
 static int residual(cfdl_ctx *c, const SysDesc &sys, int nblk, int chunk, int absmax,
                     float *rout = nullptr) {
-  hipLaunchKernelGGL(k_resid_partial, dim3(nblk, sys.ny), dim3(kBlock), 0, c->st, sys, chunk,
-                     nblk, absmax, c->part, rout);
+  // three right-hand sides are always u, v, w on the whole mesh (solve_gs_n);
+  // the subdomains of a pc system have ranges of their own
+  bool shared = sys.ny == 3;
+  for (int y = 1; y < sys.ny; y++)
+    shared = shared && sys.beg[y] == sys.beg[0] && sys.end[y] == sys.end[0];
+  if (shared)
+    hipLaunchKernelGGL(k_resid_partial<3>, dim3(nblk), dim3(kBlock), 0, c->st, sys, chunk, nblk,
+                       absmax, c->part, rout);
+  else
+    hipLaunchKernelGGL(k_resid_partial<1>, dim3(nblk, sys.ny), dim3(kBlock), 0, c->st, sys, chunk,
+                       nblk, absmax, c->part, rout);
   hipLaunchKernelGGL(k_resid_final, dim3(sys.ny), dim3(kBlock), 0, c->st, c->part, nblk, c->red);
   HIPCHK(hipGetLastError());
   return CFDL_OK;
@@ -4234,7 +4306,7 @@ static int resid_run(int ne, const int *row, const int *nbr, const double *ap, c
   s.ap = ap;
   s.anb = anb;
   double *part = buf, *red = buf + 2 * nblk;
-  hipLaunchKernelGGL(k_resid_partial, dim3(nblk, 1), dim3(kBlock), 0, st, s, chunk, nblk, 0, part,
+  hipLaunchKernelGGL(k_resid_partial<1>, dim3(nblk, 1), dim3(kBlock), 0, st, s, chunk, nblk, 0, part,
                      static_cast<float *>(nullptr));
   hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(kBlock), 0, st, static_cast<const double *>(part),
                      nblk, red);
@@ -4532,7 +4604,7 @@ int seg_prefix(cfdl_batch *b, int blk) {
   nb = L.map([&](cfdl_ctx *c) { return nbk(int64_t{c->ne} + c->nbf, blk); });
   hipLaunchKernelGGL(gb_tile_gather, dim3(nb), dim3(blk), 0, st, L.g, S);
   const int np = L.map([&](cfdl_ctx *c) { return c->nblk_g; });
-  hipLaunchKernelGGL(gb_resid_partial, dim3(np, 3), dim3(kBlock), 0, st, L.g, S);
+  hipLaunchKernelGGL(gb_resid_partial, dim3(np), dim3(kBlock), 0, st, L.g, S);
   nb = L.map([&](cfdl_ctx *) { return 1; });
   hipLaunchKernelGGL(gb_resid_final, dim3(nb, 3), dim3(kBlock), 0, st, L.g, S);
   hipLaunchKernelGGL(gb_gs_init, dim3(nb), dim3(64), 0, st, L.g, S);
@@ -4558,7 +4630,7 @@ int seg_gs(cfdl_batch *b, int blk, int slot) {
       if (nb > 0) hipLaunchKernelGGL(gb_gs_colour, dim3(nb), dim3(blk), 0, st, L.g, S, i, d, 1.0);
     }
   const int np = L.map([&](cfdl_ctx *c) { return c->nblk_g; });
-  hipLaunchKernelGGL(gb_resid_partial, dim3(np, 3), dim3(kBlock), 0, st, L.g, S);
+  hipLaunchKernelGGL(gb_resid_partial, dim3(np), dim3(kBlock), 0, st, L.g, S);
   const int nb = L.map([&](cfdl_ctx *) { return 1; });
   hipLaunchKernelGGL(gb_resid_final, dim3(nb, 3), dim3(kBlock), 0, st, L.g, S);
   hipLaunchKernelGGL(gb_gs_iter_end, dim3(nb), dim3(64), 0, st, L.g, S);

@@ -488,6 +488,14 @@ __device__ inline void d_mg_copy0(int g, const Lev<T> &L, const int *__restrict_
   if (g >= L.n) return;
   const int p = pos[g], e = mg_entry(L, p), r0 = row[g], r1 = row[g + 1];
   L.ap[p] = static_cast<T>(ap[g]);
+  if (r1 - r0 == 6) {  // the loads go out before the stores
+    double v[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) v[k] = anb[r0 + k];
+#pragma unroll
+    for (int k = 0; k < 6; k++) L.anb[e + 64 * k] = static_cast<T>(v[k]);
+    return;
+  }
   for (int k = r0; k < r1; k++) L.anb[e + 64 * (k - r0)] = static_cast<T>(anb[k]);
 }
 
