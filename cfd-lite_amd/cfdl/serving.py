@@ -33,10 +33,10 @@ from .mesh import Mesh
 from .solver import UVWP, Batch
 
 # Device footprint of one context: mesh, fields, the momentum system in
-# colour numbering, the multigrid hierarchy and the FP32 copies; about
-# 64 MiB plus 1.3 KB per cell.
+# colour numbering, the multigrid hierarchy, the faces' fixed geometry and
+# the FP32 copies; about 64 MiB plus 1.8 KB per cell.
 BYTES_PER_CONTEXT = 64 << 20
-BYTES_PER_CELL = 1344
+BYTES_PER_CELL = 1760
 KINDS = ("cavity", "channel")
 
 

@@ -105,22 +105,31 @@ struct MeshDev {
   // FP32 copies of the geometry and properties for the FP32 assembly (null
   // until cfdl_set_assembly_precision selects it)
   const float *xc32, *yc32, *zc32, *vol32, *aip32, *rip32, *rho32, *mu32;
+  // per interior face, what the assembly and the flux correction need of its
+  // fixed geometry (k_face_geo): fa = area, weight of the neighbour seen from
+  // the owner and from the other cell, (r_nb - r_P).n; fd = |r_nb - r_P|, the
+  // distance of the two cells' feet on the face normal, and the vector
+  // between the feet (owner to other).  FP32 copies computed from the FP32
+  // geometry.
+  const double *fa, *fd;
+  const float *fa32, *fd32;
 };
 
 // the geometry of the arithmetic type T: the mesh's FP64 arrays, or their
 // FP32 copies
 struct Geo64 {
-  const double *xc, *yc, *zc, *vol, *aip, *rip, *rho, *mu;
+  const double *xc, *yc, *zc, *vol, *aip, *rip, *rho, *mu, *fa, *fd;
 };
 struct Geo32 {
-  const float *xc, *yc, *zc, *vol, *aip, *rip, *rho, *mu;
+  const float *xc, *yc, *zc, *vol, *aip, *rip, *rho, *mu, *fa, *fd;
 };
 template <typename T>
 __device__ inline auto geo_of(const MeshDev &m) {
   if constexpr (sizeof(T) == 8)
-    return Geo64{m.xc, m.yc, m.zc, m.vol, m.aip, m.rip, m.rho, m.mu};
+    return Geo64{m.xc, m.yc, m.zc, m.vol, m.aip, m.rip, m.rho, m.mu, m.fa, m.fd};
   else
-    return Geo32{m.xc32, m.yc32, m.zc32, m.vol32, m.aip32, m.rip32, m.rho32, m.mu32};
+    return Geo32{m.xc32, m.yc32, m.zc32, m.vol32, m.aip32, m.rip32, m.rho32, m.mu32,
+                 m.fa32, m.fd32};
 }
 
 // energy equation state (energy_t, mod_energy.f90:4-10): temperature t and
@@ -237,6 +246,44 @@ __device__ inline void centre(const MeshDev &m, int e, double *r) {
   r[0] = m.xc[e];
   r[1] = m.yc[e];
   r[2] = m.zc[e];
+}
+
+// The fixed geometry of the interior faces, once per context, by the
+// expressions calc_coef_uvw, calc_coef_p and update_uvwp evaluate
+// (mod_uvwp.f90:186-206), seen from the owner.  From the other cell the
+// normal, the centre distance vector and the feet's vector change sign and
+// nothing else does (every product and sum is the negated or the same one),
+// except the weight, whose two values are kept.  With them and a thread per
+// cell (d_coef_uvw6) at 128^3: k_coef_uvw6 713 -> 575 us, k_coef_p6 252 -> 183
+// us, k_update_faces 129 -> 92 us.  (calc_mip keeps its own: it is bound by
+// memory and reads as many bytes either way, 196 us against 209 us.)
+template <typename T>
+__global__ void k_face_geo(MeshDev m, T *fa, T *fd) {
+  const auto G = geo_of<T>(m);
+  const int fg = blockIdx.x * blockDim.x + threadIdx.x;
+  if (fg >= m.nf) return;
+  const int e = m.fcell[fg], nb = m.nbr[m.own[fg]];
+  if (nb >= m.ne) return;
+  const T *a = G.aip + 3 * fg, *rip = G.rip + 3 * fg;
+  const T area = area_of(a);
+  const T rp[3] = {G.xc[e], G.yc[e], G.zc[e]}, rpnb[3] = {G.xc[nb], G.yc[nb], G.zc[nb]};
+  T nrm[3], dr[3], drip[3], rpp[3], rnp[3], drp[3];
+  for (int i = 0; i < 3; i++) nrm[i] = a[i] / area;
+  for (int i = 0; i < 3; i++) dr[i] = rpnb[i] - rp[i];
+  for (int i = 0; i < 3; i++) drip[i] = rip[i] - rp[i];
+  T t = dot3(drip, nrm);
+  for (int i = 0; i < 3; i++) rpp[i] = rip[i] - t * nrm[i];
+  for (int i = 0; i < 3; i++) drip[i] = rip[i] - rpnb[i];
+  t = dot3(drip, nrm);
+  for (int i = 0; i < 3; i++) rnp[i] = rip[i] - t * nrm[i];
+  for (int i = 0; i < 3; i++) drp[i] = rnp[i] - rpp[i];
+  fa[4 * fg] = area;
+  fa[4 * fg + 1] = vec_weight(rip, rp, rpnb);
+  fa[4 * fg + 2] = vec_weight(rip, rpnb, rp);
+  fa[4 * fg + 3] = dot3(dr, nrm);
+  fd[5 * fg] = sqrt(dot3(dr, dr));
+  fd[5 * fg + 1] = sqrt(dot3(drp, drp));
+  for (int i = 0; i < 3; i++) fd[5 * fg + 2 + i] = drp[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -489,96 +536,70 @@ __global__ void k_coef_uvw(MeshDev m, FieldsDev f, double dt, double alpha_u) {
 }
 
 // The same assembly for meshes whose rows all have six entries (row e at 6e),
-// six threads per cell: thread j of a cell computes the terms of its row
-// entry j (the loop body above) into LDS, then the cell's first thread adds
-// them in CSR order exactly as the loop does (interior entries only for the
-// flux, secondary-stress and deferred-correction sums) and finishes the cell.
-// Interior anb are written by their entry's thread, boundary anb by the cell.
-constexpr int kFaceThreads = 256, kFaceCells = kFaceThreads / 6;
+// from the faces' fixed geometry (k_face_geo).  One thread per cell: entry k
+// of neighbouring threads' cells has neighbouring cells and faces, so a
+// wavefront's loads of it fall on few lines.  With a thread per entry (six per
+// cell, sums through LDS) each load touched up to 64 lines, and the L1's
+// lookups bound the kernel, with or without the fixed geometry.
 template <typename T>
-__device__ inline void d_coef_uvw6(int bx_, MeshDev m, FieldsDev f, double dt_, double alpha_u_) {
+__device__ inline void d_coef_uvw6(int bx_, const MeshDev &m, const FieldsDev &f, double dt_,
+                                   double alpha_u_) {
   // T = double: the reference's FP64 assembly bit for bit.  T = float: the
   // same operations in FP32 on the FP32 geometry copies and on the fields
   // rounded to FP32 (the FP32 assembly; results stored as FP64).
+  const int e = bx_ * blockDim.x + threadIdx.x;
+  if (e >= m.ne) return;
   const auto G = geo_of<T>(m);
   const T one = static_cast<T>(1), zero = static_cast<T>(0);
   const T dt = static_cast<T>(dt_), alpha_u = static_cast<T>(alpha_u_);
   auto ld = [](double x) { return static_cast<T>(x); };
-  __shared__ T st[9][kFaceThreads];  // d, fnb, fl, secondary stress, deferred correction
-  __shared__ int sin_[kFaceThreads];  // the entry is interior
-  const int lc = threadIdx.x / 6, j = threadIdx.x - 6 * lc;
-  const int e = bx_ * kFaceCells + lc;
-  const bool valid = lc < kFaceCells && e < m.ne;
-  if (valid) {
-    const int k = 6 * e + j;
-    const int nb = m.nbr[k];
-    T fnb = zero, d = zero, fl = zero, ss[3] = {zero, zero, zero}, dfc[3] = {zero, zero, zero};
-    if (nb < m.ne) {
-      const T rp[3] = {G.xc[e], G.yc[e], G.zc[e]};
-      const int fs = m.fsg[k];
-      const T sg = fs >= 0 ? one : -one;
-      const int fg = abs(fs) - 1;
-      const T *a = G.aip + 3 * fg, *rip = G.rip + 3 * fg;
-      const T area = area_of(a);
-      T nrm[3], dr[3], drip[3], rpp[3], rnp[3], drp[3];
-      for (int i = 0; i < 3; i++) nrm[i] = sg * a[i] / area;
-      const T rpnb[3] = {G.xc[nb], G.yc[nb], G.zc[nb]};
-      for (int i = 0; i < 3; i++) dr[i] = rpnb[i] - rp[i];
-      const T ds = sqrt(dot3(dr, dr));
-      const T wt = vec_weight(rip, rp, rpnb);
-      for (int i = 0; i < 3; i++) drip[i] = rip[i] - rp[i];
-      T t = dot3(drip, nrm);
-      for (int i = 0; i < 3; i++) rpp[i] = rip[i] - t * nrm[i];
-      for (int i = 0; i < 3; i++) drip[i] = rip[i] - rpnb[i];
-      t = dot3(drip, nrm);
-      for (int i = 0; i < 3; i++) rnp[i] = rip[i] - t * nrm[i];
-      for (int i = 0; i < 3; i++) drp[i] = rnp[i] - rpp[i];
-      const T dsp = sqrt(dot3(drp, drp));
-      fl = -(sg * ld(f.mip[fg]));
-      fnb = fmax(fl, zero);
-      const T muip = (one - wt) * G.mu[e] + wt * G.mu[nb];
-      d = muip * area / ds;
-      const T ge[3][3] = {{ld(f.gu[3 * e]), ld(f.gu[3 * e + 1]), ld(f.gu[3 * e + 2])},
-                          {ld(f.gv[3 * e]), ld(f.gv[3 * e + 1]), ld(f.gv[3 * e + 2])},
-                          {ld(f.gw[3 * e]), ld(f.gw[3 * e + 1]), ld(f.gw[3 * e + 2])}};
-      const T gn[3][3] = {{ld(f.gu[3 * nb]), ld(f.gu[3 * nb + 1]), ld(f.gu[3 * nb + 2])},
-                          {ld(f.gv[3 * nb]), ld(f.gv[3 * nb + 1]), ld(f.gv[3 * nb + 2])},
-                          {ld(f.gw[3 * nb]), ld(f.gw[3 * nb + 1]), ld(f.gw[3 * nb + 2])}};
-      for (int mm = 0; mm < 3; mm++) {
-        T gip[3];
-        for (int q = 0; q < 3; q++) gip[q] = (one - wt) * ge[q][mm] + wt * gn[q][mm];
-        ss[mm] = muip * area * dot3(gip, dr) / ds;
-      }
-      for (int q = 0; q < 3; q++) {
-        T gip[3];
-        for (int i = 0; i < 3; i++) gip[i] = (one - wt) * ge[q][i] + wt * gn[q][i];
-        dfc[q] = muip * area * (dot3(gip, drp) / dsp - dot3(gip, dr) / ds);
-      }
-      f.anb[k] = static_cast<double>(d + fnb);
-    }
-    st[0][threadIdx.x] = d;
-    st[1][threadIdx.x] = fnb;
-    st[2][threadIdx.x] = fl;
-    for (int i = 0; i < 3; i++) {
-      st[3 + i][threadIdx.x] = ss[i];
-      st[6 + i][threadIdx.x] = dfc[i];
-    }
-    sin_[threadIdx.x] = nb < m.ne;
+  int nbs[6], fss[6];
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    nbs[k] = m.nbr[6 * e + k];
+    fss[k] = m.fsg[6 * e + k];
   }
-  __syncthreads();
-  if (!valid || j != 0) return;
-  const T rp[3] = {G.xc[e], G.yc[e], G.zc[e]};
+  const T rp[3] = {G.xc[e], G.yc[e], G.zc[e]}, mue = G.mu[e];
+  T ge[3][3];
+  for (int i = 0; i < 3; i++) {
+    ge[0][i] = ld(f.gu[3 * e + i]);
+    ge[1][i] = ld(f.gv[3 * e + i]);
+    ge[2][i] = ld(f.gw[3 * e + i]);
+  }
   T ap = zero, sumf = zero, sumss[3] = {zero, zero, zero}, sumdefc[3] = {zero, zero, zero};
   T anbk[6];
-  for (int q = 0; q < 6; q++) {
-    const int t = threadIdx.x + q;
-    const T d = st[0][t], fnb = st[1][t];
-    if (sin_[t]) {
-      sumf = sumf + st[2][t];
-      for (int i = 0; i < 3; i++) sumss[i] = sumss[i] + st[3 + i][t];
-      for (int i = 0; i < 3; i++) sumdefc[i] = sumdefc[i] + st[6 + i][t];
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    const int nb = nbs[k], fs = fss[k], fg = abs(fs) - 1;
+    T d = zero, fnb = zero;
+    if (nb < m.ne) {
+      const T sg = fs >= 0 ? one : -one;
+      const T *fa = G.fa + 4 * fg, *fd = G.fd + 5 * fg;
+      const T area = fa[0], wt = fs >= 0 ? fa[1] : fa[2], ds = fd[0], dsp = fd[1];
+      const T rpnb[3] = {G.xc[nb], G.yc[nb], G.zc[nb]};
+      T dr[3], drp[3];
+      for (int i = 0; i < 3; i++) dr[i] = rpnb[i] - rp[i];
+      // 0 - x and not -x: from the other side a zero is +0 too
+      for (int i = 0; i < 3; i++) drp[i] = fs >= 0 ? fd[2 + i] : zero - fd[2 + i];
+      const T fl = -(sg * ld(f.mip[fg]));
+      fnb = fmax(fl, zero);
+      sumf = sumf + fl;
+      const T muip = (one - wt) * mue + wt * G.mu[nb];
+      d = muip * area / ds;
+      T gip[3][3];  // the face gradients of u, v, w
+      for (int i = 0; i < 3; i++) {
+        gip[0][i] = (one - wt) * ge[0][i] + wt * ld(f.gu[3 * nb + i]);
+        gip[1][i] = (one - wt) * ge[1][i] + wt * ld(f.gv[3 * nb + i]);
+        gip[2][i] = (one - wt) * ge[2][i] + wt * ld(f.gw[3 * nb + i]);
+      }
+      for (int q = 0; q < 3; q++) {
+        const T across[3] = {gip[0][q], gip[1][q], gip[2][q]};
+        sumss[q] = sumss[q] + muip * area * dot3(across, dr) / ds;
+      }
+      for (int q = 0; q < 3; q++)
+        sumdefc[q] = sumdefc[q] + muip * area * (dot3(gip[q], drp) / dsp - dot3(gip[q], dr) / ds);
     }
-    anbk[q] = d + fnb;
+    anbk[k] = d + fnb;
     ap = ap + d + fnb;
   }
   const T vol = G.vol[e];
@@ -588,8 +609,12 @@ __device__ inline void d_coef_uvw6(int bx_, MeshDev m, FieldsDev f, double dt_, 
   T bu = ap0 * ld(f.u0[e]) + sumf * ue - vol * ld(f.gp[3 * e]) + sumss[0] + sumdefc[0];
   T bv = ap0 * ld(f.v0[e]) + sumf * ve - vol * ld(f.gp[3 * e + 1]) + sumss[1] + sumdefc[1];
   T bw = ap0 * ld(f.w0[e]) + sumf * we - vol * ld(f.gp[3 * e + 2]) + sumss[2] + sumdefc[2];
-  for (int q = 0; q < 6; q++)
-    if (!sin_[threadIdx.x + q]) f.anb[6 * e + q] = static_cast<double>(anbk[q]);
+  // adds x to the row's entry k, in the order the boundary loop reaches it
+  auto add = [&](int k, T d, T c) {
+#pragma unroll
+    for (int q = 0; q < 6; q++)
+      if (q == k) anbk[q] = anbk[q] + d + c;
+  };
   for (int q = m.bcrow[e]; q < m.bcrow[e + 1]; q++) {
     const int k = m.bcslot[q], H = m.nbr[k];
     const int fg = m.fsg[k] - 1;  // boundary faces are always owner side
@@ -610,8 +635,7 @@ __device__ inline void d_coef_uvw6(int bx_, MeshDev m, FieldsDev f, double dt_, 
       bv = bv + fl * ve;
       bw = bw + fl * we;
       ap = ap + dd + fnb;
-      anbk[k - 6 * e] = anbk[k - 6 * e] + dd + fnb;
-      f.anb[k] = static_cast<double>(anbk[k - 6 * e]);
+      add(k - 6 * e, dd, fnb);
       continue;
     }
     if (kind != CFDL_BC_SYMMETRY) {  // 'dirichlet', :255-265
@@ -626,9 +650,10 @@ __device__ inline void d_coef_uvw6(int bx_, MeshDev m, FieldsDev f, double dt_, 
       bw = bw + d * vr[2] - d * we;
     }
     ap = ap + d + fz;
-    anbk[k - 6 * e] = anbk[k - 6 * e] + d + fz;
-    f.anb[k] = static_cast<double>(anbk[k - 6 * e]);
+    add(k - 6 * e, d, fz);
   }
+#pragma unroll
+  for (int q = 0; q < 6; q++) f.anb[6 * e + q] = static_cast<double>(anbk[q]);
   if (alpha_u != one) {
     const T apr = ap / alpha_u, da = apr - ap;
     bu = bu + da * ue;
@@ -646,7 +671,7 @@ __device__ inline void d_coef_uvw6(int bx_, MeshDev m, FieldsDev f, double dt_, 
   f.dc[e] = static_cast<double>(vol / dc);
 }
 template <typename T>
-__global__ void __launch_bounds__(kFaceThreads)
+__global__ void __launch_bounds__(kBlock)
 k_coef_uvw6(MeshDev m, FieldsDev f, double dt_, double alpha_u_) {
   d_coef_uvw6<T>(blockIdx.x, m, f, dt_, alpha_u_);
 }
@@ -751,18 +776,34 @@ __global__ void k_temperature(MeshDev m, EnergyDev en) {
 // calc_grad + matinv3, mod_solver.f90:8-81: weighted least squares over all
 // CSR neighbours (boundary halos included), one thread per cell.
 // ---------------------------------------------------------------------------
-__device__ inline void d_grad(int bx_, MeshDev m, const double *__restrict__ phi, double *__restrict__ grad) {
+// NC fields share the weights and the inverse of one cell (u, v, w: one pass
+// of 123 us at 128^3 instead of three of 62 us).
+template <int NC>
+struct GradArgs {
+  const double *phi[NC];
+  double *grad[NC];
+};
+template <int NC>
+__device__ inline void d_grad(int bx_, const MeshDev &m, const GradArgs<NC> &f) {
   const int e = bx_ * blockDim.x + threadIdx.x;
   if (e >= m.ne) return;
   double a11 = 0.0, a12 = 0.0, a13 = 0.0, a22 = 0.0, a23 = 0.0, a33 = 0.0;
-  double g[3] = {0.0, 0.0, 0.0};
-  const double xe = m.xc[e], ye = m.yc[e], ze = m.zc[e], pe = phi[e];
+  double g[NC][3], pe[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    g[c][0] = g[c][1] = g[c][2] = 0.0;
+    pe[c] = f.phi[c][e];
+  }
+  const double xe = m.xc[e], ye = m.yc[e], ze = m.zc[e];
   for (int k = m.row[e]; k < m.row[e + 1]; k++) {
     const int nb = m.nbr[k];
     const double dr[3] = {m.xc[nb] - xe, m.yc[nb] - ye, m.zc[nb] - ze};
     const double wt = 1.0 / (dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2]);
-    const double dphi = phi[nb] - pe;
-    for (int i = 0; i < 3; i++) g[i] = g[i] + wt * dphi * dr[i];
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const double dphi = f.phi[c][nb] - pe[c];
+      for (int i = 0; i < 3; i++) g[c][i] = g[c][i] + wt * dphi * dr[i];
+    }
     a11 = a11 + wt * dr[0] * dr[0];
     a12 = a12 + wt * dr[0] * dr[1];
     a13 = a13 + wt * dr[0] * dr[2];
@@ -791,12 +832,17 @@ __device__ inline void d_grad(int bx_, MeshDev m, const double *__restrict__ phi
     b11 = di; b22 = di; b33 = di;
     b12 = b13 = b21 = b23 = b31 = b32 = 0.0;
   }
-  grad[3 * e] = b11 * g[0] + b12 * g[1] + b13 * g[2];
-  grad[3 * e + 1] = b21 * g[0] + b22 * g[1] + b23 * g[2];
-  grad[3 * e + 2] = b31 * g[0] + b32 * g[1] + b33 * g[2];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    double *grad = f.grad[c];
+    grad[3 * e] = b11 * g[c][0] + b12 * g[c][1] + b13 * g[c][2];
+    grad[3 * e + 1] = b21 * g[c][0] + b22 * g[c][1] + b23 * g[c][2];
+    grad[3 * e + 2] = b31 * g[c][0] + b32 * g[c][1] + b33 * g[c][2];
+  }
 }
-__global__ void k_grad(MeshDev m, const double *__restrict__ phi, double *__restrict__ grad) {
-  d_grad(blockIdx.x, m, phi, grad);
+template <int NC>
+__global__ void k_grad(MeshDev m, GradArgs<NC> f) {
+  d_grad<NC>(blockIdx.x, m, f);
 }
 
 // ---------------------------------------------------------------------------
@@ -880,74 +926,56 @@ __global__ void k_coef_p(MeshDev m, FieldsDev f) {
   f.b[e] = b;
 }
 
-// calc_coef_p for meshes whose rows all have six entries, six threads per
-// cell as in k_coef_uvw6: entry terms in parallel, then the cell's sums in
-// CSR order.  T = float (the FP32 assembly) computes the coefficients in
-// FP32; the right-hand side, the cell's net inflow (the continuity check),
-// stays FP64 in both.
+// calc_coef_p for meshes whose rows all have six entries, one thread per cell
+// on the faces' fixed geometry, as k_coef_uvw6.  T = float (the FP32 assembly)
+// computes the coefficients in FP32; the right-hand side, the cell's net
+// inflow (the continuity check), stays FP64 in both.
 template <typename T>
-__device__ inline void d_coef_p6(int bx_, MeshDev m, FieldsDev f) {
+__device__ inline void d_coef_p6(int bx_, const MeshDev &m, const FieldsDev &f) {
+  const int e = bx_ * blockDim.x + threadIdx.x;
+  if (e >= m.ne) return;
   const auto G = geo_of<T>(m);
   const T one = static_cast<T>(1), zero = static_cast<T>(0);
-  __shared__ T sd[kFaceThreads];
-  __shared__ double sfl[kFaceThreads];
-  __shared__ int sin_[kFaceThreads];
-  const int lc = threadIdx.x / 6, j = threadIdx.x - 6 * lc;
-  const int e = bx_ * kFaceCells + lc;
-  const bool valid = lc < kFaceCells && e < m.ne;
-  if (valid) {
-    const int k = 6 * e + j;
-    const int nb = m.nbr[k];
+  int nbs[6], fss[6];
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    nbs[k] = m.nbr[6 * e + k];
+    fss[k] = m.fsg[6 * e + k];
+  }
+  const T dce = static_cast<T>(f.dc[e]), rhoe = G.rho[e];
+  T ap = zero, anbk[6];
+  double sumf = 0.0, b;
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    const int nb = nbs[k], fs = fss[k], fg = abs(fs) - 1;
     T d = zero;
-    double fl = 0.0;
     if (nb < m.ne) {
-      const T rp[3] = {G.xc[e], G.yc[e], G.zc[e]};
-      const int fs = m.fsg[k];
-      const T sg = fs >= 0 ? one : -one;
-      const int fg = abs(fs) - 1;
-      const T *a = G.aip + 3 * fg, *rip = G.rip + 3 * fg;
-      const T area = area_of(a);
-      T nrm[3], dr[3];
-      for (int i = 0; i < 3; i++) nrm[i] = sg * a[i] / area;
-      const T rpnb[3] = {G.xc[nb], G.yc[nb], G.zc[nb]};
-      for (int i = 0; i < 3; i++) dr[i] = rpnb[i] - rp[i];
-      const T wt = vec_weight(rip, rp, rpnb);
-      fl = -((fs >= 0 ? 1.0 : -1.0) * f.mip[fg]);
-      const T rhoip = (one - wt) * G.rho[e] + wt * G.rho[nb];
-      d = ((one - wt) * static_cast<T>(f.dc[e]) + wt * static_cast<T>(f.dc[nb])) / dot3(dr, nrm) *
-          rhoip * area;
-      f.anb[k] = static_cast<double>(d);
+      const T *fa = G.fa + 4 * fg;
+      const T area = fa[0], wt = fs >= 0 ? fa[1] : fa[2];
+      sumf = sumf + -((fs >= 0 ? 1.0 : -1.0) * f.mip[fg]);
+      const T rhoip = (one - wt) * rhoe + wt * G.rho[nb];
+      d = ((one - wt) * dce + wt * static_cast<T>(f.dc[nb])) / fa[3] * rhoip * area;
     }
-    sd[threadIdx.x] = d;
-    sfl[threadIdx.x] = fl;
-    sin_[threadIdx.x] = nb < m.ne;
+    anbk[k] = d;
+    ap = ap + d;
   }
-  __syncthreads();
-  if (!valid || j != 0) return;
-  T ap = zero;
-  double sumf = 0.0;
-  for (int q = 0; q < 6; q++) {
-    const int t = threadIdx.x + q;
-    if (sin_[t]) {
-      sumf = sumf + sfl[t];
-    } else {
-      f.anb[6 * e + q] = static_cast<double>(sd[t]);
-    }
-    ap = ap + sd[t];
-  }
-  double b = sumf;
+  b = sumf;
   for (int q = m.bcrow[e]; q < m.bcrow[e + 1]; q++) {
     const int k = m.bcslot[q];
     const T d = zero;  // 'dirichlet' and 'zero_flux' both add nothing
     ap = ap + d;
-    f.anb[k] = static_cast<double>(sd[threadIdx.x + (k - 6 * e)] + d);
+#pragma unroll
+    for (int j = 0; j < 6; j++)
+      if (j == k - 6 * e) anbk[j] = anbk[j] + d;
     b = b - f.mip[m.fsg[k] - 1];
   }
+#pragma unroll
+  for (int k = 0; k < 6; k++) f.anb[6 * e + k] = static_cast<double>(anbk[k]);
   f.ap[e] = static_cast<double>(ap);
   f.b[e] = b;
 }
 template <typename T>
-__global__ void __launch_bounds__(kFaceThreads) k_coef_p6(MeshDev m, FieldsDev f) {
+__global__ void __launch_bounds__(kBlock) k_coef_p6(MeshDev m, FieldsDev f) {
   d_coef_p6<T>(blockIdx.x, m, f);
 }
 
@@ -969,17 +997,10 @@ __device__ inline void d_update_faces(int bx_, MeshDev m, FieldsDev f) {
   if (fg >= m.nf) return;
   const int k = m.own[fg], e = m.fcell[fg], nb = m.nbr[k];
   if (nb >= m.ne) return;
-  const double *a = m.aip + 3 * fg, *rip = m.rip + 3 * fg;
-  const double area = area_of(a);
-  const double nrm[3] = {a[0] / area, a[1] / area, a[2] / area};
-  double rp[3], rpnb[3], dr[3];
-  centre(m, e, rp);
-  centre(m, nb, rpnb);
-  for (int i = 0; i < 3; i++) dr[i] = rpnb[i] - rp[i];
-  const double wt = vec_weight(rip, rp, rpnb);
+  const double area = m.fa[4 * fg], wt = m.fa[4 * fg + 1];
   const double dip = (1.0 - wt) * f.dc[e] + wt * f.dc[nb];
   const double rhoip = (m.rho[e] + m.rho[nb]) / 2.0;
-  const double dmip = rhoip * area * dip * (f.phic[nb] - f.phic[e]) / dot3(dr, nrm);
+  const double dmip = rhoip * area * dip * (f.phic[nb] - f.phic[e]) / m.fa[4 * fg + 3];
   f.mip[fg] = f.mip[fg] - dmip;
 }
 __global__ void k_update_faces(MeshDev m, FieldsDev f) {
@@ -2090,7 +2111,7 @@ __global__ void gb_bc_energy(GroupMap g, const BSlot *__restrict__ S) {
   d_bc_energy(bx, x.md, x.en);
 }
 template <typename T>
-__global__ void __launch_bounds__(kFaceThreads)
+__global__ void __launch_bounds__(kBlock)
 gb_coef_uvw6(GroupMap g, const BSlot *__restrict__ S) {
   BSLOT;
   d_coef_uvw6<T>(bx, x.md, x.fd, x.dt, x.alpha_u);
@@ -2144,19 +2165,25 @@ __global__ void gb_log_gs(GroupMap g, const BSlot *__restrict__ S, Names nm) {
   d_log_gs(bx, x.gctl, 3, nm, x.log, x.nlog);
 }
 // which: 0 u -> gu, 1 v -> gv, 2 w -> gw, 3 phic -> gpc
-__global__ void gb_grad(GroupMap g, const BSlot *__restrict__ S, int which) {
+// the gradient of u alone (the tuner's launch), of u, v and w, of phic
+__global__ void gb_grad_u(GroupMap g, const BSlot *__restrict__ S) {
   BSLOT;
-  const FieldsDev &f = x.fd;
-  const double *phi = which == 0 ? f.u : which == 1 ? f.v : which == 2 ? f.w : f.phic;
-  double *gr = which == 0 ? f.gu : which == 1 ? f.gv : which == 2 ? f.gw : f.gpc;
-  d_grad(bx, x.md, phi, gr);
+  d_grad<1>(bx, x.md, GradArgs<1>{{x.fd.u}, {x.fd.gu}});
+}
+__global__ void gb_grad_uvw(GroupMap g, const BSlot *__restrict__ S) {
+  BSLOT;
+  d_grad<3>(bx, x.md, GradArgs<3>{{x.fd.u, x.fd.v, x.fd.w}, {x.fd.gu, x.fd.gv, x.fd.gw}});
+}
+__global__ void gb_grad_pc(GroupMap g, const BSlot *__restrict__ S) {
+  BSLOT;
+  d_grad<1>(bx, x.md, GradArgs<1>{{x.fd.phic}, {x.fd.gpc}});
 }
 __global__ void gb_mip(GroupMap g, const BSlot *__restrict__ S) {
   BSLOT;
   d_mip(bx, x.md, x.fd, 1, x.dt);
 }
 template <typename T>
-__global__ void __launch_bounds__(kFaceThreads) gb_coef_p6(GroupMap g, const BSlot *__restrict__ S) {
+__global__ void __launch_bounds__(kBlock) gb_coef_p6(GroupMap g, const BSlot *__restrict__ S) {
   BSLOT;
   d_coef_p6<T>(bx, x.md, x.fd);
 }
@@ -3362,6 +3389,14 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
   C->md = MeshDev{ne, nf, nbf, L, d_row, d_nbr, d_fsg, d_own, d_fcell, d_bcrow, d_bcslot,
                   d_hcell, d_hslot, d_hkind, d_xc, d_yc, d_zc, d_vol, d_aip, d_rip, d_rho, d_mu,
                   d_cp, d_tc};
+  {
+    double *fa, *fd;
+    CALL(dalloc(C, &fa, 4 * int64_t{nf}));
+    CALL(dalloc(C, &fd, 5 * int64_t{nf}));
+    hipLaunchKernelGGL(k_face_geo<double>, dim3(nblocks(nf)), dim3(kBlock), 0, C->st, C->md, fa, fd);
+    HIPCHK(hipGetLastError());
+    C->md.fa = fa, C->md.fd = fd;
+  }
   trace("ctx_create: mesh uploaded");
   // --- fields ---
   const int64_t sz[CFDL_NFIELDS] = {n, n, n, n, n, n, n, 3 * int64_t{n}, 3 * int64_t{n},
@@ -3872,6 +3907,13 @@ int cfdl_set_assembly_precision(cfdl_ctx *c, int bits) {
     HIPCHK(hipGetLastError());
     c->md.xc32 = p[0], c->md.yc32 = p[1], c->md.zc32 = p[2], c->md.vol32 = p[3];
     c->md.aip32 = p[4], c->md.rip32 = p[5], c->md.rho32 = p[6], c->md.mu32 = p[7];
+    float *fa, *fd;
+    CALL(dalloc(c, &fa, 4 * int64_t{c->nf}));
+    CALL(dalloc(c, &fd, 5 * int64_t{c->nf}));
+    hipLaunchKernelGGL(k_face_geo<float>, dim3(nblocks(c->nf)), dim3(kBlock), 0, c->st, c->md, fa,
+                       fd);
+    HIPCHK(hipGetLastError());
+    c->md.fa32 = fa, c->md.fd32 = fd;
   }
   c->asm32 = bits == 32;
   return CFDL_OK;
@@ -4016,8 +4058,8 @@ int cfdl_calc_coef_energy(cfdl_ctx *c) {
 // solve_gs('e') on the enthalpy (SOR factor 1), temperature from enthalpy
 int cfdl_solve_energy(cfdl_ctx *c) {
   CALL(check_ctx(c));
-  hipLaunchKernelGGL(k_grad, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->st, c->md, c->en.t, c->en.gt);
-  hipLaunchKernelGGL(k_grad, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->st, c->md, c->en.h, c->en.gh);
+  hipLaunchKernelGGL(k_grad<2>, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->st, c->md,
+                     (GradArgs<2>{{c->en.t, c->en.h}, {c->en.gt, c->en.gh}}));
   CALL(cfdl_calc_coef_energy(c));
   double *phi = c->en.h;
   const double *b = c->fd.b;
@@ -4038,11 +4080,11 @@ int cfdl_calc_coef_uvw(cfdl_ctx *c) {
     return CFDL_ESTATE;
   }
   if (c->mhex && c->asm32)
-    hipLaunchKernelGGL(k_coef_uvw6<float>, dim3((c->ne + kFaceCells - 1) / kFaceCells),
-                       dim3(kFaceThreads), 0, c->st, c->md, c->fd, c->dt, c->alpha_u);
+    hipLaunchKernelGGL(k_coef_uvw6<float>, dim3(nblocks(c->ne)),
+                       dim3(kBlock), 0, c->st, c->md, c->fd, c->dt, c->alpha_u);
   else if (c->mhex)
-    hipLaunchKernelGGL(k_coef_uvw6<double>, dim3((c->ne + kFaceCells - 1) / kFaceCells),
-                       dim3(kFaceThreads), 0, c->st, c->md, c->fd, c->dt, c->alpha_u);
+    hipLaunchKernelGGL(k_coef_uvw6<double>, dim3(nblocks(c->ne)),
+                       dim3(kBlock), 0, c->st, c->md, c->fd, c->dt, c->alpha_u);
   else
     hipLaunchKernelGGL(k_coef_uvw, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->st, c->md, c->fd,
                        c->dt, c->alpha_u);
@@ -4077,7 +4119,8 @@ int cfdl_calc_grad(cfdl_ctx *c, int src, int dst) {
     set_error("cfdl_calc_grad: src must be an element field, dst a gradient field");
     return CFDL_EINVAL;
   }
-  hipLaunchKernelGGL(k_grad, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->st, c->md, p, g);
+  hipLaunchKernelGGL(k_grad<1>, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->st, c->md,
+                     (GradArgs<1>{{p}, {g}}));
   HIPCHK(hipGetLastError());
   return CFDL_OK;
 }
@@ -4093,11 +4136,11 @@ int cfdl_calc_mip(cfdl_ctx *c, int rhie_chow) {
 int cfdl_calc_coef_p(cfdl_ctx *c) {
   CALL(check_ctx(c));
   if (c->mhex && c->asm32)
-    hipLaunchKernelGGL(k_coef_p6<float>, dim3((c->ne + kFaceCells - 1) / kFaceCells),
-                       dim3(kFaceThreads), 0, c->st, c->md, c->fd);
+    hipLaunchKernelGGL(k_coef_p6<float>, dim3(nblocks(c->ne)),
+                       dim3(kBlock), 0, c->st, c->md, c->fd);
   else if (c->mhex)
-    hipLaunchKernelGGL(k_coef_p6<double>, dim3((c->ne + kFaceCells - 1) / kFaceCells),
-                       dim3(kFaceThreads), 0, c->st, c->md, c->fd);
+    hipLaunchKernelGGL(k_coef_p6<double>, dim3(nblocks(c->ne)),
+                       dim3(kBlock), 0, c->st, c->md, c->fd);
   else
     hipLaunchKernelGGL(k_coef_p, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->st, c->md, c->fd);
   HIPCHK(hipGetLastError());
@@ -4169,9 +4212,10 @@ int cfdl_solve_uvwp(cfdl_ctx *c) {
   CALL(check_ctx(c));
   CALL(cfdl_calc_coef_uvw(c));
   CALL(cfdl_solve_gs_uvw(c));
-  CALL(cfdl_calc_grad(c, CFDL_U, CFDL_GU));
-  CALL(cfdl_calc_grad(c, CFDL_V, CFDL_GV));
-  CALL(cfdl_calc_grad(c, CFDL_W, CFDL_GW));
+  const FieldsDev &f = c->fd;
+  hipLaunchKernelGGL(k_grad<3>, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->st, c->md,
+                     (GradArgs<3>{{f.u, f.v, f.w}, {f.gu, f.gv, f.gw}}));
+  HIPCHK(hipGetLastError());
   CALL(cfdl_calc_mip(c, 1));
   CALL(cfdl_calc_coef_p(c));
   CALL(cfdl_set_a_0(c, CFDL_PHIC));
@@ -4596,11 +4640,11 @@ int seg_prefix(cfdl_batch *b, int blk) {
   if (nb > 0) hipLaunchKernelGGL(gb_outlet_flux, dim3(nb), dim3(kOutThreads), 0, st, L.g, S);
   nb = L.map([&](cfdl_ctx *c) { return nbk(c->nbf, blk); });
   if (nb > 0) hipLaunchKernelGGL(gb_bc_energy, dim3(nb), dim3(blk), 0, st, L.g, S);
-  nb = L.map([&](cfdl_ctx *c) { return (c->ne + kFaceCells - 1) / kFaceCells; });
+  nb = L.map([&](cfdl_ctx *c) { return nblocks(c->ne); });
   if (b->asm32)
-    hipLaunchKernelGGL(gb_coef_uvw6<float>, dim3(nb), dim3(kFaceThreads), 0, st, L.g, S);
+    hipLaunchKernelGGL(gb_coef_uvw6<float>, dim3(nb), dim3(kBlock), 0, st, L.g, S);
   else
-    hipLaunchKernelGGL(gb_coef_uvw6<double>, dim3(nb), dim3(kFaceThreads), 0, st, L.g, S);
+    hipLaunchKernelGGL(gb_coef_uvw6<double>, dim3(nb), dim3(kBlock), 0, st, L.g, S);
   nb = L.map([&](cfdl_ctx *c) { return nbk(int64_t{c->ne} + c->nbf, blk); });
   hipLaunchKernelGGL(gb_tile_gather, dim3(nb), dim3(blk), 0, st, L.g, S);
   const int np = L.map([&](cfdl_ctx *c) { return c->nblk_g; });
@@ -4646,7 +4690,7 @@ int seg_gs(cfdl_batch *b, int blk, int slot) {
 // each; the launches recompute the same values) between events; the
 // fastest is read at the end of the run and used for every element-wise
 // launch of the batch from then on.
-int batch_grad_u(cfdl_batch *b, int blk) {
+int batch_tune_launch(cfdl_batch *b) {
   BatchLaunch L(b);
   const BSlot *S = b->d_slots;
   if (b->block == 0 && b->tuned == 0 && !b->tuning) {
@@ -4654,13 +4698,11 @@ int batch_grad_u(cfdl_batch *b, int blk) {
       const int nb = L.map([&](cfdl_ctx *c) { return nbk(c->ne, kTuneBlocks[j]); });
       HIPCHK(hipEventRecord(b->tev[j], b->st));
       for (int r = 0; r < 3; r++)
-        hipLaunchKernelGGL(gb_grad, dim3(nb), dim3(kTuneBlocks[j]), 0, b->st, L.g, S, 0);
+        hipLaunchKernelGGL(gb_grad_u, dim3(nb), dim3(kTuneBlocks[j]), 0, b->st, L.g, S);
     }
     HIPCHK(hipEventRecord(b->tev[5], b->st));
     b->tuning = true;
   }
-  const int nb = L.map([&](cfdl_ctx *c) { return nbk(c->ne, blk); });
-  hipLaunchKernelGGL(gb_grad, dim3(nb), dim3(blk), 0, b->st, L.g, S, 0);
   HIPCHK(hipGetLastError());
   return CFDL_OK;
 }
@@ -4695,22 +4737,16 @@ int seg_middle(cfdl_batch *b, int blk, bool tune) {
   nb = L.map([&](cfdl_ctx *) { return 1; });
   hipLaunchKernelGGL(gb_log_gs, dim3(nb), dim3(64), 0, st, L.g, S, nm);
   HIPCHK(hipGetLastError());
-  if (tune) {
-    CALL(batch_grad_u(b, blk));
-  } else {
-    nb = L.map([&](cfdl_ctx *c) { return nbk(c->ne, blk); });
-    hipLaunchKernelGGL(gb_grad, dim3(nb), dim3(blk), 0, st, L.g, S, 0);
-  }
+  if (tune) CALL(batch_tune_launch(b));
   nb = L.map([&](cfdl_ctx *c) { return nbk(c->ne, blk); });
-  hipLaunchKernelGGL(gb_grad, dim3(nb), dim3(blk), 0, st, L.g, S, 1);
-  hipLaunchKernelGGL(gb_grad, dim3(nb), dim3(blk), 0, st, L.g, S, 2);
+  hipLaunchKernelGGL(gb_grad_uvw, dim3(nb), dim3(blk), 0, st, L.g, S);
   nb = L.map([&](cfdl_ctx *c) { return nbk(c->nf, blk); });
   hipLaunchKernelGGL(gb_mip, dim3(nb), dim3(blk), 0, st, L.g, S);
-  nb = L.map([&](cfdl_ctx *c) { return (c->ne + kFaceCells - 1) / kFaceCells; });
+  nb = L.map([&](cfdl_ctx *c) { return nblocks(c->ne); });
   if (b->asm32)
-    hipLaunchKernelGGL(gb_coef_p6<float>, dim3(nb), dim3(kFaceThreads), 0, st, L.g, S);
+    hipLaunchKernelGGL(gb_coef_p6<float>, dim3(nb), dim3(kBlock), 0, st, L.g, S);
   else
-    hipLaunchKernelGGL(gb_coef_p6<double>, dim3(nb), dim3(kFaceThreads), 0, st, L.g, S);
+    hipLaunchKernelGGL(gb_coef_p6<double>, dim3(nb), dim3(kBlock), 0, st, L.g, S);
   nb = L.map([&](cfdl_ctx *c) { return nbk(int64_t{c->ne} + c->nbf, blk); });
   hipLaunchKernelGGL(gb_zero_phic, dim3(nb), dim3(blk), 0, st, L.g, S);
   HIPCHK(hipGetLastError());
@@ -4731,7 +4767,7 @@ int seg_suffix(cfdl_batch *b, int blk) {
   nb = L.map([&](cfdl_ctx *c) { return nbk(c->nbf, blk); });
   if (nb > 0) hipLaunchKernelGGL(gb_halo_from_owner, dim3(nb), dim3(blk), 0, st, L.g, S);
   nb = L.map([&](cfdl_ctx *c) { return nbk(c->ne, blk); });
-  hipLaunchKernelGGL(gb_grad, dim3(nb), dim3(blk), 0, st, L.g, S, 3);
+  hipLaunchKernelGGL(gb_grad_pc, dim3(nb), dim3(blk), 0, st, L.g, S);
   hipLaunchKernelGGL(gb_update_cells, dim3(nb), dim3(blk), 0, st, L.g, S);
   nb = L.map([&](cfdl_ctx *c) { return nbk(c->nf, blk); });
   hipLaunchKernelGGL(gb_update_faces, dim3(nb), dim3(blk), 0, st, L.g, S);
