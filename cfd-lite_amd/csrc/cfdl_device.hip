@@ -415,7 +415,7 @@ k_outlet_flux(MeshDev m, double *mip, const int *fin, int nin, const int *fout, 
 // the Rhie-Chow / SIMPLEC coefficients (:276-284).
 // ---------------------------------------------------------------------------
 __global__ void k_coef_uvw(MeshDev m, FieldsDev f, double dt, double alpha_u) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int e = xcd_block() * blockDim.x + threadIdx.x;
   if (e >= m.ne) return;
   double rp[3];
   centre(m, e, rp);
@@ -673,7 +673,7 @@ __device__ inline void d_coef_uvw6(int bx_, const MeshDev &m, const FieldsDev &f
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
 k_coef_uvw6(MeshDev m, FieldsDev f, double dt_, double alpha_u_) {
-  d_coef_uvw6<T>(blockIdx.x, m, f, dt_, alpha_u_);
+  d_coef_uvw6<T>(xcd_block(), m, f, dt_, alpha_u_);
 }
 
 // ---------------------------------------------------------------------------
@@ -714,7 +714,7 @@ __global__ void k_bc_energy(MeshDev m, EnergyDev en) {
 // gradients of t and h, then the Dirichlet boundary faces of the cell in
 // halo order (f = 0, d = tc*A/ds/cp)
 __global__ void k_coef_energy(MeshDev m, FieldsDev f, EnergyDev en, double dt) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int e = xcd_block() * blockDim.x + threadIdx.x;
   if (e >= m.ne) return;
   double rp[3];
   centre(m, e, rp);
@@ -842,7 +842,7 @@ __device__ inline void d_grad(int bx_, const MeshDev &m, const GradArgs<NC> &f) 
 }
 template <int NC>
 __global__ void k_grad(MeshDev m, GradArgs<NC> f) {
-  d_grad<NC>(blockIdx.x, m, f);
+  d_grad<NC>(xcd_block(), m, f);
 }
 
 // ---------------------------------------------------------------------------
@@ -879,7 +879,7 @@ __device__ inline void d_mip(int bx_, MeshDev m, FieldsDev f, int rc, double dt)
   f.mip[fg] = mip;
 }
 __global__ void k_mip(MeshDev m, FieldsDev f, int rc, double dt) {
-  d_mip(blockIdx.x, m, f, rc, dt);
+  d_mip(xcd_block(), m, f, rc, dt);
 }
 
 // ---------------------------------------------------------------------------
@@ -887,7 +887,7 @@ __global__ void k_mip(MeshDev m, FieldsDev f, int rc, double dt) {
 // net inflow, one thread per cell; boundary loop (:344-366) in halo order.
 // ---------------------------------------------------------------------------
 __global__ void k_coef_p(MeshDev m, FieldsDev f) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int e = xcd_block() * blockDim.x + threadIdx.x;
   if (e >= m.ne) return;
   double rp[3];
   centre(m, e, rp);
@@ -976,7 +976,7 @@ __device__ inline void d_coef_p6(int bx_, const MeshDev &m, const FieldsDev &f) 
 }
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_coef_p6(MeshDev m, FieldsDev f) {
-  d_coef_p6<T>(blockIdx.x, m, f);
+  d_coef_p6<T>(xcd_block(), m, f);
 }
 
 // update_uvwp cell part, mod_uvwp.f90:383-392 (no velocity correction)
@@ -988,7 +988,7 @@ __device__ inline void d_update_cells(int bx_, int ne, FieldsDev f, double alpha
   for (int i = 0; i < 3; i++) f.gp[3 * e + i] = f.gp[3 * e + i] + alpha_p * f.gpc[3 * e + i];
 }
 __global__ void k_update_cells(int ne, FieldsDev f, double alpha_p) {
-  d_update_cells(blockIdx.x, ne, f, alpha_p);
+  d_update_cells(xcd_block(), ne, f, alpha_p);
 }
 
 // update_uvwp face part, mod_uvwp.f90:394-415 (arithmetic-mean rho)
@@ -1004,7 +1004,7 @@ __device__ inline void d_update_faces(int bx_, MeshDev m, FieldsDev f) {
   f.mip[fg] = f.mip[fg] - dmip;
 }
 __global__ void k_update_faces(MeshDev m, FieldsDev f) {
-  d_update_faces(blockIdx.x, m, f);
+  d_update_faces(xcd_block(), m, f);
 }
 
 // adjust_pc, mod_uvwp.f90:136-158 with pref = phic(1) (:129)
@@ -1121,7 +1121,7 @@ __device__ inline void d_gs_level(int bx_, SysDesc s, const int *__restrict__ ce
 template <int NC>
 __global__ void k_gs_level(SysDesc s, const int *__restrict__ cells, int base, int n, double sor,
                            int reps, const int *__restrict__ active) {
-  d_gs_level<NC>(blockIdx.x, s, cells, base, n, sor, reps, active);
+  d_gs_level<NC>(xcd_block(), s, cells, base, n, sor, reps, active);
 }
 
 // One colour of the pc system in the colour numbering, FP64 (T = double) or
@@ -1138,7 +1138,7 @@ struct ColRanges {
 template <typename T, bool HEX>
 __global__ void k_pc_colour(ColSys<T> s, ColRanges cr, T sor, int reps,
                             const int *__restrict__ active) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = xcd_block() * blockDim.x + threadIdx.x;
   if (t >= cr.off[cr.n] || !active[0]) return;
   int y = 0;
   while (t >= cr.off[y + 1]) y++;
@@ -1236,7 +1236,6 @@ k_gs_tiles(SysDesc s, const int *__restrict__ bseg, const int *__restrict__ seg,
 // their values) plus the issue of its loads, which NW wavefronts share.  The
 // segment count is at most 63 (host).
 constexpr int kLdsThreads = 64;  // one wavefront: the pipelined walk's width
-constexpr int kXcds = 8;         // XCDs of an MI355X; each has its own L2
 // The pipelined walk's values start at LDS byte address 0: the kernel has
 // no static LDS, so its dynamic block starts there.
 
@@ -1815,7 +1814,8 @@ __device__ inline void d_resid_partial(int bx_, const SysDesc &s, int chunk, int
 template <int NC>
 __global__ void __launch_bounds__(kBlock)
 k_resid_partial(SysDesc s, int chunk, int nblk, int absmax, double *part, float *rout) {
-  d_resid_partial<NC>(blockIdx.x, s, chunk, nblk, absmax, part, rout);
+  // (three right-hand sides measured slower by XCD ranges: 65 us against 58 at 128^3)
+  d_resid_partial<NC>(NC == 1 ? xcd_block() : blockIdx.x, s, chunk, nblk, absmax, part, rout);
 }
 
 __device__ inline void d_resid_final(int bx_, const double *part, int nblk, double *red) {
@@ -1984,7 +1984,7 @@ __global__ void k_pc_assemble(int ne, const int *l2g_cell, const int *rowp, cons
                               const double *ap, const double *b, const double *anb,
                               const double *phi, double *ap_p, double *b_p, double *anb_p,
                               double *phic_p, double *rap_p) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  const int c = xcd_block() * blockDim.x + threadIdx.x;
   if (c >= ne) return;
   const int g = l2g_cell[c];
   const double a = ap[g];
@@ -2049,7 +2049,7 @@ __device__ inline void d_tile_gather(int bx_, TileMap t) {
   }
 }
 __global__ void k_tile_gather(TileMap t) {
-  d_tile_gather(blockIdx.x, t);
+  d_tile_gather(xcd_block(), t);
 }
 __device__ inline void d_tile_scatter(int bx_, TileMap t) {
   const int i = bx_ * blockDim.x + threadIdx.x;
@@ -2063,7 +2063,7 @@ __device__ inline void d_tile_scatter(int bx_, TileMap t) {
     if (y < t.ny) t.phi[y][g] = v[y];
 }
 __global__ void k_tile_scatter(TileMap t) {
-  d_tile_scatter(blockIdx.x, t);
+  d_tile_scatter(xcd_block(), t);
 }
 
 

@@ -371,31 +371,31 @@ k_cg_init(Red R, const int *__restrict__ row, const int *__restrict__ nbr,
           const double *__restrict__ anb, const double *__restrict__ b,
           const double *__restrict__ phi, double *__restrict__ r, T *__restrict__ rt, CgCtl *c,
           double *part, int nit) {
-  d_cg_init<T>(blockIdx.x, R, row, nbr, pos, ap, anb, b, phi, r, rt, c, part, nit);
+  d_cg_init<T>(xcd_block(), R, row, nbr, pos, ap, anb, b, phi, r, rt, c, part, nit);
 }
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
 k_cg_rz(Red R, const double *__restrict__ r, const T *__restrict__ z, const int *__restrict__ pos,
         CgCtl *c, double *part) {
-  d_cg_rz<T>(blockIdx.x, R, r, z, pos, c, part);
+  d_cg_rz<T>(xcd_block(), R, r, z, pos, c, part);
 }
 template <typename T>
 __global__ void k_cg_p(int n, const T *__restrict__ z, const int *__restrict__ pos,
                        double *__restrict__ p, const CgCtl *c) {
-  d_cg_p<T>(blockIdx.x * blockDim.x + threadIdx.x, n, z, pos, p, c);
+  d_cg_p<T>(xcd_block() * blockDim.x + threadIdx.x, n, z, pos, p, c);
 }
 __global__ void __launch_bounds__(kRedThreads)
 k_cg_spmv(Red R, const int *__restrict__ row, const int *__restrict__ nbr,
           const double *__restrict__ ap, const double *__restrict__ anb,
           const double *__restrict__ p, double *__restrict__ q, CgCtl *c, double *part) {
-  d_cg_spmv(blockIdx.x, R, row, nbr, ap, anb, p, q, c, part);
+  d_cg_spmv(xcd_block(), R, row, nbr, ap, anb, p, q, c, part);
 }
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
 k_cg_update(Red R, double *__restrict__ phi, const double *__restrict__ p,
             const double *__restrict__ q, const int *__restrict__ pos, double *__restrict__ r,
             T *__restrict__ rt, CgCtl *c, double *part) {
-  d_cg_update<T>(blockIdx.x, R, phi, p, q, pos, r, rt, c, part);
+  d_cg_update<T>(xcd_block(), R, phi, p, q, pos, r, rt, c, part);
 }
 __global__ void k_cg_log(const CgCtl *c, LogLine *log, int *nlog, LogLine tmpl) {
   if (threadIdx.x == 0 && blockIdx.x == 0) d_cg_log(c, log, nlog, tmpl);
@@ -819,7 +819,7 @@ __device__ inline void d_mg_coarse(const Lev<T> *__restrict__ lv, int lc, int nl
 template <typename T>
 __global__ void k_mg_copy0(Lev<T> L, const int *__restrict__ pos, const int *__restrict__ row,
                            const double *__restrict__ ap, const double *__restrict__ anb) {
-  d_mg_copy0<T>(blockIdx.x * blockDim.x + threadIdx.x, L, pos, row, ap, anb);
+  d_mg_copy0<T>(xcd_block() * blockDim.x + threadIdx.x, L, pos, row, ap, anb);
 }
 template <typename T>
 __global__ void k_mg_galerkin(Lev<T> F, Lev<T> C) {
@@ -827,19 +827,19 @@ __global__ void k_mg_galerkin(Lev<T> F, Lev<T> C) {
 }
 template <typename T>
 __global__ void __launch_bounds__(1024) k_mg_sweep(Lev<T> L, int q, int mode, const CgCtl *ctl) {
-  d_mg_sweep<T>(blockIdx.x, L, q, mode, ctl);
+  d_mg_sweep<T>(xcd_block(), L, q, mode, ctl);
 }
 template <typename T>
 __global__ void k_mg_residual(Lev<T> F, int n, const CgCtl *ctl) {
-  d_mg_residual<T>(blockIdx.x * blockDim.x + threadIdx.x, n, F, ctl);
+  d_mg_residual<T>(xcd_block() * blockDim.x + threadIdx.x, n, F, ctl);
 }
 template <typename T>
 __global__ void k_mg_restrict(Lev<T> F, int n, T *bC, const CgCtl *ctl) {
-  d_mg_restrict<T>(blockIdx.x * blockDim.x + threadIdx.x, n, F, bC, ctl);
+  d_mg_restrict<T>(xcd_block() * blockDim.x + threadIdx.x, n, F, bC, ctl);
 }
 template <typename T>
 __global__ void k_mg_prolong(Lev<T> F, int n, const T *__restrict__ xc, const CgCtl *ctl) {
-  d_mg_prolong<T>(blockIdx.x * blockDim.x + threadIdx.x, n, F, xc, ctl);
+  d_mg_prolong<T>(xcd_block() * blockDim.x + threadIdx.x, n, F, xc, ctl);
 }
 template <typename T>
 __global__ void __launch_bounds__(kCoarseThreads)
@@ -877,7 +877,7 @@ __global__ void g_mg_copy0(GroupMap g, const MgSlot<T> *__restrict__ S) {
 template <typename T>
 __global__ void g_mg_galerkin(GroupMap g, const MgSlot<T> *__restrict__ S, int l) {
   int bx;
-  const MgSlot<T> &x = S[group_slot(g, bx)];
+  const MgSlot<T> &x = S[group_slot(g, bx, true)];
   const Lev<T> F = x.lv[l], C = x.lv[l + 1];
   d_mg_galerkin<T>(bx * blockDim.x + threadIdx.x, F, C);
 }
