@@ -2335,6 +2335,9 @@ struct cfdl_ctx {
   double *part = nullptr, *red = nullptr, *scal = nullptr;
   int nblk_g = 1, chunk_g = 1, nblk_p = 1, chunk_p = 1;
   int *host_flags = nullptr;  // pinned
+  // pinned buffers of copy_out (two of kStageBytes, from the first large copy)
+  char *stage = nullptr;
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
   LogLine *dlog = nullptr;
   int *dlog_n = nullptr;
   std::vector<LogLine> hlog;
@@ -3727,6 +3730,9 @@ void cfdl_ctx_destroy(cfdl_ctx *c) {
   (void)hipStreamSynchronize(c->st);
   for (auto &m : c->mg) cfdl::mgcg_destroy(m);
   if (c->host_flags) (void)hipHostFree(c->host_flags);
+  if (c->stage) (void)hipHostFree(c->stage);
+  for (auto &e : c->stage_ev)
+    if (e) (void)hipEventDestroy(e);
   for (auto &x : c->samples) {
     (void)hipEventDestroy(x.a);
     (void)hipEventDestroy(x.b);
@@ -3969,6 +3975,46 @@ int cfdl_set_field(cfdl_ctx *c, int field, const double *src, int64_t n) {
   return CFDL_OK;
 }
 
+// Device memory to the caller's array, complete on return.  Large copies go
+// through two pinned buffers, one filled while the CPU empties the other: a
+// direct copy to pageable memory pins its pages first, 17.8 GB/s against 25.8
+// this way (12.6 MB), 8.5 against 10 for the new arrays of UVWP.get, whose
+// pages are also faulted in.  Below kStageMin the direct copy is as fast.
+constexpr size_t kStageBytes = 2 << 20, kStageMin = 512 << 10;
+static int copy_out(cfdl_ctx *c, void *dst, const void *src, size_t bytes) {
+  if (bytes >= kStageMin && !c->stage) {
+    void *p = nullptr;
+    if (hipHostMalloc(&p, 2 * kStageBytes, hipHostMallocDefault) == hipSuccess) {
+      c->stage = static_cast<char *>(p);
+      for (auto &e : c->stage_ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    } else {
+      (void)hipGetLastError();
+    }
+  }
+  if (bytes < kStageMin || !c->stage || !c->stage_ev[1]) {
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    return CFDL_OK;
+  }
+  const size_t n = (bytes + kStageBytes - 1) / kStageBytes;
+  auto part = [&](size_t i) { return std::min(kStageBytes, bytes - i * kStageBytes); };
+  auto fill = [&](size_t i) -> int {
+    HIPCHK(hipMemcpyAsync(c->stage + (i & 1) * kStageBytes,
+                          static_cast<const char *>(src) + i * kStageBytes, part(i),
+                          hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipEventRecord(c->stage_ev[i & 1], c->st));
+    return CFDL_OK;
+  };
+  for (size_t i = 0; i < n && i < 2; i++) CALL(fill(i));
+  for (size_t i = 0; i < n; i++) {
+    HIPCHK(hipEventSynchronize(c->stage_ev[i & 1]));
+    std::memcpy(static_cast<char *>(dst) + i * kStageBytes, c->stage + (i & 1) * kStageBytes,
+                part(i));
+    if (i + 2 < n) CALL(fill(i + 2));
+  }
+  return CFDL_OK;
+}
+
 int cfdl_get_field(cfdl_ctx *c, int field, double *dst, int64_t n) {
   CALL(check_ctx(c));
   double *p = field_ptr(c, field);
@@ -3976,9 +4022,7 @@ int cfdl_get_field(cfdl_ctx *c, int field, double *dst, int64_t n) {
     set_error("cfdl_get_field: bad field id or size");
     return CFDL_EINVAL;
   }
-  HIPCHK(hipMemcpyAsync(dst, p, 8 * n, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
-  return CFDL_OK;
+  return copy_out(c, dst, p, 8 * static_cast<size_t>(n));
 }
 
 int cfdl_synchronize(cfdl_ctx *c) {
