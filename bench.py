@@ -12,7 +12,7 @@ are a prefix of the run (residual_target_met false); the "converge" block
 holds runs to the 1e-6 scaled residual.
 
 Prints one JSON line.  value = 2,097,152 * K / seconds for K timed steps.
-roofline: the pressure-correction Gauss-Seidel sweep kernel k_gs_tiles_lds (the dominant
+roofline: the pressure-correction Gauss-Seidel sweep kernel k_gs_flow (the dominant
 kernel), 108 algorithmic bytes per cell update (FP64 CSR sweep: b, ap, 6
 anb, 6 neighbour indices, own phi read and write) times the cells of one
 launch, over the mean launch duration: HIP events on the context stream
@@ -144,13 +144,12 @@ def run_to_convergence(eq, ne, tstep_every, max_outer, tol, check_every=10):
     return k, time.perf_counter() - t, worst
 
 
-# HBM KiB per launch of the pc sweep kernel on the 128^3 cavity, default
-# schedule, from rocprofv3 counter runs (profiles/k_gs_tiles_lds_traffic_
-# cavity128_fp64.md): mean FETCH_SIZE 6246.0 KiB x 1.99975 (the factor a copy
-# of known size calibrates) + mean WRITE_SIZE 463.2 KiB x 1.0 over the 7400
-# launches of one outer iteration.  About half the fetch is the prefetch of
-# the next launch's batches, which that launch then fetches again.
-TRAFFIC_KIB_128 = 12953.6
+# HBM KiB per launch of the pc sweep kernel (four sweeps) on the 128^3 cavity,
+# default schedule, from rocprofv3 counter runs (profiles/k_gs_flow_
+# cavity128_fp64.md): mean FETCH_SIZE 504522.5 KiB x 1.99975 (the factor a copy
+# of known size calibrates) + mean WRITE_SIZE 68853.3 KiB x 1.0 over the 50
+# launches of one outer iteration.
+TRAFFIC_KIB_128 = 1077772.1
 
 # host <-> device traffic of one drop-in solve_uvwp call
 # (cfd-lite_amd/fortran/dropin/mod_uvwp.f90: put_state, get_state, get_work)
@@ -613,14 +612,14 @@ def main():
     traffic_kib = args.traffic_kib
     schedule_env = any(os.environ.get(k) for k in ("CFDL_TILE", "CFDL_TILE_SPAN", "CFDL_GS_MODE",
                                                   "CFDL_TILE_LDS", "CFDL_TILE_PIPE", "CFDL_TILE_WAVES",
-                                                  "CFDL_TILE_PREFETCH"))
+                                                  "CFDL_TILE_PREFETCH", "CFDL_FLOW"))
     if traffic_kib is None and args.n == 128 and not schedule_env:
         traffic_kib = TRAFFIC_KIB_128
     traffic = None if traffic_kib is None else round(traffic_kib * 1024.0)
     roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
                 "algorithmic_bytes_per_launch": round(BYTES_PER_CELL_SWEEP * cells),
-                "kernel": "k_gs_tiles_lds<true, true, 1, 4> (pressure-correction Gauss-Seidel, space-time tiles in LDS)",
+                "kernel": "k_gs_flow<1> (pressure-correction Gauss-Seidel, four sweeps of space-time tiles in LDS)",
                 "launch_ms": round(kernel_ms, 5), "cells_per_launch": round(cells, 1),
                 "sampled_launches": int(st["sampled_launches"])}
     hbm_whole = ne * iteration_bytes(log[-4 * args.steps:], "reference") / secs / (HBM_PEAK_GBS * 1e9)

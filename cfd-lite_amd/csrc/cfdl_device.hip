@@ -149,6 +149,7 @@ struct FieldsDev {
 // state of a solve_gs call (up to 3 right-hand sides sharing ap/anb)
 struct GsCtl {
   int it[3], active[3];
+  int flow_err;  // a wait of k_gs_flow ran out of time
   double res_i[3], res_f[3], res_max[3], target[3];
 };
 
@@ -1317,6 +1318,183 @@ __device__ void touch_batch(const TileSys<NC> &s, const int4 *__restrict__ bdesc
   for (int k = 0; k < kTouch; k++) asm volatile("" ::"v"(v[k]));
 }
 
+// The pipelined level walk of one batch by wavefront 0, on the LDS layout its
+// kernel has filled (o_ar: byte offset of the (ap, 1/ap) records; sg: segment
+// bound of lane q relative to the first cell).  reload puts the batch's
+// original values back into LDS.
+template <int NC, typename Reload>
+__device__ __attribute__((always_inline)) inline void walk_batch(
+    int nc, int nq, int sg, unsigned o_ar, int backward, double sor, double rsor,
+    const bool (&act)[NC], Reload reload) {
+  typedef double D2 __attribute__((ext_vector_type(2)));
+  // Every segment has at most 64 cells: lane l updates cell sg[q] + l of
+  // segment q (bounds from lane q of sg).  Two operand sets alternate: while
+  // segment j computes from one, the other receives segment j+1's ap, 1/ap,
+  // b, anb, neighbour addresses and own old value (its cells are not
+  // written at level j); right after segment j's stores it receives its
+  // neighbour values.  The walk is one wavefront's, whose LDS accesses
+  // execute in issue order, so those reads see the stores without waiting
+  // for them.  Lanes without a cell read a later cell's operands and store
+  // to the 32 bytes after the table.
+  // RCP: the divisions by ap and sor use div_rcp2.  Without a branch in the
+  // walk, each lane keeps the least and greatest frexp exponent of its
+  // dividends x and a NaN detector (0*nv is NaN for an infinite or NaN
+  // result, which an out-of-range 1/ap or an overflow produces); if any
+  // lane saw a dividend outside [-kRcpExp, kRcpExp] or a non-finite
+  // result, the batch is walked again with hardware division from its
+  // original values, which global memory still holds.
+  const int lane = threadIdx.x;
+  const double sm1 = sor - 1.0;
+  // The next segment's neighbour addresses are read first and unpacked
+  // before this level's arithmetic (they are next in the LDS queue after
+  // this level's values); its other operands are used only after this
+  // level's store, so the own values stay raw (p).
+  struct Ops {
+    int st, en;   // the segment's cells [st, en) (uniform)
+    unsigned pv;  // LDS byte address of the lane's cell's values (a later cell without a cell)
+    bool on;
+    double a, ya, bv[NC], p[NC], an[6], v[NC][6];
+    unsigned sl[6];
+  };
+  // LDS byte addresses of the walk's arrays (the dynamic block starts at
+  // 0), so that an operand's address is one add or 24-bit multiply-add
+  typedef const __attribute__((address_space(3))) double *LdsD;
+  const unsigned b_ar = o_ar, b_b = b_ar + 16u * nc, b_an = b_b + 8u * NC * nc,
+                 b_sl = (b_an + 48u * nc + 15u) & ~15u, b_dum = b_sl + 16u * nc;
+  auto lds_f64 = [](unsigned a) { return *reinterpret_cast<LdsD>(static_cast<size_t>(a)); };
+  // operands and own values of the segment of cells [st, en)
+  auto load_ops = [&](int st, int en, Ops &o) {
+    o.st = st;
+    o.en = en;
+    const int ii = st + lane;
+    o.on = ii < en;
+    // lanes past the segment read a later cell of the batch (its last
+    // past the end): real operands, so the division guard stays valid
+    const unsigned ic = min(ii, nc - 1);
+    // 12 of the record's 16 bytes (a fourth, dead register would be
+    // reused at once and make the compiler wait for this read)
+    typedef unsigned U3 __attribute__((ext_vector_type(3)));
+    const U3 w = *reinterpret_cast<const __attribute__((address_space(3))) U3 *>(
+        static_cast<size_t>(b_sl + 16u * ic));
+    __builtin_amdgcn_sched_barrier(0);  // first in the LDS queue after the values
+#pragma unroll
+    for (int k = 0; k < 6; k++) o.sl[k] = (k & 1 ? w[k >> 1] >> 16 : w[k >> 1] & 0xffffu);
+    const unsigned c8 = 8u * ic;
+    o.pv = NC == 1 ? c8 : __umul24(ic, 8u * NC);
+    const D2 ar = *reinterpret_cast<const __attribute__((address_space(3))) D2 *>(
+        static_cast<size_t>(b_ar + 2u * c8));
+    o.a = ar.x;
+    o.ya = ar.y;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      o.bv[c] = lds_f64(b_b + 8u * c * nc + c8);
+      o.p[c] = lds_f64(o.pv + 8u * c);
+    }
+    const unsigned an = __umul24(ic, 48u) + b_an;
+#pragma unroll
+    for (int k = 0; k < 6; k++) o.an[k] = lds_f64(an + 8u * k);
+  };
+  // neighbour values at the LDS byte addresses the host stored
+  auto load_v = [&](Ops &o) {
+#pragma unroll
+    for (int k = 0; k < 6; k++)
+#pragma unroll
+      for (int c = 0; c < NC; c++)
+        o.v[c][k] = *reinterpret_cast<const __attribute__((address_space(3))) double *>(
+            static_cast<size_t>(o.sl[k] + 8 * c));
+  };
+  // The visit direction is a compile-time argument (bwd is a
+  // std::integral_constant): the next segment shares one bound with the
+  // current one, so a level reads one segment bound (lane q of sg).
+  auto walk = [&](bool rcp, auto bwd) __attribute__((always_inline)) -> bool {
+    constexpr bool BWD = decltype(bwd)::value;
+    int emin = 0, emax = 0;
+    double nan_seen = 0.0;
+    // level j of the walk: the j-th segment, then (more) the operands of
+    // the next
+    auto step = [&](int j, Ops &cur, Ops &nxt, bool more) {
+      if (more) {
+        if (BWD)
+          load_ops(__builtin_amdgcn_readlane(sg, nq - 2 - j), cur.st, nxt);
+        else
+          load_ops(cur.en, __builtin_amdgcn_readlane(sg, j + 2), nxt);
+      }
+      // the operand loads go out before this level's arithmetic
+      __builtin_amdgcn_sched_barrier(0);
+      double xg[NC], ng[NC];
+      // with several right-hand sides every one is computed, and one whose
+      // solve has stopped (not act) stores past the table, like a lane
+      // without a cell (fewer instructions than a select per use)
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        if (NC == 1 && !act[c]) continue;
+        double sum = cur.bv[c];
+#pragma unroll
+        for (int k = 0; k < 6; k++) sum = sum + cur.an[k] * cur.v[c][k];
+        const double x = sum + sm1 * cur.a * cur.p[c];
+        double nv;
+        if (rcp)
+          nv = div_rcp2(x, cur.a, cur.ya, sor, rsor);
+        else
+          nv = x / cur.a / sor;
+        xg[c] = x;
+        ng[c] = nv;
+        // unconditional store, so no branch separates it from the next
+        // segment's loads; lanes without a cell store past the table
+        *reinterpret_cast<__attribute__((address_space(3))) double *>(
+            static_cast<size_t>(((NC == 1 || act[c]) && cur.on ? cur.pv : b_dum) + 8u * c)) = nv;
+      }
+      wave_sync();  // the walk is one wavefront (kLdsThreads = 64)
+      if (more) load_v(nxt);
+      // the guard's bookkeeping waits with the next level's values, off
+      // the chain from this level's dividend to its store
+      __builtin_amdgcn_sched_barrier(0);
+      if (rcp) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          if (NC == 1 && !act[c]) continue;
+          const int ex = __builtin_amdgcn_frexp_exp(xg[c]);  // 0 for x = 0
+          emin = min(emin, ex);
+          emax = max(emax, ex);
+          nan_seen = fma(0.0, ng[c], nan_seen);
+        }
+      }
+    };
+    Ops A, B;
+    if (BWD)
+      load_ops(__builtin_amdgcn_readlane(sg, nq - 1), __builtin_amdgcn_readlane(sg, nq), A);
+    else
+      load_ops(__builtin_amdgcn_readlane(sg, 0), __builtin_amdgcn_readlane(sg, 1), A);
+    load_v(A);
+    // the loop's levels all have a next segment; the last one or two
+    // levels follow it
+    int j = 0;
+    for (; j + 2 < nq; j += 2) {
+      step(j, A, B, true);
+      step(j + 1, B, A, true);
+    }
+    if (j + 1 < nq) {
+      step(j, A, B, true);
+      step(j + 1, B, A, false);
+    } else {
+      step(j, A, B, false);
+    }
+    return emin < -kRcpExp || emax > kRcpExp || nan_seen != nan_seen;
+  };
+  auto walk_dir = [&](bool rcp) __attribute__((always_inline)) -> bool {
+    return backward ? walk(rcp, std::true_type{}) : walk(rcp, std::false_type{});
+  };
+  if (rsor > 0.0) {
+    if (__builtin_amdgcn_ballot_w64(walk_dir(true))) {
+      reload();
+      wave_sync();
+      walk_dir(false);
+    }
+  } else {
+    walk_dir(false);
+  }
+}
+
 template <bool HEX, bool PIPE, int NC, int NW>
 __global__ void __launch_bounds__(kLdsThreads * NW)
 k_gs_tiles_lds(int batch0, const int4 *__restrict__ bdesc, const int *__restrict__ active,
@@ -1508,174 +1686,11 @@ k_gs_tiles_lds(int batch0, const int4 *__restrict__ bdesc, const int *__restrict
   if constexpr (PIPE) {
     // wavefront 0 walks; the others wait at the barrier before the write-back
     if (NW == 1 || threadIdx.x < kLdsThreads) {
-      // Every segment has at most 64 cells: lane l updates cell sg[q] + l of
-      // segment q (bounds from lane q of sg).  Two operand sets alternate: while
-      // segment j computes from one, the other receives segment j+1's ap, 1/ap,
-      // b, anb, neighbour addresses and own old value (its cells are not
-      // written at level j); right after segment j's stores it receives its
-      // neighbour values.  The walk is one wavefront's, whose LDS accesses
-      // execute in issue order, so those reads see the stores without waiting
-      // for them.  Lanes without a cell read a later cell's operands and store
-      // to the 32 bytes after the table.
-      // RCP: the divisions by ap and sor use div_rcp2.  Without a branch in the
-      // walk, each lane keeps the least and greatest frexp exponent of its
-      // dividends x and a NaN detector (0*nv is NaN for an infinite or NaN
-      // result, which an out-of-range 1/ap or an overflow produces); if any
-      // lane saw a dividend outside [-kRcpExp, kRcpExp] or a non-finite
-      // result, the batch is walked again with hardware division from its
-      // original values, which global memory still holds.
-      const int lane = threadIdx.x;
-      const double sm1 = sor - 1.0;
-      // The next segment's neighbour addresses are read first and unpacked
-      // before this level's arithmetic (they are next in the LDS queue after
-      // this level's values); its other operands are used only after this
-      // level's store, so the own values stay raw (p).
-      struct Ops {
-        int st, en;   // the segment's cells [st, en) (uniform)
-        unsigned pv;  // LDS byte address of the lane's cell's values (a later cell without a cell)
-        bool on;
-        double a, ya, bv[NC], p[NC], an[6], v[NC][6];
-        unsigned sl[6];
-      };
-      // LDS byte addresses of the walk's arrays (the dynamic block starts at
-      // 0), so that an operand's address is one add or 24-bit multiply-add
-      typedef const __attribute__((address_space(3))) double *LdsD;
-      const unsigned b_ar = o_ar, b_b = b_ar + 16u * nc, b_an = b_b + 8u * NC * nc,
-                     b_sl = (b_an + 48u * nc + 15u) & ~15u, b_dum = b_sl + 16u * nc;
-      auto lds_f64 = [](unsigned a) { return *reinterpret_cast<LdsD>(static_cast<size_t>(a)); };
-      // operands and own values of the segment of cells [st, en)
-      auto load_ops = [&](int st, int en, Ops &o) {
-        o.st = st;
-        o.en = en;
-        const int ii = st + lane;
-        o.on = ii < en;
-        // lanes past the segment read a later cell of the batch (its last
-        // past the end): real operands, so the division guard stays valid
-        const unsigned ic = min(ii, nc - 1);
-        // 12 of the record's 16 bytes (a fourth, dead register would be
-        // reused at once and make the compiler wait for this read)
-        typedef unsigned U3 __attribute__((ext_vector_type(3)));
-        const U3 w = *reinterpret_cast<const __attribute__((address_space(3))) U3 *>(
-            static_cast<size_t>(b_sl + 16u * ic));
-        __builtin_amdgcn_sched_barrier(0);  // first in the LDS queue after the values
+      walk_batch<NC>(nc, nq, sg, o_ar, backward, sor, rsor, act, [&] {
+        for (int r = threadIdx.x; r < nc; r += kLdsThreads)
 #pragma unroll
-        for (int k = 0; k < 6; k++) o.sl[k] = (k & 1 ? w[k >> 1] >> 16 : w[k >> 1] & 0xffffu);
-        const unsigned c8 = 8u * ic;
-        o.pv = NC == 1 ? c8 : __umul24(ic, 8u * NC);
-        const D2 ar = *reinterpret_cast<const __attribute__((address_space(3))) D2 *>(
-            static_cast<size_t>(b_ar + 2u * c8));
-        o.a = ar.x;
-        o.ya = ar.y;
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-          o.bv[c] = lds_f64(b_b + 8u * c * nc + c8);
-          o.p[c] = lds_f64(o.pv + 8u * c);
-        }
-        const unsigned an = __umul24(ic, 48u) + b_an;
-#pragma unroll
-        for (int k = 0; k < 6; k++) o.an[k] = lds_f64(an + 8u * k);
-      };
-      // neighbour values at the LDS byte addresses the host stored
-      auto load_v = [&](Ops &o) {
-#pragma unroll
-        for (int k = 0; k < 6; k++)
-#pragma unroll
-          for (int c = 0; c < NC; c++)
-            o.v[c][k] = *reinterpret_cast<const __attribute__((address_space(3))) double *>(
-                static_cast<size_t>(o.sl[k] + 8 * c));
-      };
-      // The visit direction is a compile-time argument (bwd is a
-      // std::integral_constant): the next segment shares one bound with the
-      // current one, so a level reads one segment bound (lane q of sg).
-      auto walk = [&](bool rcp, auto bwd) __attribute__((always_inline)) -> bool {
-        constexpr bool BWD = decltype(bwd)::value;
-        int emin = 0, emax = 0;
-        double nan_seen = 0.0;
-        // level j of the walk: the j-th segment, then (more) the operands of
-        // the next
-        auto step = [&](int j, Ops &cur, Ops &nxt, bool more) {
-          if (more) {
-            if (BWD)
-              load_ops(__builtin_amdgcn_readlane(sg, nq - 2 - j), cur.st, nxt);
-            else
-              load_ops(cur.en, __builtin_amdgcn_readlane(sg, j + 2), nxt);
-          }
-          // the operand loads go out before this level's arithmetic
-          __builtin_amdgcn_sched_barrier(0);
-          double xg[NC], ng[NC];
-          // with several right-hand sides every one is computed, and one whose
-          // solve has stopped (not act) stores past the table, like a lane
-          // without a cell (fewer instructions than a select per use)
-#pragma unroll
-          for (int c = 0; c < NC; c++) {
-            if (NC == 1 && !act[c]) continue;
-            double sum = cur.bv[c];
-#pragma unroll
-            for (int k = 0; k < 6; k++) sum = sum + cur.an[k] * cur.v[c][k];
-            const double x = sum + sm1 * cur.a * cur.p[c];
-            double nv;
-            if (rcp)
-              nv = div_rcp2(x, cur.a, cur.ya, sor, rsor);
-            else
-              nv = x / cur.a / sor;
-            xg[c] = x;
-            ng[c] = nv;
-            // unconditional store, so no branch separates it from the next
-            // segment's loads; lanes without a cell store past the table
-            *reinterpret_cast<__attribute__((address_space(3))) double *>(
-                static_cast<size_t>(((NC == 1 || act[c]) && cur.on ? cur.pv : b_dum) + 8u * c)) = nv;
-          }
-          wave_sync();  // the walk is one wavefront (kLdsThreads = 64)
-          if (more) load_v(nxt);
-          // the guard's bookkeeping waits with the next level's values, off
-          // the chain from this level's dividend to its store
-          __builtin_amdgcn_sched_barrier(0);
-          if (rcp) {
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-              if (NC == 1 && !act[c]) continue;
-              const int ex = __builtin_amdgcn_frexp_exp(xg[c]);  // 0 for x = 0
-              emin = min(emin, ex);
-              emax = max(emax, ex);
-              nan_seen = fma(0.0, ng[c], nan_seen);
-            }
-          }
-        };
-        Ops A, B;
-        if (BWD)
-          load_ops(__builtin_amdgcn_readlane(sg, nq - 1), __builtin_amdgcn_readlane(sg, nq), A);
-        else
-          load_ops(__builtin_amdgcn_readlane(sg, 0), __builtin_amdgcn_readlane(sg, 1), A);
-        load_v(A);
-        // the loop's levels all have a next segment; the last one or two
-        // levels follow it
-        int j = 0;
-        for (; j + 2 < nq; j += 2) {
-          step(j, A, B, true);
-          step(j + 1, B, A, true);
-        }
-        if (j + 1 < nq) {
-          step(j, A, B, true);
-          step(j + 1, B, A, false);
-        } else {
-          step(j, A, B, false);
-        }
-        return emin < -kRcpExp || emax > kRcpExp || nan_seen != nan_seen;
-      };
-      auto walk_dir = [&](bool rcp) __attribute__((always_inline)) -> bool {
-        return backward ? walk(rcp, std::true_type{}) : walk(rcp, std::false_type{});
-      };
-      if (rsor > 0.0) {
-        if (__builtin_amdgcn_ballot_w64(walk_dir(true))) {
-          for (int r = threadIdx.x; r < nc; r += kLdsThreads)
-#pragma unroll
-            for (int c = 0; c < NC; c++) pphi[NC * r + c] = s.phi[c][c0 + r];
-          wave_sync();
-          walk_dir(false);
-        }
-      } else {
-        walk_dir(false);
-      }
+          for (int c = 0; c < NC; c++) pphi[NC * r + c] = s.phi[c][c0 + r];
+      });
     } else {
       // wavefronts 1.. meanwhile bring the next launch's batches that will
       // run in this workgroup's slot (same block index modulo the XCD count,
@@ -1726,6 +1741,203 @@ k_gs_tiles_lds(int batch0, const int4 *__restrict__ bdesc, const int *__restrict
       __hip_atomic_store(&s.phi[c][c0 + r], PIPE ? pphi[NC * r + c] : lphi[c * np + r],
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
+}
+
+// Several sweeps of the same batches in one launch.  Workgroups take (sweep,
+// batch) tickets in schedule order from a counter and wait, per batch, for the
+// batches it depends on instead of for a whole launch: a batch may start once
+// every neighbouring batch of an earlier launch (forward; of a later one,
+// backward) has finished this sweep and the batch itself the sweep before.
+//   * No workgroup waits for a larger ticket, and each works on its tickets in
+//     increasing order, so the smallest unfinished one always runs: the waits
+//     end whatever part of the grid is resident.  They are bounded all the
+//     same (kFlowTicks): past that *err is set, every wait returns at once and
+//     the host reports the failure.
+//   * done[b] counts batch b's finished sweeps since the solve began.  Values
+//     move between workgroups through memory (system-scope stores, agent-scope
+//     loads, which bypass the XCDs' L2s); a batch's stores are complete
+//     (vmcnt 0, then the barrier) before its count is stored.
+//   * A batch's neighbours of a later launch (forward) still hold their values
+//     of the sweep before: they wait for this batch, and it has waited for
+//     them in the sweep before, as its own finished sweep shows.
+// Bound by the dependency chain: per batch the wait's round trips (its stores
+// reaching memory, the count, the poll, the values: about 2 us) and 0.15 us per
+// level.  A launch per step added the kernel boundary and a full gather after
+// it, and every step lasted as long as its longest batch.  Three outer
+// iterations, a launch per step / this kernel: 16^3 11.2 / 9.3 ms, 32^3 22.5 /
+// 18.4 ms, 61 x 47 x 53 70.5 / 53.9 ms, 64^3 63.8 / 49.3 ms, 128^3 158 / 135 ms,
+// 192^3 267 / 224 ms.
+template <int NC>
+struct FlowArgs {
+  TileSys<NC> s;
+  const int4 *bdesc;
+  const int *seg, *xslot;
+  const unsigned short *lnbr;
+  const int *dptr, *dep;  // batch b's neighbours dep[dptr[2b] .. dptr[2b+1]) earlier, .. dptr[2b+2]) later
+  int *done, *err;
+  unsigned *ticket;
+  unsigned base;           // the counter's value before this launch
+  int nb, nsweep, sweep0;  // batches; sweeps of this launch; sweeps finished before it
+  int slot;                // LDS byte offset of the ticket slot (after the largest batch)
+};
+constexpr long long kFlowTicks = 2000000000LL;  // 20 s of the 100 MHz counter
+
+__device__ inline int flow_load(const int *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline double flow_load(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <int NC>
+__global__ void __launch_bounds__(kLdsThreads * 4)
+k_gs_flow(FlowArgs<NC> A, const int *__restrict__ active, double sor, double rsor) {
+  extern __shared__ double lds[];
+  constexpr int T = kLdsThreads * 4;
+  typedef unsigned U4 __attribute__((ext_vector_type(4)));
+  typedef double D2 __attribute__((ext_vector_type(2)));
+  const TileSys<NC> &s = A.s;
+  bool act[NC];
+  bool any = false;
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    act[c] = active[c] != 0;
+    any = any || act[c];
+  }
+  if (!any) return;
+  const int tid = threadIdx.x;
+  volatile unsigned *slot =
+      reinterpret_cast<volatile unsigned *>(reinterpret_cast<char *>(lds) + A.slot);
+  auto draw = [&] {
+    return __hip_atomic_fetch_add(A.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) -
+           A.base;
+  };
+  if (tid == kLdsThreads) *slot = draw();
+  __syncthreads();
+  const unsigned n = static_cast<unsigned>(A.nb) * static_cast<unsigned>(A.nsweep);
+  for (unsigned t = __builtin_amdgcn_readfirstlane(*slot); t < n;
+       t = __builtin_amdgcn_readfirstlane(*slot)) {
+    const int sw = static_cast<int>(t / A.nb), i = static_cast<int>(t - sw * A.nb);
+    const int backward = sw & 1, b = backward ? A.nb - 1 - i : i, need = A.sweep0 + sw + 1;
+    const int4 d0 = A.bdesc[2 * b], d1 = A.bdesc[2 * b + 1];
+    const int s0 = d0.x, nq = d0.y, c0 = d0.z, nc = d0.w;
+    const int r0 = d1.x, x0 = d1.z, nx = d1.w;
+    const int p0 = A.dptr[2 * b + backward], nd = A.dptr[2 * b + backward + 1] - p0;
+    const int np = nc + nx;
+    // the pipelined walk's LDS layout (k_gs_tiles_lds)
+    double *pphi = lds;
+    const unsigned o_ar = (8u * NC * np + 15u) & ~15u;
+    D2 *par = reinterpret_cast<D2 *>(reinterpret_cast<char *>(lds) + o_ar);
+    double *pb = reinterpret_cast<double *>(par + nc);
+    double *panb = pb + NC * nc;
+    U4 *psl = reinterpret_cast<U4 *>(reinterpret_cast<char *>(lds) +
+                                     ((o_ar + 8u * (2 + NC + 6) * nc + 15u) & ~15u));
+    const int sg = A.seg[s0 + min(tid, nq)] - c0;
+    // what no sweep changes, and the outside indices, before the wait
+    const unsigned *pl = reinterpret_cast<const unsigned *>(A.lnbr + r0);
+    constexpr int X = 3;
+    int xs[X];
+#pragma unroll
+    for (int u = 0; u < X; u++) xs[u] = A.xslot[max(x0 + min(u * T + tid, nx - 1), 0)];
+    for (int i0 = 0; i0 < nc; i0 += 2 * T) {
+      double va[2], vr[2], vn[2][6], vb[NC][2];
+      unsigned sl[2][3];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int ic = min(i0 + u * T + tid, nc - 1);
+        va[u] = s.ap[c0 + ic];
+        vr[u] = s.rap[c0 + ic];
+#pragma unroll
+        for (int c = 0; c < NC; c++) vb[c][u] = s.b[c][c0 + ic];
+#pragma unroll
+        for (int k = 0; k < 6; k++) vn[u][k] = s.anb[r0 + 6 * ic + k];
+#pragma unroll
+        for (int k = 0; k < 3; k++) sl[u][k] = pl[3 * ic + k];
+      }
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int ic = i0 + u * T + tid;
+        if (ic < nc) {
+          par[ic] = D2{va[u], vr[u]};
+#pragma unroll
+          for (int c = 0; c < NC; c++) pb[c * nc + ic] = vb[c][u];
+#pragma unroll
+          for (int k = 0; k < 6; k++) panb[6 * ic + k] = vn[u][k];
+          psl[ic] = U4{sl[u][0], sl[u][1], sl[u][2], 0u};
+        }
+      }
+    }
+    // wait for the neighbouring batches (one lane each) and the batch itself
+    if (tid < kLdsThreads) {
+      const int *f = A.done + (tid < nd ? A.dep[p0 + tid] : b);
+      const int want = tid < nd ? need : need - 1;
+      const bool on = tid <= nd;
+      long long start = 0;
+      for (int k = 0; __builtin_amdgcn_ballot_w64(on && flow_load(f) < want); k++) {
+        if ((k & 1023) == 1023) {
+          const long long now = wall_clock64();
+          if (start == 0) start = now;
+          if (now - start > kFlowTicks)
+            __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (flow_load(A.err)) break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+    }
+    __syncthreads();
+    // the values, which the wait has made final
+    {
+      double vx[NC][X], vp[NC][X];
+#pragma unroll
+      for (int u = 0; u < X; u++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          vx[c][u] = flow_load(s.phi[c] + static_cast<unsigned>(xs[u]));
+          vp[c][u] = flow_load(s.phi[c] + c0 + min(u * T + tid, nc - 1));
+        }
+#pragma unroll
+      for (int u = 0; u < X; u++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          const int j = u * T + tid;
+          if (j < nx) pphi[NC * (nc + j) + c] = vx[c][u];
+          if (j < nc) pphi[NC * j + c] = vp[c][u];
+        }
+      for (int j = X * T + tid; j < max(nx, nc); j += T)
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          if (j < nx) pphi[NC * (nc + j) + c] = flow_load(s.phi[c] + A.xslot[x0 + j]);
+          if (j < nc) pphi[NC * j + c] = flow_load(s.phi[c] + c0 + j);
+        }
+    }
+    __syncthreads();
+    if (tid < kLdsThreads)
+      walk_batch<NC>(nc, nq, sg, o_ar, backward, sor, rsor, act, [&] {
+        for (int r = tid; r < nc; r += kLdsThreads)
+#pragma unroll
+          for (int c = 0; c < NC; c++) pphi[NC * r + c] = flow_load(s.phi[c] + c0 + r);
+      });
+    else if (tid == kLdsThreads)
+      *slot = draw();  // the next ticket's round trip runs beside the walk
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      if (!act[c]) continue;
+      for (int r = tid; r < nc; r += T)
+        __hip_atomic_store(&s.phi[c][c0 + r], pphi[NC * r + c], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0)
+      __hip_atomic_store(A.done + b, need, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+// the counts and the ticket counter of a solve's sweeps
+__global__ void k_flow_reset(int *done, int n, unsigned *ticket) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) done[i] = 0;
+  if (i == 0) *ticket = 0;
 }
 
 // Residual partial sums: block (x, y) covers cells [beg_y + x*chunk, ...).
@@ -2315,6 +2527,12 @@ struct cfdl_ctx {
     bool prefetch = true;  // idle wavefronts bring the next launch's batches into L2
     int nbatch = 0, nseg = 0;
     size_t lds_bytes = 0;  // 0: batches too large for LDS, global-memory kernel
+    // k_gs_flow: neighbouring batches, finished sweeps, ticket counter; per
+    // solve the sweeps enqueued and the tickets drawn (0 workgroups: not used)
+    int *dptr = nullptr, *dep = nullptr, *done = nullptr;
+    unsigned *ticket = nullptr;
+    int flow_wgs = 0, flow_sweeps = 0;
+    unsigned flow_base = 0;
   } ts, tm;
   // the global system in tile numbering (tiled solve_gs): new -> old cell,
   // CSR, and copies of the shared coefficients, right-hand sides and values
@@ -2597,6 +2815,65 @@ static void tiled_launches(cfdl_ctx *c, const cfdl_ctx::TileSched &t, const SysD
   }
 }
 
+static int flow_failed() {
+  set_error("a Gauss-Seidel sweep waited more than 20 s for another part of its work");
+  return CFDL_EHIP;
+}
+// whether a wait of k_gs_flow has run out of time so far (synchronises); its
+// results are invalid then, and every later call reports it
+static int flow_check(cfdl_ctx *c) {
+  if (c->ts.flow_wgs == 0 && c->tm.flow_wgs == 0) return CFDL_OK;
+  HIPCHK(hipMemcpyAsync(c->host_flags, &c->gctl->flow_err, sizeof(int), hipMemcpyDeviceToHost,
+                        c->st));
+  HIPCHK(hipStreamSynchronize(c->st));
+  return c->host_flags[0] ? flow_failed() : CFDL_OK;
+}
+
+// nsweep sweeps (forward, backward, forward, ..) in one launch of k_gs_flow
+template <int NC>
+static int flow_launch(cfdl_ctx *c, cfdl_ctx::TileSched &t, const SysDesc &sys, int nsweep,
+                       double sor, const int *active) {
+  const bool rcp_ok = c->rcp && sor >= kRcpDivMin && sor <= kRcpDivMax;
+  FlowArgs<NC> a{};
+  for (int k = 0; k < NC; k++) {
+    a.s.phi[k] = sys.phi[k];
+    a.s.b[k] = sys.b[k];
+  }
+  a.s.ap = sys.ap;
+  a.s.anb = sys.anb;
+  a.s.rap = sys.rap;
+  a.s.row = sys.row;
+  a.bdesc = t.bdesc;
+  a.seg = t.seg;
+  a.xslot = t.xslot;
+  a.lnbr = (NC == 1 && t.lnbr1) ? t.lnbr1 : t.lnbr;
+  a.dptr = t.dptr;
+  a.dep = t.dep;
+  a.done = t.done;
+  a.err = &c->gctl->flow_err;
+  a.ticket = t.ticket;
+  a.base = t.flow_base;
+  a.nb = t.nbatch;
+  a.nsweep = nsweep;
+  a.sweep0 = t.flow_sweeps;
+  a.slot = static_cast<int>(t.lds_bytes);
+  hipLaunchKernelGGL(k_gs_flow<NC>, dim3(t.flow_wgs), dim3(kLdsThreads * 4), t.lds_bytes + 16,
+                     c->st, a, active, sor, rcp_ok ? 1.0 / sor : 0.0);
+  HIPCHK(hipGetLastError());
+  // every workgroup draws one ticket past the end
+  t.flow_base += static_cast<unsigned>(t.nbatch) * nsweep + t.flow_wgs;
+  t.flow_sweeps += nsweep;
+  return CFDL_OK;
+}
+static int flow_begin(cfdl_ctx *c, cfdl_ctx::TileSched &t) {
+  t.flow_sweeps = 0;
+  t.flow_base = 0;
+  hipLaunchKernelGGL(k_flow_reset, dim3(nblocks(t.nbatch)), dim3(kBlock), 0, c->st, t.done,
+                     t.nbatch, t.ticket);
+  HIPCHK(hipGetLastError());
+  return CFDL_OK;
+}
+
 static int pc_sweep_tiled(cfdl_ctx *c, const SysDesc &sys, bool forward, const int *active) {
   const cfdl_ctx::TileSched &t = c->ts;
   const int nl = static_cast<int>(t.launch_ptr.size()) - 1;
@@ -2617,6 +2894,18 @@ static int pc_sweep_tiled(cfdl_ctx *c, const SysDesc &sys, bool forward, const i
   c->pc_cells += c->ne;
   c->gs_launches += nl;
   HIPCHK(hipGetLastError());
+  return CFDL_OK;
+}
+
+// the two symmetric iterations of a pc block in one launch
+static int pc_block_flow(cfdl_ctx *c, const SysDesc &sys, const int *active) {
+  cfdl_ctx::Sample *smp = nullptr;
+  CALL(sample_begin(c, &smp));
+  CALL(flow_launch<1>(c, c->ts, sys, 4, 1.02, active));
+  CALL(sample_end(c, smp, 1, 4 * int64_t{c->ne}));
+  c->pc_launches += 1;
+  c->pc_cells += 4 * int64_t{c->ne};
+  c->gs_launches += 1;
   return CFDL_OK;
 }
 
@@ -2717,6 +3006,11 @@ static int solve_gs_n(cfdl_ctx *c, int ny, double **phi, const double **b,
       }
       c->gs_launches += static_cast<int>(turns.size());
       HIPCHK(hipGetLastError());
+    } else if (tiled && c->tm.flow_wgs > 0) {
+      if (it == 0) CALL(flow_begin(c, c->tm));
+      CALL(ny == 3 ? flow_launch<3>(c, c->tm, s, 2, sor, gs_active(c))
+                   : flow_launch<1>(c, c->tm, s, 2, sor, gs_active(c)));
+      c->gs_launches += 1;
     } else if (tiled) {
       const int nl = static_cast<int>(c->tm.launch_ptr.size()) - 1;
       if (ny == 3) {
@@ -2735,9 +3029,10 @@ static int solve_gs_n(cfdl_ctx *c, int ny, double **phi, const double **b,
     CALL(residual(c, s, c->nblk_g, c->chunk_g, 1));
     hipLaunchKernelGGL(k_gs_iter_end, dim3(1), dim3(64), 0, c->st, c->gctl, c->red, ny,
                        static_cast<double>(c->ne), c->nit);
-    HIPCHK(hipMemcpyAsync(c->host_flags, gs_active(c), sizeof(int) * 3, hipMemcpyDeviceToHost,
+    HIPCHK(hipMemcpyAsync(c->host_flags, gs_active(c), sizeof(int) * 4, hipMemcpyDeviceToHost,
                           c->st));
     HIPCHK(hipStreamSynchronize(c->st));
+    if (c->host_flags[3]) return flow_failed();
     bool any = false;
     for (int y = 0; y < ny; y++) any = any || c->host_flags[y];
     if (!any) break;
@@ -2796,12 +3091,15 @@ static int multi_subdomain_solver(cfdl_ctx *c) {
   SysDesc s1 = s;  // the sweeps see the whole concatenated system as one RHS
   s1.ny = 1;
   const int *act = pc_active(c);
+  const bool flow = !col && c->tiled && c->ts.flow_wgs > 0;
+  if (flow) CALL(flow_begin(c, c->ts));
   const int nblock = (c->nit + 1) / 2;
   for (int blk = 1; blk <= nblock; blk++) {
     // smoother_gs(..., 2): two symmetric iterations
     if (mixed) CALL(pc_block_colour(c, s32, act));
     if (c->pc_order == CFDL_PC_COLORED) CALL(pc_block_colour(c, s64, act));
-    for (int rep = 0; rep < 2 && !col; rep++) {
+    if (flow) CALL(pc_block_flow(c, s1, act));
+    for (int rep = 0; rep < 2 && !col && !flow; rep++) {
       if (c->tiled) {
         CALL(pc_sweep_tiled(c, s1, true, act));
         CALL(pc_sweep_tiled(c, s1, false, act));
@@ -3035,6 +3333,59 @@ static void plan_tiles(int ne, const std::vector<int> &row, const std::vector<in
   }
 }
 
+// The neighbouring batches of every batch (those holding its outside
+// neighbours), of earlier and of later launches, and the counters of
+// k_gs_flow; no table, and so the launch-by-launch sweeps, if a batch has
+// more of either than the waiting wavefront has lanes.
+static int flow_tables(cfdl_ctx *c, const std::vector<int> &rowp, const std::vector<int> &nbrp,
+                       const std::vector<int> &seg, const std::vector<int> &bseg,
+                       cfdl_ctx::TileSched *tp) {
+  cfdl_ctx::TileSched &t = *tp;
+  const int ne = c->ne, nb = t.nbatch;
+  std::vector<int> bof(ne), dptr, dep, part[2];
+  for (int b = 0; b < nb; b++)
+    for (int e = seg[bseg[b]]; e < seg[bseg[b + 1] - 1]; e++) bof[e] = b;
+  std::vector<int> launch(nb), seen(nb, -1);
+  for (size_t m = 0; m + 1 < t.launch_ptr.size(); m++)
+    for (int b = t.launch_ptr[m]; b < t.launch_ptr[m + 1]; b++) launch[b] = static_cast<int>(m);
+  dptr.push_back(0);
+  for (int b = 0; b < nb; b++) {
+    part[0].clear();
+    part[1].clear();
+    for (int k = rowp[seg[bseg[b]]]; k < rowp[seg[bseg[b + 1] - 1]]; k++) {
+      const int d = nbrp[k] < ne ? bof[nbrp[k]] : b;
+      if (d == b || seen[d] == b) continue;
+      seen[d] = b;
+      part[launch[d] > launch[b] ? 1 : 0].push_back(d);
+    }
+    for (const auto &p : part) {
+      if (p.size() >= static_cast<size_t>(kLdsThreads)) return CFDL_OK;
+      dep.insert(dep.end(), p.begin(), p.end());
+      dptr.push_back(static_cast<int>(dep.size()));
+    }
+  }
+  const char *fl = std::getenv("CFDL_FLOW");
+  const int per_cu = static_cast<int>((160 * 1024) / (t.lds_bytes + 16));
+  // a workgroup per CU, more where the middle launches have more batches (three
+  // outer iterations with 256 / 512 / 768: 61 x 47 x 53 53.9 / 54.9 / 54.9 ms,
+  // 128^3 135.1 / 135.9 / 137.7 ms, 192^3 317 / 232 / 224 ms)
+  const int mean = nb / static_cast<int>(t.launch_ptr.size() - 1);
+  const int wgs = fl ? std::atoi(fl) : 256 * std::min(per_cu, 1 + mean / 140);
+  if (wgs <= 0 || per_cu < 1) return CFDL_OK;
+  CALL(upload(c, &t.dptr, dptr));
+  CALL(upload(c, &t.dep, dep));
+  CALL(dalloc(c, &t.done, nb));
+  CALL(dalloc(c, &t.ticket, 1));
+  int lds_dev = 0;
+  HIPCHK(hipDeviceGetAttribute(&lds_dev, hipDeviceAttributeMaxSharedMemoryPerBlock, c->dev));
+  HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gs_flow<1>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_dev));
+  HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gs_flow<3>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, lds_dev));
+  t.flow_wgs = std::min(wgs, nb);
+  return CFDL_OK;
+}
+
 // Batch tables of the tiled sweeps on the renumbered pc system, whose cells
 // are ordered by (subdomain, launch, tile, level): each batch is the run of
 // cells with equal (subdomain, launch, tile), each segment the run of equal
@@ -3191,6 +3542,7 @@ static int build_tile_tables(cfdl_ctx *c, const std::vector<int> &rowp,
     bdesc[2 * i] = make_int4(s0, nq, c0, nc);
     bdesc[2 * i + 1] = make_int4(rowp[c0], rowp[c0 + nc] - rowp[c0], xptr[i], xptr[i + 1] - xptr[i]);
   }
+  if (t.pipe && t.nw == 4 && t.lds_bytes > 0) CALL(flow_tables(c, rowp, nbrp, seg, bseg, &t));
   CALL(upload(c, &t.bdesc, bdesc));
   CALL(upload(c, &t.bseg, bseg));
   CALL(upload(c, &t.seg, seg));
@@ -3710,6 +4062,7 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
   CALL(dalloc(C, &C->red, 2 * kMaxSys));
   CALL(dalloc(C, &C->scal, 8));
   CALL(dalloc(C, &C->gctl, 1));
+  HIPCHK(hipMemset(C->gctl, 0, sizeof(GsCtl)));
   CALL(dalloc(C, &C->pctl, 1));
   CALL(dalloc(C, &C->dlog, kLogCap));
   CALL(dalloc(C, &C->dlog_n, 1));
@@ -4022,13 +4375,14 @@ int cfdl_get_field(cfdl_ctx *c, int field, double *dst, int64_t n) {
     set_error("cfdl_get_field: bad field id or size");
     return CFDL_EINVAL;
   }
-  return copy_out(c, dst, p, 8 * static_cast<size_t>(n));
+  CALL(copy_out(c, dst, p, 8 * static_cast<size_t>(n)));
+  return flow_check(c);
 }
 
 int cfdl_synchronize(cfdl_ctx *c) {
   CALL(check_ctx(c));
   HIPCHK(hipStreamSynchronize(c->st));
-  return CFDL_OK;
+  return flow_check(c);
 }
 
 int cfdl_ctx_reset(cfdl_ctx *c) {
@@ -4316,6 +4670,7 @@ int cfdl_run_energy(cfdl_ctx *c, int ntstep, int ncoef) { return run_loop(c, nts
 
 static int drain_log(cfdl_ctx *c) {
   HIPCHK(hipStreamSynchronize(c->st));
+  CALL(flow_check(c));
   int n = 0;
   HIPCHK(hipMemcpy(&n, c->dlog_n, sizeof(int), hipMemcpyDeviceToHost));
   if (n > 0) {
