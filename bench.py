@@ -16,8 +16,9 @@ roofline: the pressure-correction Gauss-Seidel sweep kernel k_gs_flow (the domin
 kernel), 108 algorithmic bytes per cell update (FP64 CSR sweep: b, ap, 6
 anb, 6 neighbour indices, own phi read and write) times the cells of one
 launch, over the mean launch duration: HIP events on the context stream
-around every 7th sweep of the timed region (all of its launches, back to
-back), elapsed time divided by launches.  traffic: the HBM bytes per launch
+around every 7th block of four sweeps of the timed region (one launch; all
+launches of a sweep with a launch-by-launch schedule), elapsed time divided
+by launches.  traffic: the HBM bytes per launch
 that rocprofv3 counted for this kernel on the 128^3 workload with the
 default schedule (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, the factors a 256 MiB
 device copy gives), reported for that workload only; --traffic-kib gives

@@ -778,7 +778,7 @@ __global__ void k_temperature(MeshDev m, EnergyDev en) {
 // CSR neighbours (boundary halos included), one thread per cell.
 // ---------------------------------------------------------------------------
 // NC fields share the weights and the inverse of one cell (u, v, w: one pass
-// of 123 us at 128^3 instead of three of 62 us).
+// of 110 us at 128^3 instead of three of 62 us).
 template <int NC>
 struct GradArgs {
   const double *phi[NC];
@@ -2560,8 +2560,8 @@ struct cfdl_ctx {
   int *dlog_n = nullptr;
   std::vector<LogLine> hlog;
   // launch counters and sampled timing of the pressure-correction sweep
-  // kernel: events around every sample_every-th sweep (all its launches,
-  // back to back on the stream)
+  // kernel: events around every sample_every-th step (a sweep, or a block of
+  // sweeps that run together; all its launches, back to back on the stream)
   int64_t gs_launches = 0, pc_launches = 0, pc_cells = 0, outer = 0, pc_sweeps = 0;
   int sample_every = 0;
   struct Sample {
@@ -2653,7 +2653,7 @@ static int sweep(cfdl_ctx *c, const Sched &s, const SysDesc &sys, int nc, double
 
 // Sampled timing of the pressure-correction sweeps: HIP events on the
 // context stream before the first and after the last launch of every
-// sample_every-th sweep.  The launches run back to back in between, so
+// sample_every-th step (a sweep, or a block's sweeps that run together).  The launches run back to back in between, so
 // elapsed / launches is the mean launch duration without the dispatch
 // latency that an event pair around a single launch adds.
 static int sample_begin(cfdl_ctx *c, cfdl_ctx::Sample **smp) {

@@ -391,8 +391,9 @@ void cfdl_batch_destroy(cfdl_batch *b);
 
 /* Launch counters and sampled kernel timing (no counterpart in the
    reference, which has no timers).  cfdl_set_profile(c, k) brackets every
-   k-th pressure-correction sweep (all of its launches, back to back) with
-   HIP events on the context stream (0 = off).  cfdl_stats synchronises and
+   k-th pressure-correction step (all of its launches, back to back: a sweep
+   where it runs launch by launch, else a block's sweeps) with HIP events on
+   the context stream (0 = off).  cfdl_stats synchronises and
    fills up to 8 values: [0] Gauss-Seidel launches (all solves),
    [1] pressure-correction sweep launches, [2] cells updated by those
    launches, [3] outer iterations, [4] launches inside sampled sweeps,
