@@ -2303,6 +2303,7 @@ struct BSlot {
   double *part, *red, *scal;
   LogLine *log;
   int *nlog;
+  uint64_t serial;  // the context's
 };
 
 #define BSLOT                                                                       \
@@ -2461,6 +2462,7 @@ struct DevBuf {
 }  // namespace
 
 struct cfdl_ctx {
+  const uint64_t serial = cfdl::next_serial();
   int dev = 0;
   hipStream_t st = nullptr;
   // while the case is attached to a batch (cfdl_batch_attach) its work runs
@@ -4848,7 +4850,10 @@ struct cfdl_batch {
   int *d_flags = nullptr;
   int *h_flags = nullptr;  // pinned, two sets of kMaxGroup
   hipEvent_t ev[2] = {nullptr, nullptr};
-  std::vector<char> key;   // the descriptors on the device
+  // The descriptors on the device.  With the cases' serial numbers: the graphs'
+  // block counts come from host tables that the descriptors do not show, and a
+  // later context may get a closed one's addresses.
+  std::vector<char> key;
   int block = 0;           // lane count of the element-wise launches; 0 = tuned
   int tuned = 0;           // the tuner's choice for the current composition
   bool tuning = false;     // tuner events recorded, not yet read
@@ -4933,6 +4938,7 @@ int batch_slot(cfdl_ctx *c, BSlot *s) {
   s->scal = c->scal;
   s->log = c->dlog;
   s->nlog = c->dlog_n;
+  s->serial = c->serial;
   return CFDL_OK;
 }
 

@@ -1,6 +1,7 @@
 // cfdl_internal.h -- shared host-side types of libcfdl_hip.so.
 #pragma once
 
+#include <atomic>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -18,6 +19,13 @@ inline int pk_elem(int p) { return static_cast<int>(static_cast<unsigned>(p) >> 
 inline int pk_face(int p) { return p & 31; }
 
 void set_error(const std::string &msg);
+
+// A number no other call returns, for objects whose identity a kept graph or
+// table is valid for: an address may be a later object's again.
+inline uint64_t next_serial() {
+  static std::atomic<uint64_t> n{0};
+  return ++n;
+}
 
 }  // namespace cfdl
 

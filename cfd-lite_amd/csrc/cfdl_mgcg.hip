@@ -994,6 +994,7 @@ struct MgSlot {
   LogLine *log;
   int *nlog;
   LogLine tmpl;
+  uint64_t serial;  // the solver's
 };
 
 template <typename T>
@@ -1098,6 +1099,7 @@ inline int nb(int n, int b) { return (n + b - 1) / b; }
 }  // namespace
 // device copy of the hierarchy and the solve's work vectors
 struct MgCgSolver {
+  const uint64_t serial = next_serial();
   int fp32 = 0, ne = 0, nbf = 0, nlev = 0, lc = 0;
   size_t coarse_lds = 0;  // LDS of the workgroup that runs levels lc ..
   std::vector<void *> mem;
@@ -1503,7 +1505,10 @@ struct MgGroup {
   int *flags = nullptr;   // device active flags
   int *hflags = nullptr;  // pinned, two sets of kMaxGroup
   hipEvent_t ev[2] = {nullptr, nullptr};
-  std::vector<char> key;  // the composition whose descriptors are on the device
+  // The composition whose descriptors are on the device, with the solvers'
+  // serial numbers: launch shapes come from their host tables (colours, sizes
+  // of levels), and a later solver may get a destroyed one's addresses.
+  std::vector<char> key;
   int launches = 0;
   ~MgGroup() {
     if (slots) (void)hipFree(slots);
@@ -1582,6 +1587,7 @@ int group_begin(MgGroup *G, MgCgSolver *const *ss, const MgCgSystem *sys, int n,
     x.lv = dev_levels<T>(s);
     x.log = sys[k].log;
     x.nlog = sys[k].nlog;
+    x.serial = s->serial;
     std::memcpy(x.tmpl.name, sys[k].name, 8);
     R.maxtop = std::max(R.maxtop, s->lc < s->nlev ? s->lc : s->nlev - 1);
     R.maxlev = std::max(R.maxlev, s->nlev);

@@ -207,3 +207,32 @@ def test_batch_graphs_equal_direct_launches_after_every_run():
     assert bd.graph_stats() == (0, 0)
     bg.close()
     bd.close()
+
+
+def test_batch_graphs_follow_a_replaced_case():
+    """A case in the place of a closed one, with the same counts but other
+    cell centres (other coarse levels, so other block counts), whose memory
+    may be the closed one's: it runs with graphs of its own.  A case that
+    leaves and joins again keeps its graphs."""
+    b = cfdl.Batch(block=256)
+    old = make_case("cavity", 24, 200.0, jitter=0.0)
+    b.attach(old)
+    b.run(1, 2)
+    first, _ = b.graph_stats()
+    b.detach(old)
+    b.attach(old)
+    b.run(1, 2)
+    assert b.graph_stats()[0] == first
+    for jitter in (0.3, 0.2):
+        b.detach(old)
+        old.close()
+        old = make_case("cavity", 24, 200.0, jitter=jitter)
+        b.attach(old)
+        before, _ = b.graph_stats()
+        b.run(1, 2)
+        assert b.graph_stats()[0] > before
+        alone = make_case("cavity", 24, 200.0, jitter=jitter)
+        alone.run(1, 2)
+        same(old, alone)
+        alone.close()
+    b.close()
