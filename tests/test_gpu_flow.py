@@ -4,6 +4,7 @@ for bit: one workgroup for all batches (no wait depends on another being
 resident), a few, more than there are batches; small and large tiles; solves
 that stop on a cap or inside a momentum iteration; two contexts at once."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -56,3 +57,18 @@ def test_two_contexts_at_once():
     for eq in eqs:
         for k, v in want.items():
             assert np.array_equal(eq.get(k), v), k
+
+
+def test_synchronising_an_idle_context_asks_the_device_nothing():
+    """The failure word of the sweeps is read from host memory: a call that
+    finds its stream idle returns without a round trip to the device (a copy
+    of one word and its synchronisation take at least 8 us)."""
+    eq = cfdl.UVWP.cavity(cfdl.Mesh.box(8).partition(2), mu=0.0025)
+    eq.run(1, 1)
+    eq.synchronize()
+    best = 1.0
+    for _ in range(500):
+        t = time.perf_counter()
+        eq.synchronize()
+        best = min(best, time.perf_counter() - t)
+    assert best < 4e-6, "%.1f us" % (best * 1e6)
