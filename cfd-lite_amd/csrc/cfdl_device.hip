@@ -149,7 +149,6 @@ struct FieldsDev {
 // state of a solve_gs call (up to 3 right-hand sides sharing ap/anb)
 struct GsCtl {
   int it[3], active[3];
-  int flow_err;  // a wait of k_gs_flow ran out of time
   double res_i[3], res_f[3], res_max[3], target[3];
 };
 
@@ -1751,8 +1750,10 @@ k_gs_tiles_lds(int batch0, const int4 *__restrict__ bdesc, const int *__restrict
 //   * No workgroup waits for a larger ticket, and each works on its tickets in
 //     increasing order, so the smallest unfinished one always runs: the waits
 //     end whatever part of the grid is resident.  They are bounded all the
-//     same (kFlowTicks): past that *err is set, every wait returns at once and
-//     the host reports the failure.
+//     same (FlowCtl::ticks): past that err is set, a workgroup takes no further
+//     ticket after a wait that sees it (a wait looks at it every 1024 polls),
+//     later launches return at once, and the host reports the failure until
+//     the context is reset.
 //   * done[b] counts batch b's finished sweeps since the solve began.  Values
 //     move between workgroups through memory (system-scope stores, agent-scope
 //     loads, which bypass the XCDs' L2s); a batch's stores are complete
@@ -1767,6 +1768,11 @@ k_gs_tiles_lds(int batch0, const int4 *__restrict__ bdesc, const int *__restrict
 // iterations, a launch per step / this kernel: 16^3 11.2 / 9.3 ms, 32^3 22.5 /
 // 18.4 ms, 61 x 47 x 53 70.5 / 53.9 ms, 64^3 63.8 / 49.3 ms, 128^3 158 / 135 ms,
 // 192^3 267 / 224 ms.
+struct FlowCtl {
+  int err;          // a wait has run out of time
+  int *host_err;    // the same in pinned host memory, which the host reads without a copy
+  long long ticks;  // a wait's limit
+};
 template <int NC>
 struct FlowArgs {
   TileSys<NC> s;
@@ -1774,14 +1780,14 @@ struct FlowArgs {
   const int *seg, *xslot;
   const unsigned short *lnbr;
   const int *dptr, *dep;  // batch b's neighbours dep[dptr[2b] .. dptr[2b+1]) earlier, .. dptr[2b+2]) later
-  int *done, *err;
-  int *host_err;  // the same in pinned host memory, which the host reads without a copy
+  int *done;
+  FlowCtl *ctl;
   unsigned *ticket;
   unsigned base;           // the counter's value before this launch
   int nb, nsweep, sweep0;  // batches; sweeps of this launch; sweeps finished before it
   int slot;                // LDS byte offset of the ticket slot (after the largest batch)
 };
-constexpr long long kFlowTicks = 2000000000LL;  // 20 s of the 100 MHz counter
+constexpr long long kTicksPerMs = 100000;  // of the 100 MHz counter
 
 __device__ inline int flow_load(const int *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1805,7 +1811,7 @@ k_gs_flow(FlowArgs<NC> A, const int *__restrict__ active, double sor, double rso
     act[c] = active[c] != 0;
     any = any || act[c];
   }
-  if (!any) return;
+  if (!any || A.ctl->err) return;
   const int tid = threadIdx.x;
   volatile unsigned *slot =
       reinterpret_cast<volatile unsigned *>(reinterpret_cast<char *>(lds) + A.slot);
@@ -1813,7 +1819,10 @@ k_gs_flow(FlowArgs<NC> A, const int *__restrict__ active, double sor, double rso
     return __hip_atomic_fetch_add(A.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) -
            A.base;
   };
-  if (tid == kLdsThreads) *slot = draw();
+  if (tid == kLdsThreads) {
+    slot[1] = 0;  // a wait of this workgroup has failed
+    *slot = draw();
+  }
   __syncthreads();
   const unsigned n = static_cast<unsigned>(A.nb) * static_cast<unsigned>(A.nsweep);
   for (unsigned t = __builtin_amdgcn_readfirstlane(*slot); t < n;
@@ -1878,11 +1887,14 @@ k_gs_flow(FlowArgs<NC> A, const int *__restrict__ active, double sor, double rso
         if ((k & 1023) == 1023) {
           const long long now = wall_clock64();
           if (start == 0) start = now;
-          if (now - start > kFlowTicks) {
-            __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(A.host_err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          if (now - start > A.ctl->ticks) {
+            __hip_atomic_store(&A.ctl->err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(A.ctl->host_err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
           }
-          if (flow_load(A.err)) break;
+          if (flow_load(&A.ctl->err)) {
+            slot[1] = 1;
+            break;
+          }
         }
         __builtin_amdgcn_s_sleep(1);
       }
@@ -1921,7 +1933,7 @@ k_gs_flow(FlowArgs<NC> A, const int *__restrict__ active, double sor, double rso
           for (int c = 0; c < NC; c++) pphi[NC * r + c] = flow_load(s.phi[c] + c0 + r);
       });
     else if (tid == kLdsThreads)
-      *slot = draw();  // the next ticket's round trip runs beside the walk
+      *slot = slot[1] ? n : draw();  // the next ticket's round trip runs beside the walk
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < NC; c++) {
@@ -2539,6 +2551,7 @@ struct cfdl_ctx {
     int flow_wgs = 0, flow_sweeps = 0;
     unsigned flow_base = 0;
   } ts, tm;
+  FlowCtl *flow = nullptr;
   // the global system in tile numbering (tiled solve_gs): new -> old cell,
   // CSR, and copies of the shared coefficients, right-hand sides and values
   bool mtiled = false;
@@ -2820,15 +2833,17 @@ static void tiled_launches(cfdl_ctx *c, const cfdl_ctx::TileSched &t, const SysD
   }
 }
 
-// Whether a wait of k_gs_flow had run out of time when the stream was last
-// synchronised; its results are invalid then, and every later call that asks
-// reports it.  The kernel writes the word to pinned memory: a copy of the
-// device's flag would add a round trip (11.9 against 0.4 us) to every call
-// that has just synchronised.
+// Whether a wait of k_gs_flow is known to have run out of time: the context's
+// values are invalid then, and every call on it reports so until
+// cfdl_ctx_reset (check_ctx; the calls that synchronise look again after it,
+// so no value of such a sweep is read without an error).  The kernel writes
+// the word to pinned memory: a copy of the device's flag would add a round
+// trip (11.9 against 0.4 us) to every call that has just synchronised.
 constexpr int kFlowFlag = 8;  // its place in host_flags
 static int flow_check(cfdl_ctx *c) {
   if (!__atomic_load_n(c->host_flags + kFlowFlag, __ATOMIC_ACQUIRE)) return CFDL_OK;
-  set_error("a Gauss-Seidel sweep waited more than 20 s for another part of its work");
+  set_error("a Gauss-Seidel sweep's wait for another part of its work ran out of time; the "
+            "context's values are invalid until cfdl_ctx_reset");
   return CFDL_EHIP;
 }
 
@@ -2853,8 +2868,7 @@ static int flow_launch(cfdl_ctx *c, cfdl_ctx::TileSched &t, const SysDesc &sys, 
   a.dptr = t.dptr;
   a.dep = t.dep;
   a.done = t.done;
-  a.err = &c->gctl->flow_err;
-  a.host_err = c->host_flags + kFlowFlag;
+  a.ctl = c->flow;
   a.ticket = t.ticket;
   a.base = t.flow_base;
   a.nb = t.nbatch;
@@ -3566,7 +3580,7 @@ static int check_ctx(cfdl_ctx *c) {
     set_error("null context");
     return CFDL_EINVAL;
   }
-  return CFDL_OK;
+  return flow_check(c);
 }
 
 // Device scratch of cfdl_calc_residual_noalloc: the block partials (2 per
@@ -4066,7 +4080,6 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
   CALL(dalloc(C, &C->red, 2 * kMaxSys));
   CALL(dalloc(C, &C->scal, 8));
   CALL(dalloc(C, &C->gctl, 1));
-  HIPCHK(hipMemset(C->gctl, 0, sizeof(GsCtl)));
   CALL(dalloc(C, &C->pctl, 1));
   CALL(dalloc(C, &C->dlog, kLogCap));
   CALL(dalloc(C, &C->dlog_n, 1));
@@ -4076,6 +4089,14 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
   }
   HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&C->host_flags), 64, hipHostMallocDefault));
   std::memset(C->host_flags, 0, 64);
+  {
+    // CFDL_FLOW_WAIT_MS: the limit of a wait; 0: its first look at the clock
+    const char *fw = std::getenv("CFDL_FLOW_WAIT_MS");
+    const long long ms = fw ? std::atoll(fw) : 20000;
+    const FlowCtl f{0, C->host_flags + kFlowFlag, ms > 0 ? ms * kTicksPerMs : -1};
+    CALL(dalloc(C, &C->flow, 1));
+    HIPCHK(hipMemcpy(C->flow, &f, sizeof(f), hipMemcpyHostToDevice));
+  }
   HIPCHK(hipStreamSynchronize(C->st));
   trace("ctx_create: done");
   *out = c.release();
@@ -4391,7 +4412,7 @@ int cfdl_synchronize(cfdl_ctx *c) {
 }
 
 int cfdl_ctx_reset(cfdl_ctx *c) {
-  CALL(check_ctx(c));
+  if (!c) return check_ctx(c);
   for (int f = 0; f < CFDL_NFIELDS; f++)
     hipLaunchKernelGGL(k_fill, dim3(nblocks(c->fsize[f])), dim3(kBlock), 0, c->st, c->fields[f],
                        c->fsize[f], 0.0);
@@ -4401,6 +4422,10 @@ int cfdl_ctx_reset(cfdl_ctx *c) {
   HIPCHK(hipStreamSynchronize(c->st));
   const int zero = 0;
   HIPCHK(hipMemcpy(c->dlog_n, &zero, sizeof(int), hipMemcpyHostToDevice));
+  if (flow_check(c) != CFDL_OK) {  // the values that a failed sweep left are gone
+    HIPCHK(hipMemcpy(&c->flow->err, &zero, sizeof(int), hipMemcpyHostToDevice));
+    c->host_flags[kFlowFlag] = 0;
+  }
   c->hlog.clear();
   c->outer = 0;
   return CFDL_OK;
@@ -4804,6 +4829,7 @@ int cfdl_set_profile(cfdl_ctx *c, int sample_every) {
 int cfdl_stats(cfdl_ctx *c, double *stats, int n) {
   CALL(check_ctx(c));
   HIPCHK(hipStreamSynchronize(c->st));
+  CALL(flow_check(c));
   double ms = 0.0, cells = 0.0, nl = 0.0;
   for (size_t k = 0; k < c->nsamples; k++) {
     float t = 0.f;
@@ -4950,6 +4976,7 @@ int batch_check(cfdl_batch *b, cfdl_ctx *c) {
     set_error("cfdl_batch: the case is on another device");
     return CFDL_EINVAL;
   }
+  CALL(flow_check(c));
   if (!c->mhex) {
     set_error("cfdl_batch: cases need hexahedral rows (six entries each)");
     return CFDL_ESTATE;

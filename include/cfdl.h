@@ -19,7 +19,11 @@
  *
  * Threading: one context = one HIP stream = one calling thread.  Calls on a
  * context are asynchronous with respect to the host except where stated;
- * cfdl_get_field and the log read-out synchronise.
+ * cfdl_get_field and the log read-out synchronise.  A Gauss-Seidel sweep in
+ * the reference order waits inside a launch for its other parts, at most 20 s
+ * each time; if a wait runs out, the calls that synchronise and every call
+ * after them return CFDL_EHIP (no values of such a sweep are returned) until
+ * cfdl_ctx_reset, which makes the context usable again.
  */
 #ifndef CFDL_H
 #define CFDL_H

@@ -72,3 +72,42 @@ def test_synchronising_an_idle_context_asks_the_device_nothing():
         eq.synchronize()
         best = min(best, time.perf_counter() - t)
     assert best < 4e-6, "%.1f us" % (best * 1e6)
+
+
+@pytest.mark.parametrize("solve", ["uvw", "pc"])
+def test_expired_wait_is_reported_until_reset(monkeypatch, solve):
+    """A limit of zero lets the first wait of 1024 polls run out: a column of
+    2 x 2 cells cut into 4000 batches, each waiting for the one before it (several
+    us), with a workgroup for every batch.  The launch ends, every call that
+    could hand out its values fails, and so do the calls after them, until a
+    reset; then the context works as a new one (in an order that has no
+    waits, as the limit stays)."""
+    mesh = cfdl.Mesh.box(2, 2, 8000).partition(2)
+    fresh = cfdl.UVWP.cavity(mesh, mu=0.0025)
+    for key, value in (("FLOW_WAIT_MS", "0"), ("TILE", "2x2x2"), ("FLOW", "4000")):
+        monkeypatch.setenv("CFDL_" + key, value)
+    eq = cfdl.UVWP.cavity(mesh, mu=0.0025)
+    if solve == "pc":
+        eq.set_gs_order("colored")
+        try:
+            eq.run(1, 1)  # queues the sweeps; may already see that one failed
+        except cfdl.CfdlError:
+            pass
+    else:
+        with pytest.raises(cfdl.CfdlError, match="ran out of time"):
+            eq.run(1, 1)
+    for call in (eq.synchronize, lambda: eq.get("phic"), eq.log, eq.stats, lambda: eq.run(1, 1),
+                 lambda: eq.solve("pc"), eq.solve_uvwp, lambda: eq.set_pc_order("colored")):
+        with pytest.raises(cfdl.CfdlError, match="ran out of time"):
+            call()
+    eq.reset()
+    for s in (eq, fresh):
+        s.set_gs_order("colored")
+        s.set_pc_order("colored")
+        s.run(1, 2)
+    for name in ("u", "v", "w", "p", "mip", "gp", "phic"):
+        assert np.array_equal(eq.get(name), fresh.get(name)), name
+    assert eq.log() == fresh.log()
+    eq.set_gs_order("reference")
+    with pytest.raises(cfdl.CfdlError, match="ran out of time"):
+        eq.run(1, 1)  # the limit still holds
