@@ -34,9 +34,9 @@ from .solver import UVWP, Batch
 
 # Device footprint of one context: mesh, fields, the momentum system in
 # colour numbering, the multigrid hierarchy, the faces' fixed geometry and
-# the FP32 copies; about 64 MiB plus 1.8 KB per cell.
+# the FP32 copies; at most 64 MiB plus 1.3 KB per cell (tests/test_gpu_footprint.py).
 BYTES_PER_CONTEXT = 64 << 20
-BYTES_PER_CELL = 1760
+BYTES_PER_CELL = 1344
 KINDS = ("cavity", "channel")
 
 

@@ -104,13 +104,14 @@ struct MeshDev {
   const double *cp, *tc;  // thermal properties of the energy equation
   // FP32 copies of the geometry and properties for the FP32 assembly (null
   // until cfdl_set_assembly_precision selects it)
-  const float *xc32, *yc32, *zc32, *vol32, *aip32, *rip32, *rho32, *mu32;
+  const float *xc32, *yc32, *zc32, *vol32, *rho32, *mu32;
   // per interior face, what the assembly and the flux correction need of its
   // fixed geometry (k_face_geo): fa = area, weight of the neighbour seen from
-  // the owner and from the other cell, (r_nb - r_P).n; fd = |r_nb - r_P|, the
-  // distance of the two cells' feet on the face normal, and the vector
-  // between the feet (owner to other).  FP32 copies computed from the FP32
-  // geometry.
+  // the owner and from the other cell, (r_nb - r_P).n; fd = the vector between
+  // the two cells' feet on the face normal (owner to other).  FP32 versions
+  // from the FP32 geometry.  fd serves the assembly alone, so a context holds
+  // the one of its precision (72 or 36 B a cell); fa in FP64 the flux
+  // correction too.
   const double *fa, *fd;
   const float *fa32, *fd32;
 };
@@ -118,18 +119,17 @@ struct MeshDev {
 // the geometry of the arithmetic type T: the mesh's FP64 arrays, or their
 // FP32 copies
 struct Geo64 {
-  const double *xc, *yc, *zc, *vol, *aip, *rip, *rho, *mu, *fa, *fd;
+  const double *xc, *yc, *zc, *vol, *rho, *mu, *fa, *fd;
 };
 struct Geo32 {
-  const float *xc, *yc, *zc, *vol, *aip, *rip, *rho, *mu, *fa, *fd;
+  const float *xc, *yc, *zc, *vol, *rho, *mu, *fa, *fd;
 };
 template <typename T>
 __device__ inline auto geo_of(const MeshDev &m) {
   if constexpr (sizeof(T) == 8)
-    return Geo64{m.xc, m.yc, m.zc, m.vol, m.aip, m.rip, m.rho, m.mu, m.fa, m.fd};
+    return Geo64{m.xc, m.yc, m.zc, m.vol, m.rho, m.mu, m.fa, m.fd};
   else
-    return Geo32{m.xc32, m.yc32, m.zc32, m.vol32, m.aip32, m.rip32, m.rho32, m.mu32,
-                 m.fa32, m.fd32};
+    return Geo32{m.xc32, m.yc32, m.zc32, m.vol32, m.rho32, m.mu32, m.fa32, m.fd32};
 }
 
 // energy equation state (energy_t, mod_energy.f90:4-10): temperature t and
@@ -264,7 +264,11 @@ __global__ void k_face_geo(MeshDev m, T *fa, T *fd) {
   if (fg >= m.nf) return;
   const int e = m.fcell[fg], nb = m.nbr[m.own[fg]];
   if (nb >= m.ne) return;
-  const T *a = G.aip + 3 * fg, *rip = G.rip + 3 * fg;
+  T a[3], rip[3];
+  for (int i = 0; i < 3; i++) {
+    a[i] = static_cast<T>(m.aip[3 * fg + i]);
+    rip[i] = static_cast<T>(m.rip[3 * fg + i]);
+  }
   const T area = area_of(a);
   const T rp[3] = {G.xc[e], G.yc[e], G.zc[e]}, rpnb[3] = {G.xc[nb], G.yc[nb], G.zc[nb]};
   T nrm[3], dr[3], drip[3], rpp[3], rnp[3], drp[3];
@@ -281,9 +285,8 @@ __global__ void k_face_geo(MeshDev m, T *fa, T *fd) {
   fa[4 * fg + 1] = vec_weight(rip, rp, rpnb);
   fa[4 * fg + 2] = vec_weight(rip, rpnb, rp);
   fa[4 * fg + 3] = dot3(dr, nrm);
-  fd[5 * fg] = sqrt(dot3(dr, dr));
-  fd[5 * fg + 1] = sqrt(dot3(drp, drp));
-  for (int i = 0; i < 3; i++) fd[5 * fg + 2 + i] = drp[i];
+  if (fd)
+    for (int i = 0; i < 3; i++) fd[3 * fg + i] = drp[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -574,13 +577,14 @@ __device__ inline void d_coef_uvw6(int bx_, const MeshDev &m, const FieldsDev &f
     T d = zero, fnb = zero;
     if (nb < m.ne) {
       const T sg = fs >= 0 ? one : -one;
-      const T *fa = G.fa + 4 * fg, *fd = G.fd + 5 * fg;
-      const T area = fa[0], wt = fs >= 0 ? fa[1] : fa[2], ds = fd[0], dsp = fd[1];
+      const T *fa = G.fa + 4 * fg, *fd = G.fd + 3 * fg;
+      const T area = fa[0], wt = fs >= 0 ? fa[1] : fa[2];
       const T rpnb[3] = {G.xc[nb], G.yc[nb], G.zc[nb]};
       T dr[3], drp[3];
       for (int i = 0; i < 3; i++) dr[i] = rpnb[i] - rp[i];
       // 0 - x and not -x: from the other side a zero is +0 too
-      for (int i = 0; i < 3; i++) drp[i] = fs >= 0 ? fd[2 + i] : zero - fd[2 + i];
+      for (int i = 0; i < 3; i++) drp[i] = fs >= 0 ? fd[i] : zero - fd[i];
+      const T ds = sqrt(dot3(dr, dr)), dsp = sqrt(dot3(drp, drp));
       const T fl = -(sg * ld(f.mip[fg]));
       fnb = fmax(fl, zero);
       sumf = sumf + fl;
@@ -618,7 +622,7 @@ __device__ inline void d_coef_uvw6(int bx_, const MeshDev &m, const FieldsDev &f
   for (int q = m.bcrow[e]; q < m.bcrow[e + 1]; q++) {
     const int k = m.bcslot[q], H = m.nbr[k];
     const int fg = m.fsg[k] - 1;  // boundary faces are always owner side
-    const T *a = G.aip + 3 * fg;
+    const T a[3] = {ld(m.aip[3 * fg]), ld(m.aip[3 * fg + 1]), ld(m.aip[3 * fg + 2])};
     const T area = area_of(a);
     const T nrm[3] = {a[0] / area, a[1] / area, a[2] / area};
     const T dr[3] = {G.xc[H] - rp[0], G.yc[H] - rp[1], G.zc[H] - rp[2]};
@@ -2469,6 +2473,8 @@ struct Sched {
 
 struct DevBuf {
   std::vector<void *> ptrs;
+  char *slab = nullptr;  // the rest of the last reserve()
+  size_t left = 0;
   ~DevBuf() {
     for (void *p : ptrs) (void)hipFree(p);
   }
@@ -2591,16 +2597,40 @@ struct cfdl_ctx {
   size_t nsamples = 0;
 };
 
+static int dev_malloc(void **q, size_t bytes) {
+  const hipError_t e = hipMalloc(q, bytes);
+  if (e == hipSuccess) return CFDL_OK;
+  set_error(std::string("hipMalloc of ") + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
+  return CFDL_ENOMEM;
+}
+// One allocation for the arrays that the next dallocs ask for, bytes[i] each.
+// An allocation of some MB takes whole 2 MiB pages: with one per array a
+// context of a 96^3 mesh held 96 MiB that it could not use.
+static size_t slab_bytes(int64_t bytes) {
+  return (static_cast<size_t>(bytes > 0 ? bytes : 1) + 255) & ~size_t{255};
+}
+static int reserve(cfdl_ctx *c, std::initializer_list<int64_t> bytes) {
+  size_t sum = 0;
+  for (int64_t b : bytes) sum += slab_bytes(b);
+  void *q = nullptr;
+  CALL(dev_malloc(&q, sum));
+  c->mem.ptrs.push_back(q);
+  c->mem.slab = static_cast<char *>(q);
+  c->mem.left = sum;
+  return CFDL_OK;
+}
 template <typename T>
 static int dalloc(cfdl_ctx *c, T **p, int64_t n) {
   void *q = nullptr;
   const size_t bytes = sizeof(T) * static_cast<size_t>(n > 0 ? n : 1);
-  hipError_t e = hipMalloc(&q, bytes);
-  if (e != hipSuccess) {
-    set_error(std::string("hipMalloc of ") + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
-    return CFDL_ENOMEM;
+  if (slab_bytes(bytes) <= c->mem.left) {
+    q = c->mem.slab;
+    c->mem.slab += slab_bytes(bytes);
+    c->mem.left -= slab_bytes(bytes);
+  } else {
+    CALL(dev_malloc(&q, bytes));
+    c->mem.ptrs.push_back(q);
   }
-  c->mem.ptrs.push_back(q);
   *p = static_cast<T *>(q);
   return CFDL_OK;
 }
@@ -2613,6 +2643,29 @@ static int upload(cfdl_ctx *c, T **p, const std::vector<T> &v) {
 }
 
 static inline int nblocks(int64_t n) { return static_cast<int>((n + kBlock - 1) / kBlock); }
+
+// fa, and the FP64 assembly's fd if it is not there (rows of six entries only)
+static int face_geo64(cfdl_ctx *c) {
+  if (c->md.fd) return CFDL_OK;
+  void *fd = nullptr;
+  if (c->mhex) {
+    CALL(dev_malloc(&fd, 24 * size_t(std::max(c->nf, 1))));
+    c->mem.ptrs.push_back(fd);
+  }
+  hipLaunchKernelGGL(k_face_geo<double>, dim3(nblocks(c->nf)), dim3(kBlock), 0, c->st, c->md,
+                     const_cast<double *>(c->md.fa), static_cast<double *>(fd));
+  c->md.fd = static_cast<double *>(fd);
+  HIPCHK(hipGetLastError());
+  return CFDL_OK;
+}
+static void face_geo64_drop(cfdl_ctx *c) {
+  if (!c->md.fd) return;
+  (void)hipStreamSynchronize(c->st);
+  void *fd = const_cast<double *>(c->md.fd);
+  c->mem.ptrs.erase(std::find(c->mem.ptrs.begin(), c->mem.ptrs.end(), fd));
+  (void)hipFree(fd);
+  c->md.fd = nullptr;
+}
 
 // Dependency levels of a sweep over cells [beg, end) in increasing (fwd) or
 // decreasing (bwd) order: a cell waits for neighbours in the same range that
@@ -3720,6 +3773,10 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
   }
   trace("ctx_create: host tables");
   cfdl_ctx *C = c.get();
+  const int64_t e4 = 4 * int64_t{ne}, e8 = 2 * e4, f4 = 4 * int64_t{nf}, h4 = 4 * int64_t{nbf},
+                L4 = 4 * int64_t{L}, n8 = 8 * int64_t{n};  // bytes
+  CALL(reserve(C, {e4 + 4, L4, L4, f4, f4, e4 + 4, h4, h4, h4, h4, h4, h4, n8, n8, n8, e8, 6 * f4,
+                   6 * f4, e8, e8, e8, e8, 8 * f4}));
   int *d_row, *d_nbr, *d_fsg, *d_own, *d_fcell, *d_bcrow, *d_bcslot, *d_hcell, *d_hslot, *d_hkind;
   CALL(upload(C, &d_row, row));
   CALL(upload(C, &d_nbr, nbr));
@@ -3763,12 +3820,10 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
                   d_hcell, d_hslot, d_hkind, d_xc, d_yc, d_zc, d_vol, d_aip, d_rip, d_rho, d_mu,
                   d_cp, d_tc};
   {
-    double *fa, *fd;
+    double *fa;
     CALL(dalloc(C, &fa, 4 * int64_t{nf}));
-    CALL(dalloc(C, &fd, 5 * int64_t{nf}));
-    hipLaunchKernelGGL(k_face_geo<double>, dim3(nblocks(nf)), dim3(kBlock), 0, C->st, C->md, fa, fd);
-    HIPCHK(hipGetLastError());
-    C->md.fa = fa, C->md.fd = fd;
+    C->md.fa = fa;
+    CALL(face_geo64(C));
   }
   trace("ctx_create: mesh uploaded");
   // --- fields ---
@@ -3776,6 +3831,9 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
                                     3 * int64_t{n}, 3 * int64_t{n}, 3 * int64_t{n}, nf, nf, ne,
                                     ne, ne, ne, ne, ne, ne, L, n, n, 3 * int64_t{n},
                                     n, 3 * int64_t{n}, n, n, 3 * int64_t{n}};
+  int64_t fbytes = 0;
+  for (int64_t k : sz) fbytes += slab_bytes(8 * k);
+  CALL(reserve(C, {fbytes}));
   for (int f = 0; f < CFDL_NFIELDS; f++) {
     C->fsize[f] = sz[f];
     CALL(dalloc(C, &C->fields[f], sz[f]));
@@ -3817,7 +3875,6 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
   {
     std::vector<int> lev(ne);
     levels(row, nbr, 0, ne, true, lev);
-    CALL(make_sched(C, lev, ne, &C->gf));
     if (C->tiled) {
       // the global system in tile numbering, for the tiled solve_gs
       std::vector<int> all(ne), grp{0, ne}, tid, launch;
@@ -3843,6 +3900,7 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
       CALL(build_tile_tables(C, rowm, nbrm, zero, launchm, tidm, levm, 3, &C->tm));
       C->mtiled = C->tm.lds_bytes > 0;
       if (C->mtiled) {
+        CALL(reserve(C, {e4, e4 + 4, L4, e8, e8, 2 * L4, e8, n8, e8, n8, e8, n8}));
         CALL(upload(C, &C->l2g_m, n2o));
         CALL(upload(C, &C->rowm, rowm));
         CALL(upload(C, &C->nbrm, nbrm));
@@ -3855,8 +3913,11 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
         }
       }
     }
-    levels(row, nbr, 0, ne, false, lev);
-    CALL(make_sched(C, lev, ne, &C->gb));
+    if (!C->mtiled) {  // one launch per level
+      CALL(make_sched(C, lev, ne, &C->gf));
+      levels(row, nbr, 0, ne, false, lev);
+      CALL(make_sched(C, lev, ne, &C->gb));
+    }
     // colour order of solve_gs: greedy colouring in global order (a cell
     // takes the least colour none of its earlier interior neighbours has),
     // cells renumbered by (colour, global order)
@@ -3887,6 +3948,7 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
         rowc[i + 1] = rowc[i] + (row[g + 1] - row[g]);
         for (int k = row[g]; k < row[g + 1]; k++) nbrc.push_back(nbr[k] < ne ? o2n[nbr[k]] : nbr[k]);
       }
+      CALL(reserve(C, {e4, e4 + 4, L4}));
       CALL(upload(C, &C->l2g_gc, n2o));
       CALL(upload(C, &C->rowgc, rowc));
       CALL(upload(C, &C->nbrgc, nbrc));
@@ -4278,28 +4340,35 @@ int cfdl_set_assembly_precision(cfdl_ctx *c, int bits) {
   }
   if (bits == 32 && !c->md.xc32) {
     // FP32 copies of the geometry and properties (properties are re-copied
-    // by cfdl_set_properties)
+    // by cfdl_set_properties), in the place of the FP64 assembly's fd
     const int n = c->ne + c->nbf;
-    float *p[8];
-    const double *src[8] = {c->md.xc, c->md.yc, c->md.zc, c->md.vol, c->md.aip, c->md.rip,
-                            c->md.rho, c->md.mu};
-    const int64_t cnt[8] = {n, n, n, c->ne, 3 * int64_t{c->nf}, 3 * int64_t{c->nf}, c->ne, c->ne};
-    for (int i = 0; i < 8; i++) {
+    float *p[6];
+    const double *src[6] = {c->md.xc, c->md.yc, c->md.zc, c->md.vol, c->md.rho, c->md.mu};
+    const int64_t cnt[6] = {n, n, n, c->ne, c->ne, c->ne}, n4 = 4 * int64_t{n},
+                  e4 = 4 * int64_t{c->ne}, f4 = 4 * int64_t{c->nf};
+    face_geo64_drop(c);
+    if (const int rc = reserve(c, {n4, n4, n4, e4, e4, e4, 4 * f4, 3 * f4})) {
+      (void)face_geo64(c);
+      return rc;
+    }
+    for (int i = 0; i < 6; i++) {
       CALL(dalloc(c, &p[i], cnt[i]));
       hipLaunchKernelGGL(k_to_f32, dim3(std::min<int64_t>((cnt[i] + kBlock - 1) / kBlock, 65535)),
                          dim3(kBlock), 0, c->st, src[i], p[i], cnt[i]);
     }
     HIPCHK(hipGetLastError());
     c->md.xc32 = p[0], c->md.yc32 = p[1], c->md.zc32 = p[2], c->md.vol32 = p[3];
-    c->md.aip32 = p[4], c->md.rip32 = p[5], c->md.rho32 = p[6], c->md.mu32 = p[7];
+    c->md.rho32 = p[4], c->md.mu32 = p[5];
     float *fa, *fd;
     CALL(dalloc(c, &fa, 4 * int64_t{c->nf}));
-    CALL(dalloc(c, &fd, 5 * int64_t{c->nf}));
+    CALL(dalloc(c, &fd, 3 * int64_t{c->nf}));
     hipLaunchKernelGGL(k_face_geo<float>, dim3(nblocks(c->nf)), dim3(kBlock), 0, c->st, c->md, fa,
                        fd);
     HIPCHK(hipGetLastError());
     c->md.fa32 = fa, c->md.fd32 = fd;
   }
+  if (bits == 64) CALL(face_geo64(c));
+  if (bits == 32) face_geo64_drop(c);
   c->asm32 = bits == 32;
   return CFDL_OK;
 }
