@@ -3306,10 +3306,12 @@ static double tile_launches(int ne, const std::vector<int> &row, const std::vect
   int ntile = 1;
   for (int e = 0; e < ne; e++) ntile = std::max(ntile, tid[e] + 1);
   struct Batch {
-    int first = -1, last = -1;  // levels
+    int launch, first, last = -1;  // last: level
     int cells = 0, levels = 0, seg = 0, segmax = 0;
   };
-  std::vector<std::vector<Batch>> bat(ntile);  // per tile, by launch
+  // per tile, its batches by launch (those that exist: a chain of n tiles has n
+  // launches and one batch a tile)
+  std::vector<std::vector<Batch>> bat(ntile);
   launch->assign(ne, 0);
   int nl = 0;
   for (int e : order) {
@@ -3320,13 +3322,14 @@ static double tile_launches(int ne, const std::vector<int> &row, const std::vect
       L = std::max(L, (*launch)[d] + (tid[d] != tid[e] ? 1 : 0));
     }
     std::vector<Batch> &tb = bat[tid[e]];
-    for (;; L++) {
-      if (static_cast<int>(tb.size()) <= L) tb.resize(L + 1);
-      if (tb[L].first < 0) tb[L].first = lev[e];
-      if (lev[e] - tb[L].first < span) break;
+    auto it = std::lower_bound(tb.begin(), tb.end(), L,
+                               [](const Batch &x, int l) { return x.launch < l; });
+    for (;; L++, ++it) {
+      if (it == tb.end() || it->launch != L) it = tb.insert(it, Batch{L, lev[e]});
+      if (lev[e] - it->first < span) break;
     }
     (*launch)[e] = L;
-    Batch &b = tb[L];
+    Batch &b = *it;
     if (lev[e] != b.last) b.levels++, b.seg = 0;
     b.last = lev[e];
     b.cells++;
@@ -3336,13 +3339,12 @@ static double tile_launches(int ne, const std::vector<int> &row, const std::vect
   std::vector<int> nb(nl, 0), longest(nl, 0);
   int cells = 1, seg = 0;
   for (const auto &tb : bat)
-    for (size_t L = 0; L < tb.size(); L++)
-      if (tb[L].cells > 0) {
-        nb[L]++;
-        longest[L] = std::max(longest[L], tb[L].levels);
-        cells = std::max(cells, tb[L].cells);
-        seg = std::max(seg, tb[L].segmax);
-      }
+    for (const Batch &x : tb) {
+      nb[x.launch]++;
+      longest[x.launch] = std::max(longest[x.launch], x.levels);
+      cells = std::max(cells, x.cells);
+      seg = std::max(seg, x.segmax);
+    }
   // LDS of a batch cell: coefficients, addresses, values and right-hand sides,
   // and about 0.7 outside neighbours
   const double fit = 160.0 * 1024 / (80 + 21.6 * nrhs) / cells;

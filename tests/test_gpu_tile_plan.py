@@ -1,9 +1,14 @@
 """The tile shape and layer-aligned cuts the sweep schedules are planned with,
 against the oracle bit for bit: uneven and one-layer boxes, distorted cells,
 more layers than a tile holds, edges one past a tile's, a mesh whose layers
-are no planes (three blocks around an edge)."""
+are no planes (three blocks around an edge); the host memory planning takes."""
+import os
+import subprocess
+import sys
+
 import pytest
 
+import cfdl
 import meshgen
 from test_gpu_colour_turns import pair, three_blocks
 from test_gpu_parity import assert_fields_equal, assert_logs_match
@@ -29,3 +34,27 @@ def test_three_blocks_bitwise(nsubd):
     oc.run(1, 2)
     assert_fields_equal(eq, oc)
     assert_logs_match(eq.log(), oc.log())
+
+
+PLAN_MEMORY = """
+import resource, sys
+sys.path.insert(0, sys.argv[1])
+import cfdl
+peak = lambda: resource.getrusage(resource.RUSAGE_SELF).ru_maxrss / 1024.0  # MiB
+cfdl.UVWP.cavity(cfdl.Mesh.box(8).partition(2), mu=0.01).run(1, 1)
+mesh = cfdl.Mesh.box(1, 1, 40000).partition(2)
+before = peak()
+eq = cfdl.UVWP.cavity(mesh, mu=0.01)
+print("growth", peak() - before)
+"""
+
+
+def test_planning_memory_follows_the_batches():
+    """A column of 40,000 cells is a chain of 10,000 tiles and as many steps;
+    a table of every tile's every step is 1.2 GB a shape, the batches that
+    exist are a few MB (64 MiB covers them and the context's own copies)."""
+    out = subprocess.run([sys.executable, "-c", PLAN_MEMORY, os.path.dirname(cfdl.__path__[0])],
+                         capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr[-2000:]
+    growth = float(out.stdout.split("growth")[1])
+    assert growth < 64.0, "%.0f MiB" % growth
