@@ -3,6 +3,7 @@
 for bit: one workgroup for all batches (no wait depends on another being
 resident), a few, more than there are batches; small and large tiles; solves
 that stop on a cap or inside a momentum iteration; two contexts at once."""
+import ctypes as C
 import threading
 import time
 
@@ -11,6 +12,7 @@ import pytest
 
 import cfdl
 import meshgen
+import oracle_lib
 from test_gpu_colour_turns import pair
 from test_gpu_parity import assert_fields_equal, assert_logs_match
 
@@ -39,6 +41,75 @@ def test_shapes_and_caps_bitwise(monkeypatch, tile, span, nit):
     oc.run(1, 2)
     assert_fields_equal(eq, oc, ["u", "v", "w", "p", "mip", "gp", "phic"])
     assert_logs_match(eq.log(), oc.log())
+
+
+def shuffled_pair(n, seed, shuffle):
+    """A box whose cells are numbered at random, and its oracle; with shuffle
+    the context is given the cells' centres in another order, so that a
+    sweep's tiles are groups of cells from all over the mesh."""
+    g = meshgen.box_mesh(n)
+    rng = np.random.default_rng(seed)
+    ne = g["ne"]
+    cells = np.array(g["e2vx"]).reshape(-1, 8)
+    cells[:ne] = cells[:ne][rng.permutation(ne)]
+    g["e2vx"] = cells.reshape(-1)
+    m = cfdl.Mesh.from_elements(g["x"], g["y"], g["z"], g["etype"], g["esec"], g["e2vx"],
+                                names=g["names"]).partition(2)
+    i, bc = m.info(), meshgen.cavity_bc(g)
+    oc = oracle_lib.OracleCase(g, bc, nsubd=2)
+    xyz = [m.get(k) for k in ("xc", "yc", "zc")]
+    order = rng.permutation(ne)
+    if shuffle:
+        for a in xyz:
+            a[:ne] = a[:ne][order]
+    eq = cfdl.UVWP.from_arrays(
+        i["ne"], i["nf"], i["nbf"], *[m.get(k) for k in ("ef2nb_idx", "ef2nb", "s2g", "bs")], *xyz,
+        *[m.get(k) for k in ("vol", "aip", "rip", "esec")], bc, 2,
+        *[m.get(k) for k in ("gf2g", "g2gf", "g2gf_idx")], np.ones(ne), np.full(ne, 0.01), 0.01)
+    return eq, oc, rng
+
+
+@pytest.mark.parametrize("shuffle", [False, True])
+def test_batches_with_many_neighbours_run_step_by_step(shuffle):
+    """The waiting wavefront has a lane per neighbouring batch: a schedule
+    with 64 or more on one side (random tiles: up to 127 for u, v, w and 99
+    in the pc system, in segments of at most 54 cells) runs a launch a step,
+    without being told to; the same cells in tiles of neighbours run in one
+    launch an iteration or block.  Both give the oracle's bits."""
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setenv("CFDL_TILE", "1" if shuffle else "4")
+        eq, oc, rng = shuffled_pair(13, 3, shuffle)
+    ne, idx = oc.c.ne, oc.arr("ef2nb_idx") - 1
+    anb = rng.uniform(0.5, 1.0, idx[-1])
+    ap = np.add.reduceat(anb, idx[:-1]) + 0.5
+    for s in (eq, oc):
+        put = eq.set if s is eq else lambda k, v: oc.arr(k).__setitem__(slice(None), v)
+        put("anb", anb)
+        put("ap", ap)
+    rhs = {k: rng.uniform(-1.0, 1.0, ne) for k in ("bu", "bv", "bw", "b")}
+    for k, v in rhs.items():
+        eq.set(k, v)
+        oc.arr(k)[:] = v
+    for k in ("u", "v", "w", "phic"):
+        eq.set_a_0(k)
+        oc.arr(k)[:] = 0.0
+    eq.solve_gs_uvw()
+    momentum = eq.stats()["gs_launches"]
+    iterations = max(line[1] for line in eq.log())
+    eq.reset_stats()
+    eq.solve("pc")
+    pc = eq.stats()["pc_launches"]
+    assert iterations >= 2
+    assert (momentum > 2 * iterations and pc > 100) if shuffle else (momentum == iterations and pc == 50)
+    L, c = oracle_lib.lib(), oc.c
+    L.or_solve_gs.argtypes = [C.POINTER(oracle_lib.OrCase), C.c_char_p, oracle_lib.PD, oracle_lib.PD,
+                              oracle_lib.PD, oracle_lib.PD, oracle_lib.PI, oracle_lib.PI,
+                              C.c_int, C.c_int, C.c_int, C.c_int]
+    for phi, b in (("u", "bu"), ("v", "bv"), ("w", "bw")):
+        L.or_solve_gs(oc.p, phi.encode(), getattr(c, phi), c.ap, c.anb, getattr(c, b),
+                      c.ef2nb_idx, c.ef2nb, c.ne, c.nf, c.nbf, c.nit)
+    L.or_solve(oc.p, b"pc", c.phic)
+    assert_fields_equal(eq, oc, ["u", "v", "w", "phic"])
 
 
 def test_two_contexts_at_once():

@@ -150,9 +150,9 @@ def test_set_section_bc_rejects_bad_input():
 def test_64cube_jittered_relaxed_bitwise():
     """A 64^3 box with interior vertices jittered by up to 0.2 h, Re = 400 and
     the 0.7/0.3 relaxation of the 128^3 benchmark, two outer iterations.  At
-    this size the pressure-correction sweeps run full 16 x 8 x 4 tiles with
-    32-level batches, and the momentum sweeps their own tiles; every field
-    equals the oracle's bits."""
+    this size the tiles of the pressure-correction sweeps are full ones of
+    the planned shape, and so are the momentum sweeps'; every field equals
+    the oracle's bits."""
     eq, oc = make_pair(64, 0.2, 4, mu=0.0025)
     eq.set_relaxation(0.7, 0.3)
     oc.set_relaxation(0.7, 0.3)
@@ -292,6 +292,15 @@ def test_set_get_roundtrip_and_errors():
         eq.set_relaxation(0.0, 1.0)
 
 
+def _flow(monkeypatch, flow):
+    """Sweeps in one launch whose batches wait for each other (the default
+    where batches take the pipelined walk by four wavefronts), or launched
+    step by step."""
+    if flow == "steps":
+        monkeypatch.setenv("CFDL_FLOW", "0")
+
+
+@pytest.mark.parametrize("flow", ["flow", "steps"])
 @pytest.mark.parametrize("tile,mode,lds,span,pipe,waves", [
     ("2", "tiled", "1", "16", "1", "4"), ("3", "tiled", "1", "3", "1", "4"),
     ("3", "tiled", "0", "16", "1", "4"), ("8", "tiled", "1", "16", "1", "4"),
@@ -300,14 +309,17 @@ def test_set_get_roundtrip_and_errors():
     ("16x8x4", "tiled", "1", "28", "1", "4"), ("8", "tiled", "1", "16", "1", "1"),
     ("8", "tiled", "1", "16", "0", "1"), ("12", "tiled", "1", "32", "1", "1"),
     ("16x8x4", "tiled", "1", "28", "1", "1"), ("12", "tiled", "1", "63", "1", "4")])
-def test_sweep_schedules_bitwise(monkeypatch, tile, mode, lds, span, pipe, waves):
+def test_sweep_schedules_bitwise(monkeypatch, tile, mode, lds, span, pipe, waves, flow):
     """The pressure-correction sweeps run as one launch per dependency level
-    or as space-time tiles launched batch by batch (in LDS, or from global
-    memory with CFDL_TILE_LDS=0).  In LDS, level segments of at most 64 cells
-    take the register-pipelined walk unless CFDL_TILE_PIPE=0, and a batch is
-    gathered and written back by four wavefronts (whose idle three prefetch
-    the next launch's batches during the walk), or by one with
-    CFDL_TILE_WAVES=1.  Small tiles and spans put many tile boundaries into
+    or as space-time tiles: in LDS, or from global memory with
+    CFDL_TILE_LDS=0.  In LDS, level segments of at most 64 cells take the
+    register-pipelined walk unless CFDL_TILE_PIPE=0, and a batch is gathered
+    and written back by four wavefronts, or by one with CFDL_TILE_WAVES=1.
+    With the walk and four wavefronts the sweeps of a block are one launch
+    whose batches wait for their neighbours, or with CFDL_FLOW=0 a launch a
+    step, where the idle three wavefronts prefetch the next launch's batches
+    during the walk; the other schedules are launched step by step anyway.
+    Small tiles and spans put many tile boundaries into
     small meshes; tile 12 with span 32 needs more than 64 KB of LDS per batch
     and has wider segments, and with span 63 a batch holds a subdomain's
     whole sweep (the walk's most segments); tiles may have a different edge
@@ -318,6 +330,7 @@ def test_sweep_schedules_bitwise(monkeypatch, tile, mode, lds, span, pipe, waves
     monkeypatch.setenv("CFDL_TILE_SPAN", span)
     monkeypatch.setenv("CFDL_TILE_PIPE", pipe)
     monkeypatch.setenv("CFDL_TILE_WAVES", waves)
+    _flow(monkeypatch, flow)
     eq, oc = make_pair(12, 0.15, 4)
     eq.run(1, 2)
     oc.run(1, 2)
@@ -351,8 +364,9 @@ def _tiny_rows(oc, rows, names, seed):
             oc.arr(name)[r] = np.ldexp(1.0 + rng.random(), -1000 - int(rng.integers(61)))
 
 
+@pytest.mark.parametrize("flow", ["flow", "steps"])
 @pytest.mark.parametrize("case", ["tiny_rows", "small_rows", "large_rows"])
-def test_pc_sweep_division_fallback(monkeypatch, case):
+def test_pc_sweep_division_fallback(monkeypatch, case, flow):
     """The LDS sweep divides by precomputed reciprocals of ap and sor only
     where that is exact: dividends of frexp exponent within +-750 and
     divisors within [2^-64, 2^64].  A batch that meets anything else is
@@ -365,6 +379,7 @@ def test_pc_sweep_division_fallback(monkeypatch, case):
     pressure-correction solve stays bitwise equal to the oracle's.  Tile 3
     puts such rows and ordinary ones into different batches."""
     monkeypatch.setenv("CFDL_TILE", "3")
+    _flow(monkeypatch, flow)
     eq, oc = make_pair(10, 0.1, 4)
     eq.run(1, 2)
     oc.run(1, 2)
@@ -387,14 +402,16 @@ def test_pc_sweep_division_fallback(monkeypatch, case):
     assert np.count_nonzero(oc.arr("phic")[:ne]) > ne // 2
 
 
+@pytest.mark.parametrize("flow", ["flow", "steps"])
 @pytest.mark.parametrize("case", ["tiny_rows", "small_rows"])
-def test_momentum_sweep_division_fallback(monkeypatch, case):
+def test_momentum_sweep_division_fallback(monkeypatch, case, flow):
     """The three momentum solves share one LDS walk; its reciprocal division
     falls back to the hardware division batch by batch as the pressure-
     correction sweep does (decoupled rows with values near 2^-1030, or rows
     scaled by 2^-100).  u, v and w equal the oracle's solve_gs results."""
     import ctypes as C
     monkeypatch.setenv("CFDL_TILE", "3")
+    _flow(monkeypatch, flow)
     eq, oc = make_pair(10, 0.1, 4)
     eq.run(1, 2)
     oc.run(1, 2)
@@ -477,9 +494,8 @@ def test_mixed_pc_order_bitwise(n, jit, relax, nsubd, nit):
 
 
 def test_serial_assembly_kernels_bitwise(monkeypatch):
-    """The one-thread-per-cell assembly kernels (k_coef_uvw, k_coef_p), which
-    meshes with other row lengths would use, selected with CFDL_COEF_SERIAL=1
-    when the context is created: fields and solver lines match the oracle."""
+    """The assembly kernels for rows of any length (k_coef_uvw, k_coef_p),
+    selected with CFDL_COEF_SERIAL=1 when the context is created: fields and solver lines match the oracle."""
     monkeypatch.setenv("CFDL_COEF_SERIAL", "1")
     eq, oc = make_pair(9, 0.15, 4)
     eq.set_relaxation(0.7, 0.3)
