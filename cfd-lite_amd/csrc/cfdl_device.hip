@@ -2644,7 +2644,9 @@ static int upload(cfdl_ctx *c, T **p, const std::vector<T> &v) {
 
 static inline int nblocks(int64_t n) { return static_cast<int>((n + kBlock - 1) / kBlock); }
 
-// fa, and the FP64 assembly's fd if it is not there (rows of six entries only)
+// fa, and the FP64 assembly's fd if it is not there (rows of six entries
+// only): at creation, on a change back to FP64, and before an FP64 assembly
+// after a change to FP32 that ran out of memory
 static int face_geo64(cfdl_ctx *c) {
   if (c->md.fd) return CFDL_OK;
   void *fd = nullptr;
@@ -4587,6 +4589,7 @@ int cfdl_calc_coef_uvw(cfdl_ctx *c) {
               "alpha_u < 1 (cfdl_set_relaxation)");
     return CFDL_ESTATE;
   }
+  if (c->mhex && !c->asm32) CALL(face_geo64(c));
   if (c->mhex && c->asm32)
     hipLaunchKernelGGL(k_coef_uvw6<float>, dim3(nblocks(c->ne)),
                        dim3(kBlock), 0, c->st, c->md, c->fd, c->dt, c->alpha_u);
@@ -5074,6 +5077,7 @@ int batch_check(cfdl_batch *b, cfdl_ctx *c) {
     set_error("cfdl_batch: the case has no multigrid hierarchy");
     return CFDL_ESTATE;
   }
+  if (!asm32) CALL(face_geo64(c));
   // the precision of the batch is its first case's
   const cfdl_ctx *c0 = b->ctx.empty() ? c : b->ctx[0];
   if (fp32 != (c0->pc_order == CFDL_PC_MGCG_MIXED ? 1 : 0) || asm32 != (c0->asm32 ? 1 : 0)) {
