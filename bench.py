@@ -55,33 +55,42 @@ HBM_PEAK_GBS = 8000.0
 
 # Algorithmic bytes per cell of one outer iteration (each array element a
 # kernel touches counted once; FP64 8 B, FP32 and int32 4 B; hexahedral
-# interior cell): 2108 B for assembly, gradients, face fluxes and the update,
-# 100 + 316 n per momentum solve of n Gauss-Seidel iterations, and for the
-# pc solve of n iterations:
-#   reference / colour order: 100 + 226 n  (two FP64 sweeps of 108 B and a
-#     residual every tenth iteration)
-#   "mixed" (FP32 colour sweeps): 184 + 146 n  (FP32 copies of ap and anb,
-#     two 68 B sweeps, an FP64 residual every tenth iteration)
+# interior cell): 2108 B for assembly, gradients, face fluxes and the update;
+# the momentum solve of u, v and w, whose sweeps and residuals read the rows
+# once for all three (80 B, and 28 B a sweep and 16 B a residual for each):
+# 132 + 460 n for n Gauss-Seidel iterations in the reference order (two sweeps
+# of 164 B and a residual of 132 B), 132 + 378 n in colour order (half the
+# cells, the turning colour, take both updates from one pass over their rows);
+# and for the pc solve of n iterations:
+#   reference order: 100 + 226 n  (two FP64 sweeps of 108 B and a residual
+#     every tenth iteration)
+#   colour order: 100 + 145 n  (a block of two iterations is five passes over
+#     half the rows, 270 B)
+#   "mixed" (FP32 colour sweeps): 184 + 95 n  (FP32 copies of ap and anb, 170 B
+#     a block, an FP64 residual every tenth iteration)
 #   "mgcg" (FP64 V-cycle): 190 + 580 n  (initial residual and the Galerkin
-#     sums; per CG iteration a forward and a backward colour sweep of 108 B,
-#     the restriction 104 B and prolongation 20 B on the mesh, 8/7 of that
-#     over the coarse levels, plus 196 B of CG vectors and the 100 B product)
+#     sums; per CG iteration the V-cycle's forward sweep, which reads half the
+#     rows, its residuals of the other half, the restriction, the prolongation
+#     and the backward sweep, 250 B together, 8/7 of that over the coarse
+#     levels, plus 196 B of CG vectors and the 100 B product)
 #   "mgcg-mixed" (FP32 V-cycle): 274 + 442 n
 BYTES_FIXED = 2108.0
-PC_BYTES = {"reference": (100.0, 226.0), "colored": (100.0, 226.0), "mixed": (184.0, 146.0),
+GS_BYTES = {"reference": (132.0, 460.0), "colored": (132.0, 378.0)}
+PC_BYTES = {"reference": (100.0, 226.0), "colored": (100.0, 145.0), "mixed": (184.0, 95.0),
             "mgcg": (190.0, 580.0), "mgcg-mixed": (274.0, 442.0)}
 
 
-def iteration_bytes(log, pc_order):
+def iteration_bytes(log, pc_order, gs_order):
     """Algorithmic bytes per cell of the outer iterations in log (one line
     per linear solve, u v w pc per iteration): the sum over them."""
-    b0, b1 = PC_BYTES[pc_order]
-    total = 0.0
+    (m0, m1), (b0, b1) = GS_BYTES[gs_order], PC_BYTES[pc_order]
+    total, momentum = 0.0, 0
     for name, it, ri, rf, rm in log:
         if name == "pc":
-            total += BYTES_FIXED + b0 + b1 * it
+            total += BYTES_FIXED + m0 + m1 * momentum + b0 + b1 * it
+            momentum = 0
         else:
-            total += 100.0 + 316.0 * it
+            momentum = max(momentum, it)
     return total
 
 
@@ -310,7 +319,7 @@ def run_mode(cfdl, mesh, mu, order, gs, steps, warmup, channel=False, keep=False
     eq.synchronize()
     secs = time.perf_counter() - t
     log = eq.log()
-    nbytes = ne * iteration_bytes(log, order)
+    nbytes = ne * iteration_bytes(log, order, gs)
     out = {"pc_order": order, "gs_order": gs, "value": round(ne * steps / secs, 1),
            "unit": "cell-iterations/s", "ms_per_step": round(1e3 * secs / steps, 3),
            "steps": steps, "warmup": warmup,
@@ -617,13 +626,16 @@ def main():
     if traffic_kib is None and args.n == 128 and not schedule_env:
         traffic_kib = TRAFFIC_KIB_128
     traffic = None if traffic_kib is None else round(traffic_kib * 1024.0)
+    # one launch updates every cell four times, or only a step of a sweep
+    kernel = ("k_gs_flow<1> (pressure-correction Gauss-Seidel, four sweeps of space-time tiles in LDS)"
+              if cells == 4 * ne else "pressure-correction Gauss-Seidel, launched step by step")
     roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
                 "algorithmic_bytes_per_launch": round(BYTES_PER_CELL_SWEEP * cells),
-                "kernel": "k_gs_flow<1> (pressure-correction Gauss-Seidel, four sweeps of space-time tiles in LDS)",
+                "kernel": kernel,
                 "launch_ms": round(kernel_ms, 5), "cells_per_launch": round(cells, 1),
                 "sampled_launches": int(st["sampled_launches"])}
-    hbm_whole = ne * iteration_bytes(log[-4 * args.steps:], "reference") / secs / (HBM_PEAK_GBS * 1e9)
+    hbm_whole = ne * iteration_bytes(log[-4 * args.steps:], "reference", "reference") / secs / (HBM_PEAK_GBS * 1e9)
     progress("pc level launches %d (%.0f cells each), %d levels per symmetric sweep; "
              "outer iteration %.1f ms" % (st["pc_launches"], st["pc_cells"] / max(st["pc_launches"], 1),
                                           st["pc_levels_per_sym_sweep"], 1e3 * secs / args.steps))
