@@ -9,9 +9,11 @@
 // thread per cell / face, reading neighbours through the CSR (gathers, no
 // atomics).  The Gauss-Seidel sweeps keep the reference's exact order: cells
 // are grouped by dependency level (a cell's level is one more than the
-// highest level among its already-updated neighbours) and each level is one
-// launch, so every cell sees exactly the neighbour values it sees in the
-// sequential sweep.  Norms are fixed-order tree reductions (reproducible;
+// highest level among its already-updated neighbours) and the levels of a
+// spatial tile into batches, which wait for the batches they depend on
+// (k_gs_flow; launch by launch, or level by level, where that does not apply),
+// so every cell sees exactly the neighbour values it sees in the sequential
+// sweep.  Norms are fixed-order tree reductions (reproducible;
 // equal to the sequential sums up to rounding in the last bits).
 //
 // Device layout (HBM, 0-based; cells 0..ne-1, boundary halos ne..ne+nbf-1):
@@ -255,8 +257,11 @@ __device__ inline void centre(const MeshDev &m, int e, double *r) {
 // nothing else does (every product and sum is the negated or the same one),
 // except the weight, whose two values are kept.  With them and a thread per
 // cell (d_coef_uvw6) at 128^3: k_coef_uvw6 713 -> 575 us, k_coef_p6 252 -> 183
-// us, k_update_faces 129 -> 92 us.  (calc_mip keeps its own: it is bound by
-// memory and reads as many bytes either way, 196 us against 209 us.)
+// us, k_update_faces 129 -> 92 us.  The distances of the centres and of the
+// feet are a square root each in k_coef_uvw6: kept here as well they cost more
+// loads than roots (514 us against 431 at 128^3) and 48 B a cell.  (calc_mip
+// keeps its own: it is bound by memory and reads as many bytes either way, 196
+// us against 209 us.)
 template <typename T>
 __global__ void k_face_geo(MeshDev m, T *fa, T *fd) {
   const auto G = geo_of<T>(m);
@@ -2396,7 +2401,6 @@ __global__ void gb_log_gs(GroupMap g, const BSlot *__restrict__ S, Names nm) {
   BSLOT;
   d_log_gs(bx, x.gctl, 3, nm, x.log, x.nlog);
 }
-// which: 0 u -> gu, 1 v -> gv, 2 w -> gw, 3 phic -> gpc
 // the gradient of u alone (the tuner's launch), of u, v and w, of phic
 __global__ void gb_grad_u(GroupMap g, const BSlot *__restrict__ S) {
   BSLOT;
@@ -2726,9 +2730,10 @@ static int sweep(cfdl_ctx *c, const Sched &s, const SysDesc &sys, int nc, double
 
 // Sampled timing of the pressure-correction sweeps: HIP events on the
 // context stream before the first and after the last launch of every
-// sample_every-th step (a sweep, or a block's sweeps that run together).  The launches run back to back in between, so
-// elapsed / launches is the mean launch duration without the dispatch
-// latency that an event pair around a single launch adds.
+// sample_every-th step (a sweep, or a block's sweeps that run together).  The
+// launches run back to back in between, so elapsed / launches is the mean
+// launch duration without the dispatch latency that an event pair around a
+// single launch adds.
 static int sample_begin(cfdl_ctx *c, cfdl_ctx::Sample **smp) {
   *smp = nullptr;
   const int64_t k = c->pc_sweeps++;
@@ -3297,9 +3302,12 @@ static void bin_tiles(const std::vector<int> &grp, const std::vector<int> &cell,
 // workgroups (as many per CU as its LDS holds the largest batch of), the
 // gather (a latency and the largest batch's cells) and the levels of its
 // longest batch.  A schedule with a segment wider than a wavefront loses the
-// pipelined walk, and so counts three times.  The constants fit the measured
-// sweeps of the 16^3, 32^3, 64^3 and 128^3 cavities and the 61 x 47 x 53 box
-// in seven shapes each to within 10%.
+// pipelined walk, and so counts three times.  The constants are those of the
+// sweeps launched step by step, of which they fit the 16^3, 32^3, 64^3 and
+// 128^3 cavities and the 61 x 47 x 53 box in seven shapes each to within 10%.
+// k_gs_flow, which runs most schedules, has no such steps, and its sweeps take
+// 0.64 to 0.81 of the model's time; what counts is the order of the shapes
+// (kTileShapes).
 constexpr double kLaunchUs = 1.4, kGatherUs = 0.9, kCellUs = 1.0 / 512;
 static double tile_launches(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
                             const std::vector<int> &lev, const std::vector<int> &order,
@@ -3365,10 +3373,13 @@ struct TileShape {
 // The shapes a schedule is chosen from (CFDL_TILE / CFDL_TILE_SPAN replace
 // them): the model's best ones over cavities, jittered and odd boxes.  Small
 // batches (512 cells, several per CU) and large ones (1020 cells of at most
-// 60 a level: fewer launches, one batch per CU) each win on some meshes.
-// Runs of the reference order against one fixed 16 x 8 x 4 shape cut at the
-// first cell's centre: 16^3 13.1 -> 11.7 ms, 32^3 54.9 -> 46.2 ms, the
-// distorted 61 x 47 x 53 box 231 -> 72 ms, 128^3 352 -> 332 ms.
+// 60 a level: fewer steps, one batch per CU) each win on some meshes.  Three
+// outer iterations by k_gs_flow, the model's choice / the fastest of the five
+// / the slowest: 16^3 8.9 / 9.0 / 9.7 ms, 32^3 17.7 / 17.9 / 24.1 ms, the
+// distorted 61 x 47 x 53 box 53.9 / 53.2 / 63.2 ms, 64^3 48.0 / 48.6 / 59.7 ms,
+// 97 x 40 x 23 64.5 / 63.0 / 78.1 ms, 128^3 136.1 / 134.6 / 155.5 ms, 160^3
+// 181.3 / 179.5 / 259.8 ms (one shape for the momentum and the pc sweeps; the
+// model chooses each).
 constexpr TileShape kTileShapes[] = {{{16, 8, 4}, 32}, {{16, 16, 4}, 32}, {{16, 16, 4}, 20},
                                      {{8, 8, 8}, 32},  {{12, 8, 8}, 32}};
 static void plan_tiles(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
@@ -3410,8 +3421,9 @@ static void plan_tiles(int ne, const std::vector<int> &row, const std::vector<in
 
 // The neighbouring batches of every batch (those holding its outside
 // neighbours), of earlier and of later launches, and the counters of
-// k_gs_flow; no table, and so the launch-by-launch sweeps, if a batch has
-// more of either than the waiting wavefront has lanes.
+// k_gs_flow; no table, and so the launch-by-launch sweeps, if a batch has 64
+// or more of either (the waiting wavefront has a lane for each and one for the
+// batch itself).
 static int flow_tables(cfdl_ctx *c, const std::vector<int> &rowp, const std::vector<int> &nbrp,
                        const std::vector<int> &seg, const std::vector<int> &bseg,
                        cfdl_ctx::TileSched *tp) {
@@ -3442,8 +3454,10 @@ static int flow_tables(cfdl_ctx *c, const std::vector<int> &rowp, const std::vec
   const char *fl = std::getenv("CFDL_FLOW");
   const int per_cu = static_cast<int>((160 * 1024) / (t.lds_bytes + 16));
   // a workgroup per CU, more where the middle launches have more batches (three
-  // outer iterations with 256 / 512 / 768: 61 x 47 x 53 53.9 / 54.9 / 54.9 ms,
-  // 128^3 135.1 / 135.9 / 137.7 ms, 192^3 317 / 232 / 224 ms)
+  // outer iterations with 256 / 512 / 768: 16^3, 32^3 and 64^3 the same within
+  // 1%, 61 x 47 x 53 54.1 / 55.0 / 55.0 ms, 97 x 40 x 23 64.6 / 65.8 / 66.6 ms,
+  // 128^3 136.2 / 136.7 / 138.5 ms, 160^3 215.8 / 181.6 / 185.5 ms, 192^3 317 /
+  // 232 / 224 ms; the rule's choice is the best of them on each of the eight)
   const int mean = nb / static_cast<int>(t.launch_ptr.size() - 1);
   const int wgs = fl ? std::atoi(fl) : 256 * std::min(per_cu, 1 + mean / 140);
   if (wgs <= 0 || per_cu < 1) return CFDL_OK;
@@ -3815,8 +3829,8 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
   // thermal properties as init_properties sets them, mod_properties.f90:88-89
   CALL(up64(&d_cp, std::vector<double>(ne, 1000.0).data(), ne));
   CALL(up64(&d_tc, std::vector<double>(ne, 5.0).data(), ne));
-  // CFDL_COEF_SERIAL=1 keeps the one-thread-per-cell assembly kernels, which
-  // also serve meshes with other row lengths
+  // CFDL_COEF_SERIAL=1 takes the assembly kernels for rows of any length
+  // (k_coef_uvw, k_coef_p)
   const char *cs = std::getenv("CFDL_COEF_SERIAL");
   C->mhex = row[ne] == 6 * ne && !(cs && cs[0] == '1');
   for (int e = 0; e < ne && C->mhex; e++) C->mhex = row[e] == 6 * e;

@@ -911,7 +911,7 @@ __device__ inline void d_mg_coarse(const Lev<T> *__restrict__ lv, int lc, int nl
     wg_sweep(F, kFwd0);
     for (int p = threadIdx.x; p < mg_open(F.L); p += blockDim.x) mg_residual(F.L, p);
     __syncthreads();
-    for (int I = threadIdx.x; I < C.L.npad; I += blockDim.x) 
+    for (int I = threadIdx.x; I < C.L.npad; I += blockDim.x)
       mg_restrict(I, F.L.mptr[I], F.L.mptr[I + 1], F.L, C.L.b);
     __syncthreads();
   }
@@ -1544,9 +1544,9 @@ template <>
 GroupRun<float> &run_of<float>(MgGroup *G) { return G->rf; }
 
 // The solve of mgcg_solve for n systems at once, in phases: begin (descriptors
-// uploaded when they changed; synchronises then, so it
-// runs outside any graph capture), setup (level 0's copies, Galerkin operators,
-// initial residual), one iteration at a time (V-cycle and CG step, then the
+// uploaded when they changed; synchronises then, so it runs outside any graph
+// capture), setup (level 0's copies, Galerkin operators, initial residual),
+// one iteration at a time (V-cycle and CG step, then the
 // systems' active flags copied to a host slot), finish (the log lines).
 // Every launch covers the systems that take part in its step; each system
 // runs exactly its own sequence of steps (a system with fewer levels or

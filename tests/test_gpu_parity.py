@@ -165,9 +165,9 @@ def test_64cube_jittered_relaxed_bitwise():
 @pytest.mark.parametrize("n,jit,relax", [(8, 0.1, False), (12, 0.15, True), (32, 0.0, True)])
 def test_colored_pc_order_bitwise(n, jit, relax):
     """The colour order of the pressure-correction smoother (an extension):
-    one launch per colour on the GPU, against the oracle's sequential
+    one launch per colour and turn on the GPU, against the oracle's sequential
     Gauss-Seidel that visits the cells in the same order.  Both colour every
-    subdomain greedily in its local order.  Fields and solver lines match
+    subdomain greedily in global cell order.  Fields and solver lines match
     bit for bit."""
     eq, oc = make_pair(n, jit, 4, mu=0.0025)
     if relax:
