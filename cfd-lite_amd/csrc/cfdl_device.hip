@@ -28,6 +28,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -3222,41 +3223,51 @@ static int multi_subdomain_solver(cfdl_ctx *c) {
   return CFDL_OK;
 }
 
-// Mean distance between the centres of neighbouring cells along each axis
-// (each pair counted on the axis of its largest component; an axis without
-// pairs gets the cube root of the mean cell volume).
-static void cell_spacing(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
-                         const double *xc, const double *yc, const double *zc, const double *vol,
-                         double *h) {
-  double sum[3] = {0.0, 0.0, 0.0}, vsum = 0.0;
-  int64_t cnt[3] = {0, 0, 0};
-  for (int e = 0; e < ne; e++) {
-    vsum += vol[e];
-    for (int k = row[e]; k < row[e + 1]; k++) {
-      const int d = nbr[k];
-      if (d >= ne || d < e) continue;
-      const double r[3] = {std::fabs(xc[d] - xc[e]), std::fabs(yc[d] - yc[e]),
-                           std::fabs(zc[d] - zc[e])};
-      const int i = r[0] >= r[1] && r[0] >= r[2] ? 0 : r[1] >= r[2] ? 1 : 2;
-      sum[i] += r[i];
-      cnt[i]++;
+// Per group of positions [grp[s], grp[s+1]) (the subdomains of the pc system,
+// or all cells), the mean distance between the centres of neighbouring cells
+// along each axis (each pair counted on the axis of its largest component; an
+// axis without pairs gets the cube root of the mean cell volume).  A group has
+// a spacing of its own: on graded meshes one subdomain's cells can be much
+// finer than another's.  cell[q] is the mesh cell at position q.
+static std::vector<std::array<double, 3>> cell_spacing(
+    const std::vector<int> &grp, const std::vector<int> &cell, const std::vector<int> &row,
+    const std::vector<int> &nbr, const double *xc, const double *yc, const double *zc,
+    const double *vol) {
+  std::vector<std::array<double, 3>> h(grp.size() - 1);
+  for (size_t s = 0; s < h.size(); s++) {
+    double sum[3] = {0.0, 0.0, 0.0}, vsum = 0.0;
+    int64_t cnt[3] = {0, 0, 0};
+    for (int q = grp[s]; q < grp[s + 1]; q++) {
+      const int e = cell[q];
+      vsum += vol[e];
+      for (int k = row[q]; k < row[q + 1]; k++) {
+        if (nbr[k] < q || nbr[k] >= grp[s + 1]) continue;
+        const int d = cell[nbr[k]];
+        const double r[3] = {std::fabs(xc[d] - xc[e]), std::fabs(yc[d] - yc[e]),
+                             std::fabs(zc[d] - zc[e])};
+        const int i = r[0] >= r[1] && r[0] >= r[2] ? 0 : r[1] >= r[2] ? 1 : 2;
+        sum[i] += r[i];
+        cnt[i]++;
+      }
     }
+    for (int i = 0; i < 3; i++)
+      h[s][i] = sum[i] > 0.0 ? sum[i] / cnt[i] : std::cbrt(vsum / (grp[s + 1] - grp[s]));
   }
-  for (int i = 0; i < 3; i++) h[i] = sum[i] > 0.0 ? sum[i] / cnt[i] : std::cbrt(vsum / ne);
+  return h;
 }
 
 // Dense ids of spatial tiles of edge[0] x edge[1] x edge[2] cell layers
 // (x, y, z): a cell's layer along an axis is its centre's distance from the
-// first one's in its group of positions [grp[s], grp[s+1]) (the subdomains of
-// the pc system, or all cells), in units of the cell spacing h, rounded to the
-// nearest.  Rounding puts the cuts between layers: a cut through a layer's
+// first one's in its group of positions [grp[s], grp[s+1]), in units of the
+// group's cell spacing h[s], rounded to the nearest.  Rounding puts the cuts between layers: a cut through a layer's
 // centres would leave a ragged face on meshes with distorted cells, where a
 // dependency chain along the face changes tile at every other cell, one
 // launch each (on the 61 x 47 x 53 box with vertices moved by 0.15 h, 69
 // launches a sweep instead of 19).  Tiles never cross groups.  cell[q] is the
 // mesh cell at position q.
 static void bin_tiles(const std::vector<int> &grp, const std::vector<int> &cell, const double *xc,
-                      const double *yc, const double *zc, const double *h, const int *edge,
+                      const double *yc, const double *zc,
+                      const std::vector<std::array<double, 3>> &h, const int *edge,
                       std::vector<int> *tid) {
   std::unordered_map<int64_t, int> tid_of;
   tid->assign(cell.size(), 0);
@@ -3274,7 +3285,7 @@ static void bin_tiles(const std::vector<int> &grp, const std::vector<int> &cell,
       const double r[3] = {xc[g], yc[g], zc[g]};
       int64_t key = static_cast<int64_t>(s);
       for (int i = 0; i < 3; i++) {
-        const int64_t layer = static_cast<int64_t>((r[i] - lo[i]) / h[i] + 0.5);
+        const int64_t layer = static_cast<int64_t>((r[i] - lo[i]) / h[s][i] + 0.5);
         key = key * (1 << 19) + layer / edge[i] % (1 << 19);
       }
       if (key != last_key) {
@@ -3312,7 +3323,7 @@ constexpr double kLaunchUs = 1.4, kGatherUs = 0.9, kCellUs = 1.0 / 512;
 static double tile_launches(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
                             const std::vector<int> &lev, const std::vector<int> &order,
                             const std::vector<int> &tid, int span, int nrhs,
-                            std::vector<int> *launch) {
+                            std::vector<int> *launch, bool *walk) {
   int ntile = 1;
   for (int e = 0; e < ne; e++) ntile = std::max(ntile, tid[e] + 1);
   struct Batch {
@@ -3363,7 +3374,8 @@ static double tile_launches(int ne, const std::vector<int> &row, const std::vect
   for (int L = 0; L < nl; L++)
     us += kLaunchUs + std::ceil(nb[L] / (256.0 * std::max(1.0, std::floor(fit)))) *
                           (batch_us + level_us * longest[L]);
-  return seg > kLdsThreads || fit < 1.0 ? 3.0 * us : us;
+  *walk = seg <= kLdsThreads && fit >= 1.0;
+  return *walk ? us : 3.0 * us;
 }
 
 // A tile shape and the levels its batches may span
@@ -3382,10 +3394,19 @@ struct TileShape {
 // model chooses each).
 constexpr TileShape kTileShapes[] = {{{16, 8, 4}, 32}, {{16, 16, 4}, 32}, {{16, 16, 4}, 20},
                                      {{8, 8, 8}, 32},  {{12, 8, 8}, 32}};
+// Finer shapes, compared too where none of those keeps its batches in LDS and
+// its segments within a wavefront: tiles are boxes in space, and on a graded
+// mesh those of the fine cells hold many times the mean.  Three outer
+// iterations without / with them: 32^3 growing by e^2 along each axis 228 / 49
+// ms, 48^3 by e^2 529 / 73 ms, by e^4 724 / 342 ms; planning takes 25 ms more at
+// 48^3.  Where a shape above has the walk the finer ones are slower (8 x 8 x 8
+// against 16 x 16 x 4 at 64^3: 59.7 / 48.6 ms), so they are not compared.
+constexpr TileShape kFineShapes[] = {{{8, 8, 2}, 20}, {{8, 4, 2}, 32}, {{4, 4, 2}, 32},
+                                     {{2, 2, 2}, 32}, {{1, 1, 1}, 32}};
 static void plan_tiles(int ne, const std::vector<int> &row, const std::vector<int> &nbr,
                        const std::vector<int> &lev, const std::vector<int> &grp,
                        const std::vector<int> &cell, const double *xc, const double *yc,
-                       const double *zc, const double *h, int nrhs,
+                       const double *zc, const double *vol, int nrhs,
                        const std::vector<TileShape> &shapes, std::vector<int> *tid,
                        std::vector<int> *launch) {
   // cells by level (stable: in set-up order within a level)
@@ -3393,30 +3414,35 @@ static void plan_tiles(int ne, const std::vector<int> &row, const std::vector<in
   for (int e = 0; e < ne; e++) start[lev[e] + 1]++;
   for (size_t l = 1; l < start.size(); l++) start[l] += start[l - 1];
   for (int e = 0; e < ne; e++) order[start[lev[e]]++] = e;
+  const std::vector<std::array<double, 3>> h = cell_spacing(grp, cell, row, nbr, xc, yc, zc, vol);
   struct Plan {
     std::vector<int> tid, launch;
-    double us;
+    double us = 0.0;
+    bool walk = false;
+  } best;
+  auto compare = [&](const std::vector<TileShape> &list) {
+    std::vector<std::future<Plan>> plans;  // one host thread per shape
+    for (const TileShape &s : list)
+      plans.push_back(std::async([&, s] {
+        Plan p;
+        bin_tiles(grp, cell, xc, yc, zc, h, s.edge, &p.tid);
+        p.us = tile_launches(ne, row, nbr, lev, order, p.tid, s.span, nrhs, &p.launch, &p.walk);
+        return p;
+      }));
+    for (size_t i = 0; i < list.size(); i++) {
+      Plan p = plans[i].get();
+      if (trace_on())
+        std::fprintf(stderr, "cfdl: tiles %dx%dx%d span %d: %d launches, %.0f us a sweep\n",
+                     list[i].edge[0], list[i].edge[1], list[i].edge[2], list[i].span,
+                     *std::max_element(p.launch.begin(), p.launch.end()) + 1, p.us);
+      if (best.tid.empty() || p.us < best.us) best = std::move(p);
+    }
   };
-  std::vector<std::future<Plan>> plans;  // one host thread per shape
-  for (const TileShape &s : shapes)
-    plans.push_back(std::async([&, s] {
-      Plan p;
-      bin_tiles(grp, cell, xc, yc, zc, h, s.edge, &p.tid);
-      p.us = tile_launches(ne, row, nbr, lev, order, p.tid, s.span, nrhs, &p.launch);
-      return p;
-    }));
-  double best = 0.0;
-  for (size_t i = 0; i < shapes.size(); i++) {
-    Plan p = plans[i].get();
-    if (trace_on())
-      std::fprintf(stderr, "cfdl: tiles %dx%dx%d span %d: %d launches, %.0f us a sweep\n",
-                   shapes[i].edge[0], shapes[i].edge[1], shapes[i].edge[2], shapes[i].span,
-                   *std::max_element(p.launch.begin(), p.launch.end()) + 1, p.us);
-    if (i > 0 && p.us >= best) continue;
-    best = p.us;
-    tid->swap(p.tid);
-    launch->swap(p.launch);
-  }
+  compare(shapes);
+  if (!best.walk && shapes.size() > 1)
+    compare(std::vector<TileShape>(std::begin(kFineShapes), std::end(kFineShapes)));
+  tid->swap(best.tid);
+  launch->swap(best.launch);
 }
 
 // The neighbouring batches of every batch (those holding its outside
@@ -3883,8 +3909,6 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
     if (sp) f.span = std::min(63, std::max(1, std::atoi(sp)));
     shapes.assign(1, f);
   }
-  double hmean[3];
-  cell_spacing(ne, row, nbr, xc, yc, zc, vol, hmean);
   const char *mode = std::getenv("CFDL_GS_MODE");
   C->tiled = !(mode && std::string(mode) == "level");
   const char *rc = std::getenv("CFDL_TILE_RCP");
@@ -3897,7 +3921,7 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
       // the global system in tile numbering, for the tiled solve_gs
       std::vector<int> all(ne), grp{0, ne}, tid, launch;
       for (int e = 0; e < ne; e++) all[e] = e;
-      plan_tiles(ne, row, nbr, lev, grp, all, xc, yc, zc, hmean, 3, shapes, &tid, &launch);
+      plan_tiles(ne, row, nbr, lev, grp, all, xc, yc, zc, vol, 3, shapes, &tid, &launch);
       std::vector<int> n2o(all), o2n(ne);
       std::stable_sort(n2o.begin(), n2o.end(), [&](int x, int y) {
         if (launch[x] != launch[y]) return launch[x] < launch[y];
@@ -4032,7 +4056,7 @@ int cfdl_ctx_create(int ne, int nf, int nbf, const int *ef2nb_idx, const int *ef
     for (int s = 0; s < nsubd; s++) levels(rowo, nbro, C->co[s], C->co[s + 1], true, lev);
     for (int q = 0; q < ne; q++) C->pc_nlev = std::max(C->pc_nlev, lev[q]);
     std::vector<int> tid, launch;
-    plan_tiles(ne, rowo, nbro, lev, C->co, l2g, xc, yc, zc, hmean, 1, shapes, &tid,
+    plan_tiles(ne, rowo, nbro, lev, C->co, l2g, xc, yc, zc, vol, 1, shapes, &tid,
                &launch);
     // renumber the pc system by (subdomain, launch, tile, level): every
     // (launch, tile) batch of the tiled sweeps becomes a contiguous range

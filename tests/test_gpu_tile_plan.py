@@ -6,6 +6,7 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 import cfdl
@@ -34,6 +35,30 @@ def test_three_blocks_bitwise(nsubd):
     oc.run(1, 2)
     assert_fields_equal(eq, oc)
     assert_logs_match(eq.log(), oc.log())
+
+
+def graded(n, s):
+    """A box whose cells grow by a factor e^s along each axis."""
+    g = meshgen.box_mesh(n)
+    for k in ("x", "y", "z"):
+        top = g[k].max()
+        g[k] = top * (np.exp(s * g[k] / top) - 1.0) / (np.exp(s) - 1.0)
+    return g
+
+
+@pytest.mark.parametrize("n,s,nsubd", [(24, 2.0, 4), (24, 2.0, 2), (15, 4.0, 4), (20, 3.0, 1)])
+def test_graded_boxes_bitwise(n, s, nsubd):
+    """Cells much finer than the mean: the boxes of the usual shapes hold too
+    many of them for the LDS or the walk, and finer shapes take their place,
+    so that the sweeps of a block still run in one launch."""
+    eq, oc = pair(graded(n, s), nsubd)
+    eq.run(1, 2)
+    oc.run(1, 2)
+    assert_fields_equal(eq, oc)
+    assert_logs_match(eq.log(), oc.log())
+    st = eq.stats()
+    if nsubd > 1:  # 50 blocks a solve
+        assert st["pc_launches"] == 2 * 50
 
 
 PLAN_MEMORY = """
